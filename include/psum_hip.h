@@ -438,11 +438,11 @@ psum_status psum_stepper_set_interp_order(void* h, int order);
 
 /* Multigrid kernel-shape options that may change after creation, as
  * whitespace "key value" pairs: "fuse 0|1" (2D fused tile smoothing and
- * residual + restriction, default 1), "tail 0|1" (the coarse end of each
- * V-cycle, levels of at most 33^2 / 9^3 nodes down to a coarsest level of
- * at most 10^2 / 5^3, in one workgroup; default 0) and "line 0|1" (3D 7-point
+ * residual + restriction, default 1) and "line 0|1" (3D 7-point
  * levels in chunks of four nodes per thread, 3D prolongation over planes,
- * default 1).  Results are bit-identical either way.  A batch instance's
+ * default 1); "tail 0|1" is accepted and has no effect (the coarse end of
+ * every V-cycle is one dense product).  Results are bit-identical either
+ * way.  A batch instance's
  * change makes the batch capture its step graph again at its next run.  No
  * reference counterpart (tuning knobs). */
 psum_status psum_stepper_mg_tuning(void* h, const char* options);

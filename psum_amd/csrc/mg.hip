@@ -47,6 +47,9 @@ using namespace psum_hip;
 namespace {
 
 constexpr int kMgThreads = 256;
+// right-hand sides hold this many zeros beyond their nodes (the dense product
+// reads whole 16-byte vectors of its operator's rows)
+constexpr int kOpPad = 4;
 
 #define MG_HIP(expr)                                                                        \
     do {                                                                                    \
@@ -669,341 +672,6 @@ __global__ __launch_bounds__(kMgThreads) void k_restrict_plane(DevLevel F, DevLe
     xc[i] = first_sweep != (T)0 ? bv * (first_sweep * (T)1) : (T)0;
 }
 
-// ---- V-cycle tail in one workgroup -----------------------------------------
-// The coarse end of the hierarchy (levels lt..Lc, at most kMaxTail) is
-// latency-bound: a handful of nodes per level, three launches per level.
-// k_vtail runs all of it in one 1024-thread workgroup.  It first stages in
-// LDS every tail level's class ids, class tables and transfer tables, the
-// iterate and right-hand side of level lt, and then keeps every level's two
-// iterates and right-hand side there: pre-sweeps, residual, restriction down
-// to the coarsest level, its dense solve (the inverse is read from global
-// memory), then prolongation and post-sweeps back up to level lt, whose
-// iterate it writes back.  Each phase is the per-node arithmetic of
-// k_smooth, k_residual, k_restrict, k_coarse_solve and k_prolong_add (2D or
-// 3D) in the same order, so the result is bit-identical to the
-// launch-per-phase path.
-constexpr int kMaxTail = 6;
-constexpr int kTailThreads = 1024;
-// coarsest nodes: one compute unit reads the dense inverse (n^2 doubles)
-// from memory at a few tens of GB/s, so it must stay small (2D: 10^2, 3D:
-// 5^3 nodes)
-template <int D>
-constexpr int tail_coarse() { return D == 2 ? 100 : 125; }
-// one compute unit runs the tail: 64 lanes of VALU per clock, so a 2D level
-// of 64^2 nodes already costs what its own multi-block launches cost; the
-// tail takes 2D levels of at most 33^2 nodes and 3D levels of at most 9^3
-// (a 17^3 level's 27-point sweep takes ~20 us on one compute unit against
-// ~4.4 us as a launch of its own; levels 9^3 and 5^3 of the 3D box take
-// 52 us per V-cycle in the tail, 54 us in their own launches)
-template <int D>
-constexpr int tail_level_nodes() { return D == 2 ? 1089 : 729; }
-constexpr int kTailRows = (125 + kTailThreads / 64 - 1) / (kTailThreads / 64);   // rows per wave
-
-template <typename T>
-struct TailLevel {
-    int n[3], wrap[3], N, compact, ncls;
-    // byte offsets into the workgroup's LDS
-    int ox, oy, ob, ocls, orx, oa, odinv;
-    const uint16_t* cls;
-    const T* rx;          // relax rows, ncls x 3^D
-    const T* a;           // scaled operator rows, ncls x 3^D
-    const T* dinv;        // ncls
-};
-
-template <typename T>
-struct TailTransfer {
-    int wrap[3];
-    // byte offsets per axis: restriction (per coarse index) and prolongation
-    // (per fine index) tables
-    int orf[3], orn[3], orw[3], opc[3], opw[3];
-    const int *rf[3], *rn[3], *pc[3];
-    const T *rw[3], *pw[3];
-};
-
-template <typename T>
-struct TailArgs {
-    int nl;                         // tail levels; the last is the coarsest
-    int pre, post;
-    T two3;
-    TailLevel<T> lev[kMaxTail];
-    TailTransfer<T> tr[kMaxTail - 1];
-    const T* x_in;                  // level lt iterate after the restriction
-    const T* b_in;                  // level lt right-hand side
-    T* x_out;
-    const double* cinv;
-};
-
-template <typename U>
-__device__ __forceinline__ void tail_copy(unsigned char* lds, int off, const U* __restrict__ g, int n)
-{
-    U* d = reinterpret_cast<U*>(lds + off);
-    for (int i = threadIdx.x; i < n; i += kTailThreads) d[i] = g[i];
-}
-
-// stencil_apply<T, D, COMPACT> on a tail level: sum_k coef[k] * x[nb_k] over
-// the 3^D offsets (first axis slowest), clamped or wrapped neighbours;
-// COMPACT: the 2D+1 axis offsets
-template <typename T, int D, bool COMPACT>
-__device__ __forceinline__ T tail_stencil(const T* coef, const T* x, const int* c, const TailLevel<T>& t)
-{
-    T s = (T)0;
-    if constexpr (D == 2) {
-#pragma unroll
-        for (int a = -1; a <= 1; ++a)
-#pragma unroll
-            for (int b = -1; b <= 1; ++b) {
-                if (COMPACT && a != 0 && b != 0) continue;
-                const int k = (a + 1) * 3 + (b + 1);
-                const int q0 = nb_index(c[0], a, t.n[0], t.wrap[0]);
-                const int q1 = nb_index(c[1], b, t.n[1], t.wrap[1]);
-                s = s + coef[k] * x[q0 * t.n[1] + q1];
-            }
-    } else {
-#pragma unroll
-        for (int a = -1; a <= 1; ++a)
-#pragma unroll
-            for (int b = -1; b <= 1; ++b)
-#pragma unroll
-                for (int e = -1; e <= 1; ++e) {
-                    if (COMPACT && ((a != 0) + (b != 0) + (e != 0)) > 1) continue;
-                    const int k = (a + 1) * 9 + (b + 1) * 3 + (e + 1);
-                    const int q0 = nb_index(c[0], a, t.n[0], t.wrap[0]);
-                    const int q1 = nb_index(c[1], b, t.n[1], t.wrap[1]);
-                    const int q2 = nb_index(c[2], e, t.n[2], t.wrap[2]);
-                    s = s + coef[k] * x[(q0 * t.n[1] + q1) * t.n[2] + q2];
-                }
-    }
-    return s;
-}
-
-template <int D, typename T>
-__device__ __forceinline__ void tail_coords(const TailLevel<T>& t, int i, int* c)
-{
-    if constexpr (D == 3) {
-        const int q = i / t.n[2];
-        c[2] = i - q * t.n[2];
-        c[1] = q % t.n[1];
-        c[0] = q / t.n[1];
-    } else {
-        c[0] = i / t.n[1];
-        c[1] = i - c[0] * t.n[1];
-    }
-}
-
-// out = stencil(rows, x) * m + b * f for every node of level t
-template <typename T, int D>
-__device__ __forceinline__ void tail_apply(unsigned char* lds, const TailLevel<T>& t, int orows, const T* x,
-                                           T* out, T m, T f)
-{
-    constexpr int K = D == 2 ? 9 : 27;
-    const uint16_t* cls = reinterpret_cast<const uint16_t*>(lds + t.ocls);
-    const T* rows = reinterpret_cast<const T*>(lds + orows);
-    const T* b = reinterpret_cast<const T*>(lds + t.ob);
-    for (int i = threadIdx.x; i < t.N; i += kTailThreads) {
-        int c[3];
-        tail_coords<D>(t, i, c);
-        const T* coef = rows + (int)cls[i] * K;
-        const T v = t.compact ? tail_stencil<T, D, true>(coef, x, c, t) : tail_stencil<T, D, false>(coef, x, c, t);
-        out[i] = v * m + b[i] * f;
-    }
-}
-
-template <typename T, int D>
-__global__ __launch_bounds__(kTailThreads) void k_vtail(TailArgs<T> a)
-{
-    extern __shared__ __align__(16) unsigned char lds[];
-    constexpr int K = D == 2 ? 9 : 27;
-    const int nl = a.nl, Lc = a.nl - 1;
-    // stage tables, level lt's iterate and right-hand side
-    for (int l = 0; l < nl; ++l) {
-        const TailLevel<T>& t = a.lev[l];
-        tail_copy<uint16_t>(lds, t.ocls, t.cls, t.N);
-        tail_copy<T>(lds, t.orx, t.rx, t.ncls * K);
-        tail_copy<T>(lds, t.oa, t.a, t.ncls * K);
-        tail_copy<T>(lds, t.odinv, t.dinv, t.ncls);
-        if (l < Lc) {
-            const TailTransfer<T>& r = a.tr[l];
-            const TailLevel<T>& c = a.lev[l + 1];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                tail_copy<int>(lds, r.orf[d], r.rf[d], c.n[d]);
-                tail_copy<int>(lds, r.orn[d], r.rn[d], c.n[d]);
-                tail_copy<T>(lds, r.orw[d], r.rw[d], 3 * c.n[d]);
-                tail_copy<int>(lds, r.opc[d], r.pc[d], t.n[d]);
-                tail_copy<T>(lds, r.opw[d], r.pw[d], 2 * t.n[d]);
-            }
-        }
-    }
-    tail_copy<T>(lds, a.lev[0].ox, a.x_in, a.lev[0].N);
-    tail_copy<T>(lds, a.lev[0].ob, a.b_in, a.lev[0].N);
-    __syncthreads();
-    // bit l: which of level l's two LDS iterates holds its current iterate
-    unsigned cur = 0;
-    auto X = [&](int l) {
-        return reinterpret_cast<T*>(lds + (((cur >> l) & 1u) ? a.lev[l].oy : a.lev[l].ox));
-    };
-    auto Y = [&](int l) {
-        return reinterpret_cast<T*>(lds + (((cur >> l) & 1u) ? a.lev[l].ox : a.lev[l].oy));
-    };
-    for (int l = 0; l < Lc; ++l) {
-        const TailLevel<T>& t = a.lev[l];
-        // coarse levels received their first sweep from the restriction
-        const int sweeps = a.pre > 0 ? a.pre - 1 : 0;
-        for (int s = 0; s < sweeps; ++s) {
-            tail_apply<T, D>(lds, t, t.orx, X(l), Y(l), (T)1, a.two3 * (T)1);
-            __syncthreads();
-            cur ^= 1u << l;
-        }
-        // r = (A x)*(-1) + b*1 into the free iterate
-        T* r = Y(l);
-        tail_apply<T, D>(lds, t, t.oa, X(l), r, (T)-1, (T)1);
-        __syncthreads();
-        // b_c = (R r) o D_c^-1 ; x_c = b_c * (2/3) (first sweep) or 0
-        const TailLevel<T>& cl = a.lev[l + 1];
-        const TailTransfer<T>& tr = a.tr[l];
-        const int *rf[3], *rn[3];
-        const T* rw[3];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            rf[d] = reinterpret_cast<const int*>(lds + tr.orf[d]);
-            rn[d] = reinterpret_cast<const int*>(lds + tr.orn[d]);
-            rw[d] = reinterpret_cast<const T*>(lds + tr.orw[d]);
-        }
-        const uint16_t* ccls = reinterpret_cast<const uint16_t*>(lds + cl.ocls);
-        const T* cdinv = reinterpret_cast<const T*>(lds + cl.odinv);
-        const T fs = (l + 1 < Lc && a.pre > 0) ? a.two3 : (T)0;
-        T* bc = reinterpret_cast<T*>(lds + cl.ob);
-        T* xc = reinterpret_cast<T*>(lds + cl.ox);
-        for (int i = threadIdx.x; i < cl.N; i += kTailThreads) {
-            int c[3];
-            tail_coords<D>(cl, i, c);
-            T sum = (T)0;
-            const int f0 = rf[0][c[0]], m0 = rn[0][c[0]];
-            const int f1 = rf[1][c[1]], m1 = rn[1][c[1]];
-            if constexpr (D == 2) {
-                for (int p = 0; p < m0; ++p) {
-                    const T w0 = rw[0][3 * c[0] + p];
-                    const int i0 = wrap_index(f0 + p, t.n[0], tr.wrap[0]);
-                    for (int q = 0; q < m1; ++q) {
-                        const T w = w0 * rw[1][3 * c[1] + q];
-                        const int i1 = wrap_index(f1 + q, t.n[1], tr.wrap[1]);
-                        sum = sum + w * r[i0 * t.n[1] + i1];
-                    }
-                }
-            } else {
-                const int f2 = rf[2][c[2]], m2 = rn[2][c[2]];
-                for (int p = 0; p < m0; ++p) {
-                    const T w0 = rw[0][3 * c[0] + p];
-                    const int i0 = wrap_index(f0 + p, t.n[0], tr.wrap[0]);
-                    for (int q = 0; q < m1; ++q) {
-                        const T w01 = w0 * rw[1][3 * c[1] + q];
-                        const int i1 = wrap_index(f1 + q, t.n[1], tr.wrap[1]);
-                        const int row = (i0 * t.n[1] + i1) * t.n[2];
-                        for (int e = 0; e < m2; ++e) {
-                            const T w = w01 * rw[2][3 * c[2] + e];
-                            sum = sum + w * r[row + wrap_index(f2 + e, t.n[2], tr.wrap[2])];
-                        }
-                    }
-                }
-            }
-            const T bv = sum * cdinv[ccls[i]];
-            bc[i] = bv;
-            xc[i] = fs != (T)0 ? bv * (fs * (T)1) : (T)0;
-        }
-        cur &= ~(1u << (l + 1));
-        __syncthreads();
-    }
-    {
-        // x = Ainv b on the coarsest level: one wave per row, lane-strided
-        // FP64 partials and a butterfly (k_coarse_solve)
-        const int n = a.lev[Lc].N;
-        const T* b = reinterpret_cast<const T*>(lds + a.lev[Lc].ob);
-        T* x = reinterpret_cast<T*>(lds + a.lev[Lc].ox);
-        // rows wave, wave + 16, ... (at most kTailRows per wave) are summed
-        // together so that all their loads are in flight at once; each row
-        // still adds its terms in ascending j
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        double sacc[kTailRows];
-#pragma unroll
-        for (int k = 0; k < kTailRows; ++k) sacc[k] = 0.0;
-        for (int j = lane; j < n; j += 64) {
-            const double bj = (double)b[j];
-#pragma unroll
-            for (int k = 0; k < kTailRows; ++k) {
-                const int row = wave + k * (kTailThreads / 64);
-                if (row < n) sacc[k] += a.cinv[(int64_t)row * n + j] * bj;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < kTailRows; ++k) {
-            const int row = wave + k * (kTailThreads / 64);
-            const double v = wave_sum(sacc[k]);
-            if (row < n && lane == 0) x[row] = (T)v;
-        }
-        __syncthreads();
-    }
-    for (int l = Lc - 1; l >= 0; --l) {
-        const TailLevel<T>& t = a.lev[l];
-        const TailLevel<T>& cl = a.lev[l + 1];
-        const TailTransfer<T>& tr = a.tr[l];
-        const int* pc[3];
-        const T* pw[3];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            pc[d] = reinterpret_cast<const int*>(lds + tr.opc[d]);
-            pw[d] = reinterpret_cast<const T*>(lds + tr.opw[d]);
-        }
-        const T* xc = X(l + 1);
-        T* xf = X(l);
-        // x_f = (P x_c)*1 + x_f*(1*1)
-        for (int i = threadIdx.x; i < t.N; i += kTailThreads) {
-            int c[3];
-            tail_coords<D>(t, i, c);
-            T sum = (T)0;
-            const int p0 = pc[0][c[0]], p1 = pc[1][c[1]];
-            const T* w0 = pw[0] + 2 * c[0];
-            const T* w1 = pw[1] + 2 * c[1];
-            if constexpr (D == 2) {
-                for (int p = 0; p < 2; ++p) {
-                    if (w0[p] == (T)0) continue;
-                    const int i0 = wrap_index(p0 + p, cl.n[0], tr.wrap[0]);
-                    for (int q = 0; q < 2; ++q) {
-                        if (w1[q] == (T)0) continue;
-                        const int i1 = wrap_index(p1 + q, cl.n[1], tr.wrap[1]);
-                        sum = sum + (w0[p] * w1[q]) * xc[i0 * cl.n[1] + i1];
-                    }
-                }
-            } else {
-                const int p2 = pc[2][c[2]];
-                const T* w2 = pw[2] + 2 * c[2];
-                for (int p = 0; p < 2; ++p) {
-                    if (w0[p] == (T)0) continue;
-                    const int i0 = wrap_index(p0 + p, cl.n[0], tr.wrap[0]);
-                    for (int q = 0; q < 2; ++q) {
-                        if (w1[q] == (T)0) continue;
-                        const T w01 = w0[p] * w1[q];
-                        const int i1 = wrap_index(p1 + q, cl.n[1], tr.wrap[1]);
-                        for (int e = 0; e < 2; ++e) {
-                            if (w2[e] == (T)0) continue;
-                            const int i2 = wrap_index(p2 + e, cl.n[2], tr.wrap[2]);
-                            sum = sum + (w01 * w2[e]) * xc[(i0 * cl.n[1] + i1) * cl.n[2] + i2];
-                        }
-                    }
-                }
-            }
-            xf[i] = sum * (T)1 + xf[i] * (T)1;
-        }
-        __syncthreads();
-        for (int s = 0; s < a.post; ++s) {
-            tail_apply<T, D>(lds, t, t.orx, X(l), Y(l), (T)1, a.two3 * (T)1);
-            __syncthreads();
-            cur ^= 1u << l;
-        }
-    }
-    const T* x0 = X(0);
-    for (int i = threadIdx.x; i < a.lev[0].N; i += kTailThreads) a.x_out[i] = x0[i];
-}
-
 // ---- batched launches ------------------------------------------------------
 // A batched launch runs one kernel body for several independent solver
 // instances: instance i owns blocks first[i] .. first[i+1]-1 of the grid and
@@ -1412,40 +1080,177 @@ __global__ __launch_bounds__(kMgThreads) void k_hadamard_many(const HadamardArgs
     hadamard_body<T>(a[i], blockIdx.x - first[i]);
 }
 
-// x = Ainv b, one wave per row, fixed-order lane partials + butterfly.
-template <typename T>
+// x = M b with the dense coarse-end operator M (row-major, rows padded to ld
+// values; M is the V-cycle from the level down, or the coarsest inverse): one
+// wave per row, 16-byte loads of the row, products summed in FP64 in a fixed
+// order (lane partials, then a butterfly).  Bound by reading M: up to the
+// 32 MB of the eight L2s (a block's rows stay on its XCD from launch to
+// launch) n = 1024 takes 2.6 us and 2025 4.3 us in FP64, launch included;
+// beyond it the Infinity Cache gives about 6 TB/s (FP64 2856: 11 us, FP32
+// 4096: 12 us).  Two or four rows per wave, or a block per row pair, were no
+// faster.  b holds ld values (zeros beyond n).
+template <typename T, typename M>
 struct CoarseArgs {
-    const double* inv;
-    int n;
+    const M* op;
+    int n, ld;
     const T* b;
     T* x;
 };
 
-template <typename T>
-__device__ __forceinline__ void coarse_solve_body(const CoarseArgs<T>& a, unsigned bid)
+template <typename T, typename M>
+__device__ __forceinline__ void coarse_solve_body(const CoarseArgs<T, M>& a, unsigned bid)
 {
+    constexpr int V = 16 / (int)sizeof(M);
+    using vec = M __attribute__((ext_vector_type(16 / sizeof(M))));
     const int row = (int)(((int64_t)bid * kMgThreads + threadIdx.x) >> 6);
     const int lane = threadIdx.x & 63;
-    const int n = a.n;
-    if (row >= n) return;
+    if (row >= a.n) return;
+    const M* __restrict__ m = a.op + (int64_t)row * a.ld;
+    const T* __restrict__ b = a.b;
     double s = 0.0;
-    for (int j = lane; j < n; j += 64) s += a.inv[(int64_t)row * n + j] * (double)a.b[j];
-    s = wave_sum(s);
+#pragma unroll 4
+    for (int j = lane * V; j < a.ld; j += 64 * V) {
+        const vec v = *reinterpret_cast<const vec*>(m + j);
+#pragma unroll
+        for (int k = 0; k < V; ++k) s += (double)v[k] * (double)b[j + k];
+    }
+    s = wave_sum_full(s);
     if (lane == 0) a.x[row] = (T)s;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kMgThreads) void k_coarse_solve(CoarseArgs<T> a)
+template <typename T, typename M>
+__global__ __launch_bounds__(kMgThreads) void k_coarse_solve(CoarseArgs<T, M> a)
 {
-    coarse_solve_body<T>(a, blockIdx.x);
+    coarse_solve_body<T, M>(a, blockIdx.x);
 }
 
-template <typename T>
-__global__ __launch_bounds__(kMgThreads) void k_coarse_solve_many(const CoarseArgs<T>* __restrict__ a,
+template <typename T, typename M>
+__global__ __launch_bounds__(kMgThreads) void k_coarse_solve_many(const CoarseArgs<T, M>* __restrict__ a,
                                                                   const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
-    coarse_solve_body<T>(a[i], blockIdx.x - first[i]);
+    coarse_solve_body<T, M>(a[i], blockIdx.x - first[i]);
+}
+
+// ---- building the dense coarse-end operator --------------------------------
+// The V-cycle from level l down, started from zero, is linear in its
+// right-hand side: its matrix is built column by column in FP64 with the
+// level kernels' terms.  An N x N matrix of columns is stored row-major, so
+// row i holds node i's value in every column; blockIdx.y is the row (its
+// class and neighbours are uniform), threads run over the columns.
+
+// Y = beta (coef X) + gamma I  (X == nullptr: X = 0)
+template <int D>
+__global__ __launch_bounds__(kMgThreads) void k_dense_stencil(DevLevel L, const double* __restrict__ coef,
+                                                              const double* __restrict__ X, double* __restrict__ Y,
+                                                              double beta, double gamma)
+{
+    const int j = (int)(blockIdx.x * kMgThreads + threadIdx.x);
+    const int64_t i = blockIdx.y, N = L.N;
+    if (j >= N) return;
+    constexpr int KS = D == 2 ? 9 : 27;
+    double s = 0.0;
+    if (X) {
+        int c[3] = {0, 0, 0};
+        node_coords<D>(L, i, c);
+        const double* row = coef + (int64_t)L.cls[i] * KS;
+        for (int k = 0; k < KS; ++k) {
+            const double v = row[k];
+            if (v == 0.0) continue;
+            const int o[3] = {D == 2 ? k / 3 - 1 : k / 9 - 1, D == 2 ? k % 3 - 1 : (k / 3) % 3 - 1, D == 2 ? 0 : k % 3 - 1};
+            int64_t q = 0;
+            for (int d = 0; d < D; ++d) q = q * L.n[d] + nb_index(c[d], o[d], L.n[d], L.wrap[d]);
+            s = s + v * X[q * N + j];
+        }
+    }
+    Y[i * N + j] = beta * s + (i == j ? gamma : 0.0);
+}
+
+// B = (R r) o D_c^-1 for every column
+template <int D>
+__global__ __launch_bounds__(kMgThreads) void k_dense_restrict(DevLevel F, DevLevel Cl, DevTransfer<double> tr,
+                                                               const double* __restrict__ dinv,
+                                                               const double* __restrict__ r, double* __restrict__ B)
+{
+    const int j = (int)(blockIdx.x * kMgThreads + threadIdx.x);
+    const int64_t i = blockIdx.y, N = F.N;
+    if (j >= N) return;
+    int c[3] = {0, 0, 0};
+    node_coords<D>(Cl, i, c);
+    double s = 0.0;
+    for (int a = 0; a < tr.rn[0][c[0]]; ++a)
+        for (int b = 0; b < tr.rn[1][c[1]]; ++b)
+            for (int e = 0; e < (D == 3 ? tr.rn[2][c[2]] : 1); ++e) {
+                double w = tr.rw[0][3 * c[0] + a] * tr.rw[1][3 * c[1] + b];
+                int64_t q = (int64_t)wrap_index(tr.rf[0][c[0]] + a, F.n[0], tr.wrap[0]) * F.n[1] +
+                            wrap_index(tr.rf[1][c[1]] + b, F.n[1], tr.wrap[1]);
+                if (D == 3) {
+                    w = w * tr.rw[2][3 * c[2] + e];
+                    q = q * F.n[2] + wrap_index(tr.rf[2][c[2]] + e, F.n[2], tr.wrap[2]);
+                }
+                s = s + w * r[q * N + j];
+            }
+    B[i * N + j] = s * dinv[Cl.cls[i]];
+}
+
+// X += P E for every column
+template <int D>
+__global__ __launch_bounds__(kMgThreads) void k_dense_prolong(DevLevel F, DevLevel Cl, DevTransfer<double> tr,
+                                                              const double* __restrict__ E, double* __restrict__ X)
+{
+    const int j = (int)(blockIdx.x * kMgThreads + threadIdx.x);
+    const int64_t i = blockIdx.y, N = F.N;
+    if (j >= N) return;
+    int c[3] = {0, 0, 0};
+    node_coords<D>(F, i, c);
+    double s = 0.0;
+    for (int h = 0; h < (1 << D); ++h) {
+        double w = 1.0;
+        int64_t q = 0;
+        for (int d = 0; d < D; ++d) {
+            const int o = (h >> (D - 1 - d)) & 1;
+            const double f = tr.pw[d][2 * c[d] + o];
+            w = w * f;
+            // a zero weight's node may lie outside the axis: not read
+            q = q * Cl.n[d] + (f == 0.0 ? 0 : wrap_index(tr.pc[d][c[d]] + o, Cl.n[d], tr.wrap[d]));
+        }
+        if (w != 0.0) s = s + w * E[q * N + j];
+    }
+    X[i * N + j] += s;
+}
+
+// E (m x n) = A (m x m) B (m x n), 32 x 32 tiles through LDS, FP64
+__global__ __launch_bounds__(kMgThreads) void k_dense_product(int m, int n, const double* __restrict__ A,
+                                                              const double* __restrict__ B, double* __restrict__ E)
+{
+    __shared__ double sa[32][33], sb[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;     // 32 x 8
+    const int r0 = (int)blockIdx.y * 32, c0 = (int)blockIdx.x * 32;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < m; k0 += 32) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = ty + 8 * q;
+            sa[r][tx] = (r0 + r < m && k0 + tx < m) ? A[(int64_t)(r0 + r) * m + k0 + tx] : 0.0;
+            sb[r][tx] = (k0 + r < m && c0 + tx < n) ? B[(int64_t)(k0 + r) * n + c0 + tx] : 0.0;
+        }
+        __syncthreads();
+        for (int k = 0; k < 32; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s[q] += sa[ty + 8 * q][k] * sb[k][tx];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (r0 + ty + 8 * q < m && c0 + tx < n) E[(int64_t)(r0 + ty + 8 * q) * n + c0 + tx] = s[q];
+}
+
+// rows of n values -> rows of ld values of type M, zeros beyond n
+template <typename M>
+__global__ __launch_bounds__(kMgThreads) void k_dense_pad(int n, int ld, const double* __restrict__ A, M* __restrict__ out)
+{
+    const int j = (int)(blockIdx.x * kMgThreads + threadIdx.x);
+    if (j < ld) out[(int64_t)blockIdx.y * ld + j] = j < n ? (M)A[(int64_t)blockIdx.y * n + j] : (M)0;
 }
 
 // FP64 residual of the unscaled operator: r = b - A x, partial sums of r^2
@@ -2232,42 +2037,15 @@ struct DevTransferBuf {
 
 namespace psum_hip {
 
-// k_vtail<T, D>'s dynamic LDS limit on the current device: raised once per
-// device, precision and dimension to the device's per-workgroup maximum (the
-// attribute is process-wide, so every solver shares the one largest
-// value), and returned.  Called when a hierarchy is built, outside any
-// stream capture.
-template <typename T, int D>
-int vtail_lds_limit()
-{
-    static std::mutex mu;
-    static std::map<int, int> limit;
-    int dev = 0;
-    MG_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = limit.find(dev);
-    if (it != limit.end()) return it->second;
-    int lim = 0;
-    MG_HIP(hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    if (lim > 65536 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_vtail<T, D>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, lim) != hipSuccess) {
-        (void)hipGetLastError();
-        lim = 65536;
-    }
-    limit[dev] = lim;
-    return lim;
-}
-
 // kernel kinds of recorded ops (base + template variant bits)
 constexpr uint16_t kKindSmooth = 0;      // + (FP64 << 3 | compact << 2 | prolong << 1 | acc)
 constexpr uint16_t kKindRRTile = 16;     // + (FP64 << 1 | compact)
 constexpr uint16_t kKindRR = 20;         // + (FP64 << 1 | compact)
-constexpr uint16_t kKindCoarse = 24;     // + FP64
-constexpr uint16_t kKindOuter = 26;      // + (norms << 2 | compact << 1 | emit FP32), 2D
-constexpr uint16_t kKindVec = 34;        // + op (0 zero, 1 add correction, 2 copy)
-constexpr uint16_t kKindHadamard = 37;   // FP64
-constexpr uint16_t kKindCount = 38;
+constexpr uint16_t kKindCoarse = 24;     // + (0 FP32 vectors with an FP64 operator, 1 FP64, 2 FP32)
+constexpr uint16_t kKindOuter = 27;      // + (norms << 2 | compact << 1 | emit FP32), 2D
+constexpr uint16_t kKindVec = 35;        // + op (0 zero, 1 add correction, 2 copy)
+constexpr uint16_t kKindHadamard = 38;   // FP64
+constexpr uint16_t kKindCount = 39;
 
 class HipMultigrid {
 public:
@@ -2280,6 +2058,7 @@ public:
         std::istringstream iss(options ? options : "");
         std::string key;
         bool k_provided = false;
+        const int pre0 = pre_, post0 = post_;
         while (iss >> key) {
             if (key == "I") iss >> I_;
             else if (key == "J") iss >> J_;
@@ -2294,24 +2073,28 @@ public:
                 corr_ = v;
             } else if (key == "tol") iss >> tol_;
             else if (key == "periodic_mode") iss >> periodic_mode_;
-            else if (key == "fuse") { iss >> fuse_; resolve_tail(); }
-            else if (key == "tail") { iss >> tail_; resolve_tail(); }
-            else if (key == "line") { iss >> line_; }
+            else if (key == "fuse") iss >> fuse_;
+            else if (key == "line") iss >> line_;
             else if (key == "graph") iss >> use_graph_;
             else if (key == "num_conv_mask" || key == "num_conv_mask_relax" ||
                      key == "num_conv_mask_restrict" || key == "num_conv_mask_interpolate" ||
-                     key == "num_conv_mask_a") {
+                     key == "num_conv_mask_a" || key == "tail") {
                 int ignored;
                 iss >> ignored;
             }
         }
         if (!k_provided) K_ = 1;
+        if (!host_.empty() && (pre_ != pre0 || post_ != post0)) {
+            drop_graphs();
+            build_operator();
+        }
     }
 
     // Kernel-shape options that may change after set_matrix: "fuse 0|1"
-    // (2D fused tile kernels), "tail 0|1" (the one-workgroup coarse end) and
-    // "line 0|1" (chunked sweeps and residuals on 7-point 3D levels).
-    // Other keys are rejected.
+    // (2D fused tile kernels) and "line 0|1" (chunked sweeps and residuals on
+    // 7-point 3D levels).  "tail 0|1" is accepted and has no effect: the
+    // coarse end is one dense product (build_operator).  Other keys are
+    // rejected.
     void set_tuning(const char* options)
     {
         std::istringstream iss(options ? options : "");
@@ -2319,13 +2102,12 @@ public:
         while (iss >> key) {
             int v = 0;
             if (!(iss >> v)) throw std::invalid_argument("hip_multigrid: tuning option " + key + " needs a value");
-            if (key == "tail") tail_ = v;
+            if (key == "tail") continue;
             else if (key == "fuse") fuse_ = v;
             else if (key == "line") line_ = v;
             else throw std::invalid_argument("hip_multigrid: unknown tuning option " + key);
         }
         rr_fit_.clear();
-        resolve_tail();
         drop_graphs();   // captured cycles hold the previous kernel shapes
     }
 
@@ -2339,8 +2121,8 @@ public:
         pre_ = pre;
         post_ = post;
         rr_fit_.clear();
-        resolve_tail();
         drop_graphs();
+        if (!host_.empty()) build_operator();
     }
 
     void set_stream(hipStream_t s) { stream_ = s; }
@@ -2403,7 +2185,7 @@ public:
         tr_host_ = std::move(T);
         rr_fit_.clear();
         upload();
-        resolve_tail();
+        build_operator();
     }
 
     void set_source_replace(unsigned long long n, const unsigned long long* idx, const double* v)
@@ -2543,14 +2325,13 @@ public:
     using RecOp = MgRecOp;
 
     // whether the core of a solve can be recorded: a fixed cycle count on a
-    // 2D hierarchy through the fused tile kernels, without the one-workgroup
-    // tail, with pre- and post-sweeps
+    // 2D hierarchy through the fused tile kernels, with pre- and post-sweeps
     bool recordable() const
     {
         if (host_.empty() || tol_ > 0.0 || host_[0].D != 2 || !fuse_ || pre_ < 1 || post_ < 1) return false;
         for (const auto& h : host_)
             if (h.D != 2) return false;
-        return tail_start<float>() < 0 && tail_start<double>() < 0;
+        return true;
     }
 
     // The ops of solve_core(b, bs, x), in order, without launching anything
@@ -2580,8 +2361,11 @@ public:
         max_cycles_ = cycles;
         corr_ = 1;
         use_graph_ = 0;
-        for (auto& c : cap64_.e) drop_graph(c);
-        for (auto& c : cap32_.e) drop_graph(c);
+        drop_graphs();
+        if (!fixed_mode_) {
+            fixed_mode_ = true;
+            if (!host_.empty()) build_operator();
+        }
     }
 
     int last_cycles() const { return last_cycles_; }
@@ -2637,11 +2421,11 @@ private:
         else hipLaunchKernelGGL((k_resid_restrict<T, C>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
     }
 
-    template <typename T>
-    void run_coarse(unsigned nb, const CoarseArgs<T>& a)
+    template <typename T, typename M>
+    void run_coarse(unsigned nb, const CoarseArgs<T, M>& a)
     {
-        if (rec_) { emit((uint16_t)(kKindCoarse + tbit<T>()), nb, a); return; }
-        hipLaunchKernelGGL((k_coarse_solve<T>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
+        if (rec_) { emit((uint16_t)(kKindCoarse + (tbit<T>() ? 1 : (tbit<M>() ? 0 : 2))), nb, a); return; }
+        hipLaunchKernelGGL((k_coarse_solve<T, M>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
     }
 
     template <int D, bool C, bool F32, bool NORMS>
@@ -2674,12 +2458,12 @@ private:
     int I_ = 0, J_ = 0, K_ = 0, depth_ = 3, pre_ = 2, post_ = 1, max_cycles_ = 10, corr_ = 4;
     int fuse_ = 1;   // 2D: fused multi-sweep tile smoothing and residual+restriction
     int line_ = 1;   // 3D 7-point levels: chunk kernels (k_smooth_line, k_residual_line)
-    // the coarse end of the V-cycle in one workgroup (k_vtail); off unless
-    // "tail 1" is set (measured: the levels' own launches are about as fast,
-    // in 2D and in 3D)
-    int tail_ = 0;
-    int tail32_ = -2, tail64_ = -2;    // first tail level per precision (-1 none, -2 not yet chosen)
-    size_t tail_bytes32_ = 0, tail_bytes64_ = 0;
+    // the coarse end as one dense operator: levels op_level_ and below
+    int op_level_ = 0;                 // the coarsest level when nothing is merged
+    int op_ld_ = 0, op_pre_ = -1, op_post_ = -1;
+    bool op_f32_ = false;
+    void* op_ = nullptr;
+    bool fixed_mode_ = false;          // set_fixed_cycles was called
     std::vector<int> rr_fit_;
     double tol_ = 0.0;
     int predicted_ = 1;                // cycles the previous solve needed
@@ -2693,7 +2477,6 @@ private:
     std::vector<double> cinv_host_;
     std::vector<DevLevelBuf> dev_;
     std::vector<DevTransferBuf> dtr_;
-    double* cinv_ = nullptr;
     double* part_ = nullptr;
     double* red_ = nullptr;
     double* red_host_ = nullptr;
@@ -2742,7 +2525,7 @@ private:
                                 (void*)t.rw[d], (void*)t.pw32[d], (void*)t.rw32[d]})
                     if (p) (void)hipFree(p);
         dtr_.clear();
-        if (cinv_) (void)hipFree(cinv_);
+        release_operator();
         if (part_) (void)hipFree(part_);
         if (red_) (void)hipFree(red_);
         if (red_host_) (void)hipHostFree(red_host_);
@@ -2750,7 +2533,6 @@ private:
         if (bprime_) (void)hipFree(bprime_);
         shift_ = nullptr;
         bprime_ = nullptr;
-        cinv_ = nullptr;
         part_ = nullptr;
         red_ = nullptr;
         red_host_ = nullptr;
@@ -2775,12 +2557,13 @@ private:
             const size_t N = (size_t)h.N;
             if (!mixed_) {
                 if (l > 0) MG_HIP(hipMalloc(&d.x, N * sizeof(double)));
-                if (l > 0) MG_HIP(hipMalloc(&d.b, N * sizeof(double)));
-                else MG_HIP(hipMalloc(&d.b, N * sizeof(double)));
+                MG_HIP(hipMalloc(&d.b, (N + kOpPad) * sizeof(double)));
+                MG_HIP(hipMemset(d.b + N, 0, kOpPad * sizeof(double)));   // read beyond N by the dense product
                 MG_HIP(hipMalloc(&d.t, N * sizeof(double)));
             } else {
                 MG_HIP(hipMalloc(&d.xf, N * sizeof(float)));
-                MG_HIP(hipMalloc(&d.bf, N * sizeof(float)));
+                MG_HIP(hipMalloc(&d.bf, (N + kOpPad) * sizeof(float)));
+                MG_HIP(hipMemset(d.bf + N, 0, kOpPad * sizeof(float)));
                 MG_HIP(hipMalloc(&d.tf, N * sizeof(float)));
             }
         }
@@ -2796,13 +2579,13 @@ private:
                 dtr_[l].pw32[d] = dev_copy(cast_vec<float>(t.pw));
                 dtr_[l].rw32[d] = dev_copy(cast_vec<float>(t.rw));
             }
-        cinv_ = dev_copy(cinv_host_);
         const int64_t nb = (int64_t)nblk(host_[0].N);
         MG_HIP(hipMalloc(&part_, (size_t)nb * 2 * sizeof(double)));
         MG_HIP(hipMalloc(&red_, 2 * sizeof(double)));
         MG_HIP(hipMalloc(&shift_, 4 * sizeof(double)));
         if (pin_ >= 0) MG_HIP(hipMalloc(&bprime_, (size_t)host_[0].N * sizeof(double)));
         MG_HIP(hipHostMalloc(&red_host_, 2 * sizeof(double), hipHostMallocDefault));
+        MG_HIP(hipStreamSynchronize(nullptr));   // the clears above, before work on other streams
     }
 
     // A 3D level of at least 2^16 nodes (and fewer than 2^32) runs its
@@ -3041,146 +2824,143 @@ private:
             hipLaunchKernelGGL((k_prolong_add<T, 3>), dim3(nblk(F.N)), dim3(kMgThreads), 0, stream_, F, C, transfer<T>(l), xc, x);
     }
 
-    // First level of the one-workgroup tail for precision T, or -1: a 2D
-    // fused or a 3D hierarchy whose levels lt..Lc (two or more, at most
-    // kMaxTail, lt >= 1, at most tail_level_nodes<D> nodes each) keep their
-    // iterates and right-hand sides in LDS and whose coarsest level has at
-    // most tail_coarse<D> nodes (its dense solve reads the inverse from one
-    // compute unit).
-    // Chosen by resolve_tail() when the hierarchy is built or the option
-    // changes, never while a stream is being captured.
-    template <typename T>
-    int tail_start() const
-    {
-        const int c = std::is_same<T, double>::value ? tail64_ : tail32_;
-        if (c == -2) throw std::logic_error("hip_multigrid: V-cycle tail used before it was resolved");
-        return c;
-    }
-
-    template <typename T>
-    void resolve_tail_for()
-    {
-        int& c = std::is_same<T, double>::value ? tail64_ : tail32_;
-        size_t& bytes = std::is_same<T, double>::value ? tail_bytes64_ : tail_bytes32_;
-        c = -1;
-        bytes = 0;
-        const int nl = (int)host_.size(), Lc = nl - 1;
-        if (nl < 3) return;
-        const int D = host_[0].D;
-        if (D != 2 && D != 3) return;
-        for (const auto& h : host_)
-            if (h.D != D) return;
-        if (tail_ != 1 || (D == 2 && !fuse_)) return;
-        const int64_t coarse = D == 2 ? tail_coarse<2>() : tail_coarse<3>();
-        const int64_t maxn = D == 2 ? tail_level_nodes<2>() : tail_level_nodes<3>();
-        if (host_[Lc].N > coarse) return;
-        const int lim = D == 2 ? vtail_lds_limit<T, 2>() : vtail_lds_limit<T, 3>();
-        for (int lt = 1; lt <= Lc - 1; ++lt) {
-            if (Lc - lt + 1 > kMaxTail || host_[lt].N > maxn) continue;
-            TailArgs<T> probe{};
-            const size_t b = tail_layout<T>(lt, probe);
-            if (b > (size_t)lim) continue;
-            c = lt;
-            bytes = b;
-            break;
-        }
-    }
-
-    // Both precisions' tails for the current hierarchy and options.
-    void resolve_tail()
-    {
-        if (host_.empty()) {
-            tail32_ = tail64_ = -2;
-            return;
-        }
-        resolve_tail_for<float>();
-        resolve_tail_for<double>();
-    }
-
-    // Fills the tail arguments for levels lt..Lc; returns the LDS bytes
-    template <typename T>
-    size_t tail_layout(int lt, TailArgs<T>& a) const
+    // ---- the coarse end as one dense operator -----------------------------
+    // The V-cycle from a level l >= 1 down starts from zero, so it is the
+    // product of its right-hand side with a fixed N_l x N_l matrix (built once
+    // per matrix and smoothing counts, k_dense_*).  One product replaces every
+    // launch of the levels it covers: 3 per 2D level (5-7 us each), 2 + pre +
+    // post per 3D level (3.7-11 us each).  The level taken is the finest whose
+    // matrix is small enough to beat those launches:
+    //   2D  33 MB: FP64 2048 nodes 4.3 us (16-18 us for the level's launches),
+    //       4096 nodes 21 us, no faster than the launches; FP32 to 67 MB,
+    //       4096 nodes 12 us against 17 + 2.8 us
+    //   3D  200 MB: 17^3 nodes 28 us (FP64) / 17 us (FP32) against 45-60 us
+    // Fixed-cycle solves (batches of many solvers, whose matrices share the
+    // caches) take at most 1089 nodes.
+    // FP32 V-cycles take the matrix in FP32 (built in FP64, products summed in
+    // FP64) where levels are merged, and the coarsest inverse alone in FP64.
+    int operator_level() const
     {
         const int Lc = (int)host_.size() - 1;
-        const int D = host_[lt].D;
-        const int K = D == 2 ? 9 : 27;
-        size_t off = 0;
-        auto take = [&](size_t nbytes) {
-            const size_t o = off;
-            off = (off + nbytes + 15) & ~(size_t)15;
-            return (int)o;
-        };
-        a.nl = Lc - lt + 1;
-        for (int k = 0; k < a.nl; ++k) {
-            const int l = lt + k;
-            const HostLevel& h = host_[l];
-            TailLevel<T>& t = a.lev[k];
-            for (int d = 0; d < 3; ++d) {
-                t.n[d] = d < D ? (int)h.n[d] : 1;
-                t.wrap[d] = d < D ? h.wrap[d] : 0;
-            }
-            t.N = (int)h.N;
-            t.compact = h.compact ? 1 : 0;
-            t.ncls = (int)h.dinv.size();
-            t.ox = take((size_t)h.N * sizeof(T));
-            t.oy = l < Lc ? take((size_t)h.N * sizeof(T)) : t.ox;
-            t.ob = take((size_t)h.N * sizeof(T));
-            t.ocls = take((size_t)h.N * sizeof(uint16_t));
-            t.orx = take((size_t)t.ncls * K * sizeof(T));
-            t.oa = take((size_t)t.ncls * K * sizeof(T));
-            t.odinv = take((size_t)t.ncls * sizeof(T));
-            if (!dev_.empty()) {
-                const DevTable<T> rx = table<T>(l, true), A = table<T>(l, false);
-                t.cls = dev_[l].cls;
-                t.rx = rx.coef;
-                t.a = A.coef;
-                t.dinv = A.dinv;
-            }
+        const int64_t limit = host_[0].D == 3 ? 200000000 : (mixed_ ? 67200000 : 33600000);
+        for (int l = 1; l < Lc; ++l) {
+            const int64_t n = host_[l].N;
+            if (fixed_mode_ ? n <= 1089 : (n < 32768 && n * n * (mixed_ ? 4 : 8) <= limit)) return l;
         }
-        for (int k = 0; k + 1 < a.nl; ++k) {
-            const int l = lt + k;
-            const HostLevel &f = host_[l], &c = host_[l + 1];
-            TailTransfer<T>& r = a.tr[k];
-            const DevTransfer<T> dt = dtr_.empty() ? DevTransfer<T>{} : transfer<T>(l);
-            for (int d = 0; d < D; ++d) {
-                r.wrap[d] = tr_host_[l][d].wrap;
-                r.orf[d] = take((size_t)c.n[d] * sizeof(int));
-                r.orn[d] = take((size_t)c.n[d] * sizeof(int));
-                r.orw[d] = take((size_t)3 * c.n[d] * sizeof(T));
-                r.opc[d] = take((size_t)f.n[d] * sizeof(int));
-                r.opw[d] = take((size_t)2 * f.n[d] * sizeof(T));
-                if (!dtr_.empty()) {
-                    r.rf[d] = dt.rf[d];
-                    r.rn[d] = dt.rn[d];
-                    r.rw[d] = dt.rw[d];
-                    r.pc[d] = dt.pc[d];
-                    r.pw[d] = dt.pw[d];
-                }
-            }
-        }
-        return off;
+        return Lc;
     }
 
-    template <typename T>
-    void launch_tail(int lt, T* x, const T* b)
+    void release_operator()
     {
-        TailArgs<T> a{};
-        const size_t bytes = tail_layout<T>(lt, a);
-        a.pre = pre_;
-        a.post = post_;
-        a.two3 = (T)(2.0 / 3);
-        a.x_in = x;
-        a.b_in = b;
-        a.x_out = x;
-        a.cinv = cinv_;
-        const int D = host_[lt].D;
-        const int lim = D == 2 ? vtail_lds_limit<T, 2>() : vtail_lds_limit<T, 3>();
-        const size_t chosen = std::is_same<T, double>::value ? tail_bytes64_ : tail_bytes32_;
-        if (bytes != chosen || bytes > (size_t)lim)
-            throw std::logic_error("hip_multigrid: V-cycle tail LDS size differs from the one resolved");
-        if (D == 2) hipLaunchKernelGGL((k_vtail<T, 2>), dim3(1), dim3(kTailThreads), bytes, stream_, a);
-        else hipLaunchKernelGGL((k_vtail<T, 3>), dim3(1), dim3(kTailThreads), bytes, stream_, a);
+        if (op_) (void)hipFree(op_);
+        op_ = nullptr;
+        op_level_ = (int)host_.size() - 1;
+        op_pre_ = op_post_ = -1;
+    }
+
+    // device memory released when the scope is left
+    struct Scratch {
+        std::vector<void*> p;
+        ~Scratch() { for (void* q : p) (void)hipFree(q); }
+        double* take(size_t n)
+        {
+            void* q = nullptr;
+            MG_HIP(hipMalloc(&q, std::max<size_t>(1, n) * sizeof(double)));
+            p.push_back(q);
+            return static_cast<double*>(q);
+        }
+        void drop(double* q)
+        {
+            p.erase(std::find(p.begin(), p.end(), (void*)q));
+            (void)hipFree(q);
+        }
+    };
+
+    // the operator for the current hierarchy, smoothing counts and cycle mode;
+    // without memory for a merged one, the coarsest inverse alone
+    void build_operator()
+    {
+        const int l = operator_level();
+        const bool merged = l < (int)host_.size() - 1;
+        if (op_ && l == op_level_ && (!merged || (pre_ == op_pre_ && post_ == op_post_))) return;
+        drop_graphs();
+        release_operator();
+        if (merged) {
+            try {
+                build_operator_at(l);
+                return;
+            } catch (const std::runtime_error&) {
+                (void)hipGetLastError();
+                release_operator();
+            }
+        }
+        build_operator_at((int)host_.size() - 1);
+    }
+
+    void build_operator_at(int target)
+    {
+        const int Lc = (int)host_.size() - 1;
+        struct Stream {
+            hipStream_t s = nullptr;
+            ~Stream() { if (s) (void)hipStreamDestroy(s); }
+        } own;
+        MG_HIP(hipStreamCreateWithFlags(&own.s, hipStreamNonBlocking));
+        hipStream_t st = own.s;
+        Scratch mem;
+        double* M = mem.take(cinv_host_.size());
+        MG_HIP(hipMemcpy(M, cinv_host_.data(), cinv_host_.size() * sizeof(double), hipMemcpyHostToDevice));
+        for (int l = Lc - 1; l >= target; --l) {
+            double* X = host_[l].D == 2 ? operator_columns<2>(l, M, mem, st) : operator_columns<3>(l, M, mem, st);
+            mem.drop(M);
+            M = X;
+        }
+        const int n = (int)host_[target].N;
+        op_f32_ = mixed_ && target < Lc;
+        const int v = op_f32_ ? 4 : 2;
+        op_ld_ = (n + v - 1) / v * v;
+        MG_HIP(hipMalloc(&op_, (size_t)n * op_ld_ * (op_f32_ ? sizeof(float) : sizeof(double))));
+        const dim3 grid(nblk(op_ld_), n);
+        if (op_f32_) hipLaunchKernelGGL(k_dense_pad<float>, grid, dim3(kMgThreads), 0, st, n, op_ld_, M, static_cast<float*>(op_));
+        else hipLaunchKernelGGL(k_dense_pad<double>, grid, dim3(kMgThreads), 0, st, n, op_ld_, M, static_cast<double*>(op_));
         MG_HIP(hipGetLastError());
+        MG_HIP(hipStreamSynchronize(st));
+        op_level_ = target;
+        op_pre_ = pre_;
+        op_post_ = post_;
+    }
+
+    // the V-cycle from level l down applied to every unit vector: pre-sweeps
+    // from zero, residual, restriction, the next level's operator M,
+    // prolongation, post-sweeps
+    template <int D>
+    double* operator_columns(int l, const double* M, Scratch& mem, hipStream_t st)
+    {
+        const DevLevel F = dl(l), C = dl(l + 1);
+        const size_t n = (size_t)F.N, m = (size_t)C.N;
+        const double two3 = 2.0 / 3;
+        const DevTable<double> rx{dev_[l].Rx, dev_[l].dinv}, ah{dev_[l].Ah, dev_[l].dinv};
+        double *X = mem.take(n * n), *Y = mem.take(n * n), *B = mem.take(m * n), *E = mem.take(m * n);
+        const dim3 th(kMgThreads), gf(nblk(F.N), (unsigned)n), gc(nblk(F.N), (unsigned)m);
+        // sweep from zero: (2/3) I; no pre-sweeps: 0
+        hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, rx.coef, (const double*)nullptr, X, 0.0, pre_ > 0 ? two3 : 0.0);
+        for (int k = 1; k < pre_; ++k) {
+            hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, rx.coef, X, Y, 1.0, two3);
+            std::swap(X, Y);
+        }
+        hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, ah.coef, X, Y, -1.0, 1.0);
+        hipLaunchKernelGGL(k_dense_restrict<D>, gc, th, 0, st, F, C, transfer<double>(l), dev_[l + 1].dinv, Y, B);
+        hipLaunchKernelGGL(k_dense_product, dim3((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32)), th, 0, st, (int)m, (int)n, M, B, E);
+        hipLaunchKernelGGL(k_dense_prolong<D>, gf, th, 0, st, F, C, transfer<double>(l), E, X);
+        for (int k = 0; k < post_; ++k) {
+            hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, rx.coef, X, Y, 1.0, two3);
+            std::swap(X, Y);
+        }
+        MG_HIP(hipGetLastError());
+        MG_HIP(hipStreamSynchronize(st));
+        mem.drop(Y);
+        mem.drop(B);
+        mem.drop(E);
+        return X;
     }
 
     // One or more V-cycles on level-0 arrays (b0 scaled, x0 warm start).
@@ -3192,12 +2972,9 @@ private:
     bool vcycles(std::vector<T*>& xs, std::vector<T*>& ts, std::vector<T*>& bs, int cycles,
                  bool first_swept = false, double* acc = nullptr)
     {
-        const int nl = (int)host_.size();
-        const int Lc = nl - 1;
         const T two3 = (T)(2.0 / 3);
         bool accd = false;
-        const int lt = tail_start<T>();          // > 0: levels lt..Lc run in k_vtail
-        const int ld = lt > 0 ? lt : Lc;
+        const int ld = op_level_;                // this level and those below: one dense product
         for (int cyc = 0; cyc < cycles; ++cyc) {
             const uint32_t it = rec_iter_ + (uint32_t)cyc;
             for (int l = 0; l < ld; ++l) {
@@ -3206,7 +2983,7 @@ private:
                 const bool swept = (l > 0 || (cyc == 0 && first_swept)) && pre_ > 0;
                 smooth_n<T>(l, xs[l], ts[l], bs[l], swept ? pre_ - 1 : pre_);
                 const DevLevel F = dl(l), C = dl(l + 1);
-                const T fs = (l + 1 < Lc && pre_ > 0) ? two3 : (T)0;
+                const T fs = (l + 1 < ld && pre_ > 0) ? two3 : (T)0;
                 if (host_[l].D == 2 && fuse_) {
                     if (rr_tile_fits(l)) {
                         const unsigned nbt = (unsigned)(((C.n[0] + kRRRows - 1) / kRRRows) * ((C.n[1] + kRRCols - 1) / kRRCols));
@@ -3230,12 +3007,13 @@ private:
                     hipLaunchKernelGGL((k_restrict<T, 3>), dim3(nblk(C.N)), dim3(kMgThreads), 0, stream_, F, C, transfer<T>(l), table<T>(l + 1, false), ts[l], bs[l + 1], xs[l + 1], fs);
             }
             rec_phase(it, kStageCoarse, 0);
-            if (lt > 0) {
-                launch_tail<T>(lt, xs[lt], bs[lt]);
+            const int n = (int)host_[ld].N;
+            const unsigned nb = (unsigned)(((int64_t)n * 64 + kMgThreads - 1) / kMgThreads);
+            if constexpr (std::is_same<T, float>::value) {
+                if (op_f32_) run_coarse<T, float>(nb, CoarseArgs<T, float>{static_cast<const float*>(op_), n, op_ld_, bs[ld], xs[ld]});
+                else run_coarse<T, double>(nb, CoarseArgs<T, double>{static_cast<const double*>(op_), n, op_ld_, bs[ld], xs[ld]});
             } else {
-                const int n = (int)host_[Lc].N;
-                const unsigned nb = (unsigned)(((int64_t)n * 64 + kMgThreads - 1) / kMgThreads);
-                run_coarse<T>(nb, CoarseArgs<T>{cinv_, n, bs[Lc], xs[Lc]});
+                run_coarse<T, double>(nb, CoarseArgs<T, double>{static_cast<const double*>(op_), n, op_ld_, bs[ld], xs[ld]});
             }
             for (int l = ld - 1; l >= 0; --l) {
                 rec_phase(it, kStageUp, 255u - (uint32_t)l);
@@ -3562,12 +3340,13 @@ void mg_batch_launch(const MgBatchPlan& plan, hipStream_t st)
             }
 #undef RRL
         } else if (k < kKindOuter) {
-            if (k - kKindCoarse)
-                hipLaunchKernelGGL((k_coarse_solve_many<double>), grid, dim3(kMgThreads), 0, st,
-                                   static_cast<const CoarseArgs<double>*>(a), f, g.n);
-            else
-                hipLaunchKernelGGL((k_coarse_solve_many<float>), grid, dim3(kMgThreads), 0, st,
-                                   static_cast<const CoarseArgs<float>*>(a), f, g.n);
+#define COARSE(T, M) hipLaunchKernelGGL((k_coarse_solve_many<T, M>), grid, dim3(kMgThreads), 0, st, static_cast<const CoarseArgs<T, M>*>(a), f, g.n)
+            switch (k - kKindCoarse) {
+            case 0: COARSE(float, double); break;
+            case 1: COARSE(double, double); break;
+            default: COARSE(float, float); break;
+            }
+#undef COARSE
         } else if (k < kKindVec) {
             const OuterArgs* oa = static_cast<const OuterArgs*>(a);
 #define OUT(C, F, N) hipLaunchKernelGGL((k_outer_residual_many<2, C, F, N>), grid, dim3(kMgThreads), 0, st, oa, f, g.n)

@@ -30,8 +30,8 @@ struct MgBatchPlan;
 const double* mg_solve_begin(HipMultigrid* h, double* b);
 void mg_solve_core(HipMultigrid* h, const double* b, const double* bs, double* x);
 void mg_solve_end(HipMultigrid* h, const double* b, double* x);
-// whether the core can be recorded (2D fused hierarchy, fixed cycle count,
-// no one-workgroup tail), the right-hand side the core reads, and its ops
+// whether the core can be recorded (2D fused hierarchy, fixed cycle count),
+// the right-hand side the core reads, and its ops
 bool mg_recordable(HipMultigrid* h);
 const double* mg_core_rhs(HipMultigrid* h, double* b);
 void mg_record_core(HipMultigrid* h, const double* b, const double* bs, double* x, std::vector<MgRecOp>& ops);

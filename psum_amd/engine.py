@@ -561,8 +561,8 @@ class Stepper:
         return out
 
     def mg_tuning(self, options):
-        """Multigrid kernel-shape options ("fuse 0|1", "tail 0|1", "line 0|1");
-        results are bit-identical either way (psum_stepper_mg_tuning)."""
+        """Multigrid kernel-shape options ("fuse 0|1", "line 0|1"; "tail"
+        is accepted without effect); results are bit-identical either way (psum_stepper_mg_tuning)."""
         check(lib().psum_stepper_mg_tuning(self.h, options.encode()), "mg_tuning")
 
     def set_smoothing(self, pre, post):

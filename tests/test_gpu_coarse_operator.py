@@ -1,0 +1,116 @@
+"""The coarse end of the V-cycle as one dense product (levels small enough
+are merged into the matrix of the V-cycle from that level down): the iterates
+are the oracle's per V-cycle, at level sizes on both sides of the limit, with
+and without pre- or post-sweeps, after a change of the sweep counts, and in a
+fixed-cycle solver.
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def _walls(nodes, seed):
+    og = O.wall_grid([n - 1 for n in nodes])
+    fixed = np.zeros(nodes, np.uint8)
+    for d in range(len(nodes)):
+        s = [slice(None)] * len(nodes)
+        for e in (0, -1):
+            s[d] = e
+            fixed[tuple(s)] = 1
+    r, c, v = O.poisson_coo(og, 1.0, fixed.ravel())
+    b = np.random.default_rng(seed).standard_normal(fixed.size)
+    b[fixed.ravel() == 1] = 0.0
+    return fixed.size, r, c, v, b
+
+
+def _periodic(nodes, seed):
+    og = O.periodic_grid(list(nodes))
+    nn = O.num_nodes(og)
+    fixed = np.zeros(nn, np.uint8)
+    fixed[0] = 1
+    r, c, v = O.poisson_coo(og, 1.0, fixed)
+    b = np.random.default_rng(seed).standard_normal(nn)
+    b -= b.mean()
+    b[0] = 0.0
+    return nn, r, c, v, b
+
+
+# second level of 2025, 2070 (FP64 limit 2049), 4096 and 64, 49 nodes in 2D;
+# 4913, 5832 (limit 5000) and 1100 in 3D
+CASES = [("walls", (89, 89), 3), ("walls", (89, 90), 3), ("periodic", (128, 128), 3), ("periodic", (16, 16), 2),
+         ("walls", (13, 14), 2), ("walls", (33, 33, 33), 3), ("walls", (35, 35, 35), 3), ("walls", (17, 20, 23), 2)]
+
+
+@pytest.mark.parametrize("kind,nodes,depth", CASES)
+@pytest.mark.parametrize("prepost", [(2, 1), (0, 2), (3, 0)])
+def test_merged_levels_match_the_oracle_per_cycle(kind, nodes, depth, prepost):
+    from psum_amd import engine as E
+    nn, r, c, v, b = (_walls if kind == "walls" else _periodic)(nodes, 3)
+    pre, post = prepost
+    K = nodes[2] if len(nodes) == 3 else 1
+    mg = O.MG(nn, r, c, v, nodes[0], nodes[1], K, depth=depth, pre=pre, post=post)
+    s = E.SolverBackend("hip_multigrid_gpu")
+    dims = f"I {nodes[0]} J {nodes[1]}" + (f" K {K}" if K > 1 else "")
+    # set up with other sweep counts: set_options rebuilds the operator
+    s.set_options(f"{dims} depth {depth} pre_relax 1 post_relax 1 max_cycles 1")
+    s.set_matrix(nn, nn, r, c, v)
+    s.set_options(f"{dims} depth {depth} pre_relax {pre} post_relax {post} max_cycles 1")
+    x_ref, x = np.zeros(nn), torch.zeros(nn, dtype=torch.float64, device="cuda")
+    for cyc in range(3):
+        mg.vcycles(b, x_ref, 1)
+        s.solve(torch.from_numpy(b).cuda(), x)
+        err = np.max(np.abs(x.cpu().numpy() - x_ref)) / np.max(np.abs(x_ref))
+        # FP64 sums of at most 5832 terms in another order
+        assert err < 1e-11, (cyc, err)
+
+
+@pytest.mark.parametrize("kind,nodes,depth", CASES)
+def test_merged_levels_in_the_mixed_solver(kind, nodes, depth):
+    """FP32 V-cycles in FP64 refinement: a single iteration is the oracle's to
+    FP32 rounding, and the solve converges to the FP64 solver's answer."""
+    from psum_amd import engine as E
+    nn, r, c, v, b = (_walls if kind == "walls" else _periodic)(nodes, 5)
+    K = nodes[2] if len(nodes) == 3 else 1
+    dims = f"I {nodes[0]} J {nodes[1]}" + (f" K {K}" if K > 1 else "")
+
+    def solve(backend, opt):
+        s = E.SolverBackend(backend)
+        s.set_options(f"{dims} depth {depth} pre_relax 2 post_relax 2 {opt}")
+        s.set_matrix(nn, nn, r, c, v)
+        x = torch.zeros(nn, dtype=torch.float64, device="cuda")
+        s.solve(torch.from_numpy(b).cuda(), x)
+        return x.cpu().numpy(), s.stats()
+    one32, _ = solve("hip_multigrid32f_gpu", "max_cycles 1 correction_interval 1")
+    one64, _ = solve("hip_multigrid_gpu", "max_cycles 1")
+    # about 2^-24 times the condition of the sweeps; 1e-5 as for the whole
+    # mixed solve against the oracle
+    assert np.max(np.abs(one32 - one64)) <= 1e-5 * np.max(np.abs(one64))
+    x32, (_, rel) = solve("hip_multigrid32f_gpu", "max_cycles 60 tol 1e-10")
+    x64, _ = solve("hip_multigrid_gpu", "max_cycles 60 tol 1e-11")
+    assert rel <= 1e-10
+    assert np.max(np.abs(x32 - x64)) <= 1e-8 * np.max(np.abs(x64))
+
+
+@pytest.mark.parametrize("dtype", ["f64", "f32"])
+def test_switching_to_fixed_cycles_keeps_the_solution(dtype):
+    """A fixed cycle count takes a smaller limit (the operator is built
+    again): the step's potential stays that of the tolerance-controlled
+    solve."""
+    from psum_amd import engine as E
+    from psum_amd.workloads import langmuir_2d
+    wl = langmuir_2d(n=128, ppc=4, seed=3, dtype=np.float64 if dtype == "f64" else np.float32)
+    phis = []
+    for fixed in (0, 25):
+        st = E.Stepper(wl["grid"], wl["species"], dtype=dtype, mixed_mg=dtype == "f32", depth=4, pre=2, post=2,
+                       max_cycles=40, tol=1e-12, dt=wl["dt"], rho_bg=1.0)
+        st.set_smoothing(3, 2)
+        if fixed:
+            st.set_schedule(fixed, 0, 0)
+        st.run(1)
+        phis.append(st.phi())
+        st.close()
+    assert np.max(np.abs(phis[0] - phis[1])) <= 1e-9 * np.max(np.abs(phis[0]))
