@@ -690,29 +690,44 @@ __device__ __forceinline__ int batch_instance(const unsigned* __restrict__ first
     return lo;
 }
 
-// ---- fused 2D kernels: several Jacobi sweeps of one tile in LDS ----------
-// A block owns a tile of kTileRows x (kTileX - 2h) output nodes and loads it
-// with a halo of h = `sweeps` nodes (kTileX = 64 columns: one wave per row,
-// conflict-free LDS rows).  Sweep k updates the region shrunk by k, so after
-// h sweeps the output nodes hold exactly what h launches of k_smooth produce
-// (same operations in the same order).  Thread (tx, ty) owns column tx and
-// rows ty, ty+4, ...; its right-hand side and class ids stay in registers,
-// the iterate ping-pongs between two LDS planes, and class tables of up to
-// kMaxClsLds classes are staged in LDS.  Halo nodes beyond a non-wrapped
-// edge are clamped copies: the stencils of real nodes give them zero
-// coefficients, as in k_smooth's clamped neighbour.  PROLONG adds P x_c to
-// every loaded node first (k_prolong_add's arithmetic), fusing the
-// coarse-grid correction with the post-sweeps; ACC adds the result into an
-// FP64 iterate (the mixed refinement's x += e, fused into the last level-0
-// sweep).
+// ---- fused 2D kernels: a tile of the level in LDS -------------------------
+// A block works on 64 columns (one wave per row) of a tile held in LDS with a
+// halo as wide as the operations need: h Jacobi sweeps (sweep k updates the
+// region shrunk by k, so the output nodes hold exactly what h launches of
+// k_smooth produce, same operations in the same order), and in k_down_tile
+// one more node for the residual.  A thread owns one column and RPT
+// consecutive rows: its right-hand side and class rows stay in registers and the 3 x 3 window slides down its rows, so a
+// sweep reads 3 (RPT + 2) LDS values per thread instead of 9 values and 9
+// coefficients per node.  The iterate ping-pongs between two LDS planes;
+// class tables of up to kMaxClsLds classes are staged in LDS.  Halo nodes
+// beyond a non-wrapped edge are clamped copies: the stencils of real nodes
+// give them zero coefficients, as in k_smooth's clamped neighbour.
+//
+// Everything a block reads is asked for before its first barrier (transfer
+// tables, coarse values, weights of the restriction): on small levels a
+// launch is a chain of memory round trips, not bandwidth.  Two geometries:
+// 1024 threads over 32 rows (16 coarse rows), and 256 threads over 8 rows
+// (3 coarse rows) for levels whose large tiles would leave most compute units
+// idle (small_tiles()).
 constexpr int kTileX = 64;
-constexpr int kTileRows = 32;
 constexpr int kMaxFuse = 3;
-constexpr int kTileRmax = kTileRows + 2 * kMaxFuse;
-constexpr int kTileThreads = 1024;
-constexpr int kTileRowGroups = kTileThreads / kTileX;                       // 16
-constexpr int kRowsPerThread = (kTileRmax + kTileRowGroups - 1) / kTileRowGroups;   // 3
 constexpr int kMaxClsLds = 32;
+
+template <bool SMALL>
+struct TileGeom {
+    static constexpr int threads = SMALL ? 256 : 1024;
+    static constexpr int groups = threads / kTileX;     // waves, one row group each
+    static constexpr int rpt = SMALL ? 4 : 3;           // consecutive rows per thread
+    static constexpr int rows = SMALL ? 8 : 32;         // output rows of a smoothing tile
+    static constexpr int crows = SMALL ? 3 : 16;        // coarse rows of a k_down_tile tile
+    // one guard row on each side, one guard value before and after: tile row
+    // i, column tx at at(i, tx)
+    static constexpr int plane = (groups * rpt + 2) * kTileX + 2;
+    static __device__ __forceinline__ int at(int i, int tx) { return (i + 1) * kTileX + tx + 1; }
+    static_assert(rows + 2 * kMaxFuse <= groups * rpt, "smoothing tile exceeds its planes");
+    static_assert(2 * crows + 1 + 2 + 2 * kMaxFuse <= groups * rpt, "k_down_tile tile exceeds its planes");
+    static_assert(crows <= groups, "one coarse row per wave");
+};
 
 // wrapped (periodic axis) or clamped node coordinate; g is at most a few
 // nodes outside [0, n)
@@ -724,6 +739,89 @@ __device__ __forceinline__ int tile_coord(int g, int n, int wrap)
         return g;
     }
     return g < 0 ? 0 : (g >= n ? n - 1 : g);
+}
+
+template <typename T, bool COMPACT>
+struct TileRow {
+    static constexpr int n = COMPACT ? 5 : 9;
+    T c[n];
+    __device__ __forceinline__ void load(const T* __restrict__ row)
+    {
+        if (COMPACT) {
+            c[0] = row[1]; c[1] = row[3]; c[2] = row[4]; c[3] = row[5]; c[4] = row[7];
+        } else {
+#pragma unroll
+            for (int q = 0; q < n; ++q) c[q] = row[q];
+        }
+    }
+    // u, m, d: the rows above, at and below the node (columns -1, 0, 1)
+    __device__ __forceinline__ T apply(const T* u, const T* m, const T* d) const
+    {
+        T t = (T)0;
+        if (COMPACT) {
+            t = t + c[0] * u[1];
+            t = t + c[1] * m[0];
+            t = t + c[2] * m[1];
+            t = t + c[3] * m[2];
+            t = t + c[4] * d[1];
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) t = t + c[q] * u[q];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) t = t + c[3 + q] * m[q];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) t = t + c[6 + q] * d[q];
+        }
+        return t;
+    }
+};
+
+// f(k, sum) for the thread's rows k: sum = the class row applied to the plane
+// (p: the thread's column in the row above its first)
+template <typename T, bool COMPACT, bool SMALL, typename R, typename F>
+__device__ __forceinline__ void tile_stencil(const T* p, R&& row, F&& f)
+{
+    constexpr int RPT = TileGeom<SMALL>::rpt;
+    T w[3][3];
+    // a compact row reads only column 0 of the rows above and below
+    auto get = [&](int r, T* q, bool side) {
+        const T* a = p + r * kTileX;
+        q[1] = a[0];
+        if (side) {
+            q[0] = a[-1];
+            q[2] = a[1];
+        }
+    };
+    get(0, w[0], !COMPACT);
+    get(1, w[1], true);
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        T* u = w[k % 3];
+        T* m = w[(k + 1) % 3];
+        T* d = w[(k + 2) % 3];
+        get(k + 2, d, !COMPACT || k + 1 < RPT);
+        f(k, row(k).apply(u, m, d));
+    }
+}
+
+// h sweeps of the thread's rows between the planes; returns the plane that
+// holds the result.  i0: the thread's first tile row, R: tile rows in use.
+template <typename T, bool COMPACT, bool SMALL, typename R, typename P>
+__device__ __forceinline__ int tile_sweeps(P& sx, int tx, int i0, int nrows, int h, const T* breg, T two3, R&& row)
+{
+    int cur = 0;
+    for (int sw = 1; sw <= h; ++sw) {
+        const T* xs = &sx[cur][TileGeom<SMALL>::at(i0 - 1, tx)];
+        T* xn = &sx[cur ^ 1][TileGeom<SMALL>::at(i0, tx)];
+        const bool colok = tx >= sw && tx < kTileX - sw;
+        tile_stencil<T, COMPACT, SMALL>(xs, row, [&](int k, T t) {
+            const int i = i0 + k;
+            if (colok && i >= sw && i < nrows - sw) xn[k * kTileX] = t * (T)1 + breg[k] * (two3 * (T)1);
+        });
+        __syncthreads();
+        cur ^= 1;
+    }
+    return cur;
 }
 
 template <typename T>
@@ -738,152 +836,149 @@ struct SmoothTileArgs {
     int h;
     DevLevel Cl;
     DevTransfer<T> tr;
+    int half;            // both axes halve: the tile's coarse values are staged in LDS
     const T* xc;
     double* xacc;
 };
 
-template <typename T, bool COMPACT, bool PROLONG, bool ACC>
+// Up to kMaxFuse sweeps of one level.  PROLONG adds P x_c to every loaded
+// node first (k_prolong_add's arithmetic), fusing the coarse-grid correction
+// with the post-sweeps; ACC adds the result into an FP64 iterate (the mixed
+// refinement's x += e, fused into the last level-0 sweep).
+template <typename T, bool COMPACT, bool PROLONG, bool ACC, bool SMALL>
 __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, unsigned bid)
 {
+    using G = TileGeom<SMALL>;
+    constexpr int RPT = G::rpt;
+    constexpr int CW = kTileX / 2 + 2, CH = (G::groups * RPT) / 2 + 2;   // staged coarse values
     const DevLevel& L = A.L;
     const DevTable<T>& relax = A.relax;
-    const int ncls = A.ncls;
-    const T* __restrict__ xin = A.xin;
-    const T* __restrict__ b = A.b;
-    T* __restrict__ xout = A.xout;
-    const T two3 = A.two3;
     const int h = A.h;
     const DevLevel& Cl = A.Cl;
     const DevTransfer<T>& tr = A.tr;
     const T* __restrict__ xc = A.xc;
-    double* __restrict__ xacc = A.xacc;
-    __shared__ T sx[2][kTileRmax * kTileX];
+    __shared__ T sx[2][G::plane];
     __shared__ T ctab[kMaxClsLds * 9];
-    const int tx = threadIdx.x & (kTileX - 1), ty = threadIdx.x / kTileX;
+    __shared__ T sxc[PROLONG ? CW * CH : 1];
+    const int tx = threadIdx.x & (kTileX - 1), ty = threadIdx.x / kTileX, i0 = ty * RPT;
     const int n0 = L.n[0], n1 = L.n[1];
     const int ostep = kTileX - 2 * h;
     const int ntc = (n1 + ostep - 1) / ostep;
-    const int t0 = (int)(bid / ntc) * kTileRows, t1 = (int)(bid % ntc) * ostep;
-    const int R = kTileRows + 2 * h;
-    const bool lds_tab = ncls <= kMaxClsLds;
+    const int t0 = (int)(bid / ntc) * G::rows, t1 = (int)(bid % ntc) * ostep;
+    const int R = G::rows + 2 * h;
+    const bool lds_tab = A.ncls <= kMaxClsLds;
     if (lds_tab)
-        for (int i = threadIdx.x; i < ncls * 9; i += kTileThreads) ctab[i] = relax.coef[i];
+        for (int i = threadIdx.x; i < A.ncls * 9; i += G::threads) ctab[i] = relax.coef[i];
     const int g1 = tile_coord(t1 - h + tx, n1, L.wrap[1]);
-    // column part of the prolongation, once per thread
-    int q1[2] = {0, 0};
-    T w1[2] = {(T)0, (T)0};
+    // coarse rows and columns lo .. lo + CH - 1, CW - 1 hold every value the
+    // tile interpolates from when both axes halve
+    const int lo0 = (t0 - h) >> 1, lo1 = (t1 - h) >> 1;
+    const bool staged = PROLONG && A.half;
+    if (staged)
+        for (int i = threadIdx.x; i < CW * CH; i += G::threads) {
+            const int r = i / CW, q = i - r * CW;
+            sxc[i] = xc[(int64_t)tile_coord(lo0 + r, Cl.n[0], tr.wrap[0]) * Cl.n[1] + tile_coord(lo1 + q, Cl.n[1], tr.wrap[1])];
+        }
+    T breg[RPT], xv[RPT];
+    int creg[RPT];
+    double xa[RPT];
+    int p0[RPT], p1 = 0;
+    T w0[RPT][2], w1[2] = {(T)0, (T)0};
     if (PROLONG) {
-        const int p1 = tr.pc[1][g1];
+        p1 = tr.pc[1][g1];
         w1[0] = tr.pw[1][2 * g1];
         w1[1] = tr.pw[1][2 * g1 + 1];
-        q1[0] = wrap_index(p1, Cl.n[1], tr.wrap[1]);
-        q1[1] = wrap_index(p1 + 1, Cl.n[1], tr.wrap[1]);
     }
-    T breg[kRowsPerThread];
-    int creg[kRowsPerThread];
+    const int g1o = t1 + tx - h;
+    const bool colout = tx >= h && tx < kTileX - h && g1o < n1;
 #pragma unroll
-    for (int k = 0; k < kRowsPerThread; ++k) {
-        const int i = ty + kTileRowGroups * k;
+    for (int k = 0; k < RPT; ++k) {
+        const int i = i0 + k;
         breg[k] = (T)0;
+        xv[k] = (T)0;
         creg[k] = 0;
+        xa[k] = 0.0;
+        p0[k] = 0;
+        w0[k][0] = w0[k][1] = (T)0;
         if (i < R) {
             const int g0 = tile_coord(t0 - h + i, n0, L.wrap[0]);
             const int64_t gi = (int64_t)g0 * n1 + g1;
-            T xv = xin[gi];
-            if (PROLONG) {
-                // k_prolong_add's sum: a over the row factor, b over the column factor
-                const int p0 = tr.pc[0][g0];
-                const T w0[2] = {tr.pw[0][2 * g0], tr.pw[0][2 * g0 + 1]};
-                T s = (T)0;
-#pragma unroll
-                for (int a = 0; a < 2; ++a) {
-                    if (w0[a] == (T)0) continue;
-                    const int i0 = wrap_index(p0 + a, Cl.n[0], tr.wrap[0]);
-#pragma unroll
-                    for (int bb = 0; bb < 2; ++bb) {
-                        if (w1[bb] == (T)0) continue;
-                        s = s + (w0[a] * w1[bb]) * xc[(int64_t)i0 * Cl.n[1] + q1[bb]];
-                    }
-                }
-                xv = s * (T)1 + xv * (T)1;
-            }
-            sx[0][i * kTileX + tx] = xv;
-            breg[k] = b[gi];
+            xv[k] = A.xin[gi];
+            breg[k] = A.b[gi];
             creg[k] = L.cls[gi];
-        }
-    }
-    __syncthreads();
-    int cur = 0;
-    for (int sw = 1; sw <= h; ++sw) {
-        const T* xs = sx[cur];
-        T* xn = sx[cur ^ 1];
-        const bool colok = tx >= sw && tx < kTileX - sw;
-#pragma unroll
-        for (int k = 0; k < kRowsPerThread; ++k) {
-            const int i = ty + kTileRowGroups * k;
-            if (!(colok && i >= sw && i < R - sw)) continue;
-            T c[9];
-            if (lds_tab) {
-#pragma unroll
-                for (int q = 0; q < 9; ++q) c[q] = ctab[creg[k] * 9 + q];
-            } else {
-#pragma unroll
-                for (int q = 0; q < 9; ++q) c[q] = relax.coef[(int64_t)creg[k] * 9 + q];
+            if (PROLONG) {
+                p0[k] = tr.pc[0][g0];
+                w0[k][0] = tr.pw[0][2 * g0];
+                w0[k][1] = tr.pw[0][2 * g0 + 1];
             }
-            const int li = i * kTileX + tx;
-            T t = (T)0;
-#pragma unroll
-            for (int da = -1; da <= 1; ++da)
-#pragma unroll
-                for (int db = -1; db <= 1; ++db) {
-                    if (COMPACT && da != 0 && db != 0) continue;
-                    t = t + c[(da + 1) * 3 + (db + 1)] * xs[li + da * kTileX + db];
-                }
-            xn[li] = t * (T)1 + breg[k] * (two3 * (T)1);
+            if (ACC && colout && i >= h && i < h + G::rows && t0 + i - h < n0) xa[k] = A.xacc[gi];
         }
-        __syncthreads();
-        cur ^= 1;
     }
-    const int g1o = t1 + tx - h;
-    if (tx < h || tx >= kTileX - h || g1o >= n1) return;
+    if (PROLONG) {
+        if (staged) __syncthreads();
+        int q1[2];
+        if (staged) {
+            q1[0] = (tr.wrap[1] ? (t1 - h + tx) >> 1 : p1) - lo1;
+            q1[1] = q1[0] + 1;
+        } else {
+            q1[0] = wrap_index(p1, Cl.n[1], tr.wrap[1]);
+            q1[1] = wrap_index(p1 + 1, Cl.n[1], tr.wrap[1]);
+        }
 #pragma unroll
-    for (int k = 0; k < kRowsPerThread; ++k) {
-        const int i = ty + kTileRowGroups * k;
-        if (i < h || i >= h + kTileRows) continue;
+        for (int k = 0; k < RPT; ++k) {
+            const int i = i0 + k;
+            if (i >= R) continue;
+            // k_prolong_add's sum: a over the row factor, b over the column factor
+            const int r0 = (tr.wrap[0] ? (t0 - h + i) >> 1 : p0[k]) - lo0;
+            T s = (T)0;
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                if (w0[k][a] == (T)0) continue;
+                const int j0 = staged ? 0 : wrap_index(p0[k] + a, Cl.n[0], tr.wrap[0]);
+#pragma unroll
+                for (int bb = 0; bb < 2; ++bb) {
+                    if (w1[bb] == (T)0) continue;
+                    const T v = staged ? sxc[(r0 + a) * CW + q1[bb]] : xc[(int64_t)j0 * Cl.n[1] + q1[bb]];
+                    s = s + (w0[k][a] * w1[bb]) * v;
+                }
+            }
+            xv[k] = s * (T)1 + xv[k] * (T)1;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+        if (i0 + k < R) sx[0][G::at(i0 + k, tx)] = xv[k];
+    __syncthreads();
+    TileRow<T, COMPACT> rows[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) rows[k].load(lds_tab ? &ctab[creg[k] * 9] : relax.coef + (int64_t)creg[k] * 9);
+    const int cur = tile_sweeps<T, COMPACT, SMALL>(sx, tx, i0, R, h, breg, A.two3, [&](int k) { return rows[k]; });
+    if (!colout) return;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        const int i = i0 + k;
         const int g0 = t0 + i - h;
-        if (g0 >= n0) continue;
+        if (i < h || i >= h + G::rows || g0 >= n0) continue;
         const int64_t gi = (int64_t)g0 * n1 + g1o;
-        const T v = sx[cur][i * kTileX + tx];
-        xout[gi] = v;
-        if (ACC) xacc[gi] += (double)v;
+        const T v = sx[cur][G::at(i, tx)];
+        A.xout[gi] = v;
+        if (ACC) A.xacc[gi] = xa[k] + (double)v;
     }
 }
 
-template <typename T, bool COMPACT, bool PROLONG, bool ACC>
-__global__ __launch_bounds__(kTileThreads) void k_smooth_tile(SmoothTileArgs<T> a)
+template <typename T, bool COMPACT, bool PROLONG, bool ACC, bool SMALL>
+__global__ __launch_bounds__(TileGeom<SMALL>::threads) void k_smooth_tile(SmoothTileArgs<T> a)
 {
-    smooth_tile_body<T, COMPACT, PROLONG, ACC>(a, blockIdx.x);
+    smooth_tile_body<T, COMPACT, PROLONG, ACC, SMALL>(a, blockIdx.x);
 }
 
 template <typename T, bool COMPACT, bool PROLONG, bool ACC>
-__global__ __launch_bounds__(kTileThreads) void k_smooth_tile_many(const SmoothTileArgs<T>* __restrict__ a,
-                                                                   const unsigned* __restrict__ first, int n)
+__global__ __launch_bounds__(TileGeom<false>::threads) void k_smooth_tile_many(const SmoothTileArgs<T>* __restrict__ a,
+                                                                               const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
-    smooth_tile_body<T, COMPACT, PROLONG, ACC>(a[i], blockIdx.x - first[i]);
+    smooth_tile_body<T, COMPACT, PROLONG, ACC, false>(a[i], blockIdx.x - first[i]);
 }
-
-// Tiled residual + restriction (2D): a block restricts a kRRRows x kRRCols
-// coarse tile.  It loads x on the fine support of that tile plus a one-node
-// halo into LDS, evaluates the fine residuals there (k_residual's
-// arithmetic), then sums each coarse node's support (k_restrict's order).
-// The host uses it only where every tile's fine support fits (at most
-// kRRFineRows x kRRFineCols nodes; true for the halving and identity
-// transfers).
-constexpr int kRRRows = 16;
-constexpr int kRRCols = 30;
-constexpr int kRRFineRows = 34;
-constexpr int kRRFineCols = 62;
 
 template <typename T>
 struct ResidRestrictArgs {
@@ -899,100 +994,151 @@ struct ResidRestrictArgs {
     T first_sweep;
 };
 
-template <typename T, bool COMPACT>
-__device__ __forceinline__ void resid_restrict_tile_body(const ResidRestrictArgs<T>& A, unsigned bid)
+// The downward half of a level in one launch (2D): h = 0 .. kMaxFuse last
+// pre-sweeps, the residual, its restriction.  A block restricts to crows x CC
+// coarse nodes (CC from h, so that their fine support, the residual's and
+// the sweeps' halos fit 64 columns); it stores the swept iterate on the fine
+// nodes of its tile (h > 0), evaluates the residuals of the support in LDS
+// (k_residual's arithmetic), and one thread sums each coarse node's support
+// (k_restrict's order).  The fine support of coarse nodes lo..hi-1 lies in
+// [st lo - (st - 1), st (hi - 1) + st - 1], st = 2 on a halved axis and 1 on
+// one kept as it is (the host checks the transfer tables, down_fits()).
+template <typename T>
+struct DownTileArgs {
+    ResidRestrictArgs<T> r;
+    DevTable<T> relax;
+    T* xout;
+    T two3;
+    int h;
+    int st[2];
+};
+
+__host__ __device__ inline int down_cols(int h, int st) { return (kTileX - 2 - 2 * h - (st - 1)) / st; }
+
+template <typename T, bool COMPACT, bool SMALL>
+__device__ __forceinline__ void down_tile_body(const DownTileArgs<T>& A, unsigned bid)
 {
-    const DevLevel& F = A.F;
-    const DevLevel& Cl = A.Cl;
-    const DevTransfer<T>& tr = A.tr;
-    const DevTable<T>& Af = A.Af;
-    const int ncls = A.ncls;
-    const DevTable<T>& Ac = A.Ac;
-    const T* __restrict__ x = A.x;
-    const T* __restrict__ bf = A.bf;
-    T* __restrict__ bc = A.bc;
-    T* __restrict__ xc = A.xc;
-    const T first_sweep = A.first_sweep;
-    __shared__ T sxx[(kRRFineRows + 2) * 64];
-    __shared__ T sr[kRRFineRows * 64];
-    __shared__ T ctab[kMaxClsLds * 9];
-    const int ntc = (Cl.n[1] + kRRCols - 1) / kRRCols;
-    const int c0lo = (int)(bid / ntc) * kRRRows, c1lo = (int)(bid % ntc) * kRRCols;
-    const int c0hi = min(c0lo + kRRRows, Cl.n[0]), c1hi = min(c1lo + kRRCols, Cl.n[1]);
-    const int f0lo = tr.rf[0][c0lo], f0hi = tr.rf[0][c0hi - 1] + tr.rn[0][c0hi - 1];
-    const int f1lo = tr.rf[1][c1lo], f1hi = tr.rf[1][c1hi - 1] + tr.rn[1][c1hi - 1];
-    const int FR = f0hi - f0lo, FC = f1hi - f1lo;
-    const bool lds_tab = ncls <= kMaxClsLds;
+    using G = TileGeom<SMALL>;
+    constexpr int RPT = G::rpt;
+    const DevLevel& F = A.r.F;
+    const DevLevel& Cl = A.r.Cl;
+    const DevTransfer<T>& tr = A.r.tr;
+    const int h = A.h;
+    __shared__ T sx[2][G::plane];
+    __shared__ T rtab[kMaxClsLds * 9], atab[kMaxClsLds * 9];
+    const int CC = down_cols(h, A.st[1]);
+    const int ntc = (Cl.n[1] + CC - 1) / CC;
+    const int c0lo = (int)(bid / ntc) * G::crows, c1lo = (int)(bid % ntc) * CC;
+    const int c0hi = min(c0lo + G::crows, Cl.n[0]), c1hi = min(c1lo + CC, Cl.n[1]);
+    // fine coordinates (before wrapping) of the tile's first row and column
+    const int u0 = A.st[0] * c0lo - A.st[0] - h, u1 = A.st[1] * c1lo - A.st[1] - h;
+    const int R = A.st[0] * (c0hi - c0lo) + (A.st[0] - 1) + 2 + 2 * h;
+    const int W = A.st[1] * (c1hi - c1lo) + (A.st[1] - 1) + 2 + 2 * h;
+    const bool lds_tab = A.r.ncls <= kMaxClsLds;
     if (lds_tab)
-        for (int i = threadIdx.x; i < ncls * 9; i += kTileThreads) ctab[i] = Af.coef[i];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+        for (int i = threadIdx.x; i < A.r.ncls * 9; i += G::threads) {
+            atab[i] = A.r.Af.coef[i];
+            rtab[i] = A.relax.coef[i];
+        }
+    const int tx = threadIdx.x & (kTileX - 1), ty = threadIdx.x / kTileX, i0 = ty * RPT;
     const int n0 = F.n[0], n1 = F.n[1];
-    if (tx < FC + 2) {
-        const int g1 = tile_coord(f1lo - 1 + tx, n1, F.wrap[1]);
-        for (int i = ty; i < FR + 2; i += kTileRowGroups) {
-            const int g0 = tile_coord(f0lo - 1 + i, n0, F.wrap[0]);
-            sxx[i * 64 + tx] = x[(int64_t)g0 * n1 + g1];
+    const int g1 = tile_coord(u1 + tx, n1, F.wrap[1]);
+    T breg[RPT], xv[RPT];
+    int creg[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        const int i = i0 + k;
+        breg[k] = (T)0;
+        xv[k] = (T)0;
+        creg[k] = 0;
+        if (i < R && tx < W) {
+            const int64_t gi = (int64_t)tile_coord(u0 + i, n0, F.wrap[0]) * n1 + g1;
+            xv[k] = A.r.x[gi];
+            breg[k] = A.r.bf[gi];
+            creg[k] = F.cls[gi];
         }
     }
+    // the coarse node this thread sums: its support and weights
+    const int c0 = c0lo + ty, c1 = c1lo + tx;
+    const bool coarse = ty < G::crows && tx < CC && c0 < c0hi && c1 < c1hi;
+    int f0 = 0, m0 = 0, f1 = 0, m1 = 0;
+    T rw0[3] = {(T)0, (T)0, (T)0}, rw1[3] = {(T)0, (T)0, (T)0}, dinv = (T)0;
+    if (coarse) {
+        f0 = tr.rf[0][c0];
+        m0 = tr.rn[0][c0];
+        f1 = tr.rf[1][c1];
+        m1 = tr.rn[1][c1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            rw0[q] = tr.rw[0][3 * c0 + q];
+            rw1[q] = tr.rw[1][3 * c1 + q];
+        }
+        dinv = A.r.Ac.dinv[Cl.cls[(int64_t)c0 * Cl.n[1] + c1]];
+    }
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+        if (i0 + k < R) sx[0][G::at(i0 + k, tx)] = xv[k];
     __syncthreads();
-    if (tx < FC) {
-        const int g1 = tile_coord(f1lo + tx, n1, F.wrap[1]);
-        for (int i = ty; i < FR; i += kTileRowGroups) {
-            const int g0 = tile_coord(f0lo + i, n0, F.wrap[0]);
-            const int64_t gi = (int64_t)g0 * n1 + g1;
-            const int cl = F.cls[gi];
-            T c[9];
-            if (lds_tab) {
+    auto row_of = [&](const T* lds, const T* coef, int k) {
+        TileRow<T, COMPACT> r;
+        r.load(lds_tab ? lds + creg[k] * 9 : coef + (int64_t)creg[k] * 9);
+        return r;
+    };
+    int cur = 0;
+    if (h > 0) {
+        TileRow<T, COMPACT> rows[RPT];
 #pragma unroll
-                for (int q = 0; q < 9; ++q) c[q] = ctab[cl * 9 + q];
-            } else {
+        for (int k = 0; k < RPT; ++k) rows[k] = row_of(rtab, A.relax.coef, k);
+        cur = tile_sweeps<T, COMPACT, SMALL>(sx, tx, i0, R, h, breg, A.two3, [&](int k) { return rows[k]; });
+        // the tile's own fine nodes
+        const int e0 = c0hi == Cl.n[0] ? n0 : A.st[0] * c0hi, e1 = c1hi == Cl.n[1] ? n1 : A.st[1] * c1hi;
+        const int o1 = u1 + tx;
+        if (o1 >= A.st[1] * c1lo && o1 < e1)
 #pragma unroll
-                for (int q = 0; q < 9; ++q) c[q] = Af.coef[(int64_t)cl * 9 + q];
+            for (int k = 0; k < RPT; ++k) {
+                const int o0 = u0 + i0 + k;
+                if (o0 >= A.st[0] * c0lo && o0 < e0)
+                    A.xout[(int64_t)o0 * n1 + o1] = sx[cur][G::at(i0 + k, tx)];
             }
-            const int li = (i + 1) * 64 + (tx + 1);
-            T t = (T)0;
-#pragma unroll
-            for (int da = -1; da <= 1; ++da)
-#pragma unroll
-                for (int db = -1; db <= 1; ++db) {
-                    if (COMPACT && da != 0 && db != 0) continue;
-                    t = t + c[(da + 1) * 3 + (db + 1)] * sxx[li + da * 64 + db];
-                }
-            sr[i * 64 + tx] = t * (T)-1 + bf[gi] * (T)1;
-        }
+    }
+    // residuals on the support, into the other plane
+    {
+        const bool colok = tx >= h + 1 && tx < W - h - 1;
+        T* rn = &sx[cur ^ 1][G::at(i0, tx)];
+        tile_stencil<T, COMPACT, SMALL>(&sx[cur][G::at(i0 - 1, tx)], [&](int k) { return row_of(atab, A.r.Af.coef, k); },
+                                        [&](int k, T t) {
+            const int i = i0 + k;
+            if (colok && i >= h + 1 && i < R - h - 1) rn[k * kTileX] = t * (T)-1 + breg[k] * (T)1;
+        });
     }
     __syncthreads();
-    if ((int)threadIdx.x >= kRRRows * kRRCols) return;
-    const int c0 = c0lo + (int)threadIdx.x / kRRCols, c1 = c1lo + (int)threadIdx.x % kRRCols;
-    if (c0 >= c0hi || c1 >= c1hi) return;
-    const int f0 = tr.rf[0][c0], m0 = tr.rn[0][c0];
-    const int f1 = tr.rf[1][c1], m1 = tr.rn[1][c1];
+    if (!coarse) return;
+    const T* sr = &sx[cur ^ 1][G::at(f0 - u0, f1 - u1)];
     T s = (T)0;
-    for (int a = 0; a < m0; ++a) {
-        const T w0 = tr.rw[0][3 * c0 + a];
-        for (int b = 0; b < m1; ++b) {
-            const T w = w0 * tr.rw[1][3 * c1 + b];
-            s = s + w * sr[(f0 + a - f0lo) * 64 + (f1 + b - f1lo)];
-        }
-    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (a < m0)
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+                if (b < m1) s = s + (rw0[a] * rw1[b]) * sr[a * kTileX + b];
     const int64_t ci = (int64_t)c0 * Cl.n[1] + c1;
-    const T bv = s * Ac.dinv[Cl.cls[ci]];
-    bc[ci] = bv;
-    xc[ci] = first_sweep != (T)0 ? bv * (first_sweep * (T)1) : (T)0;
+    const T bv = s * dinv;
+    A.r.bc[ci] = bv;
+    A.r.xc[ci] = A.r.first_sweep != (T)0 ? bv * (A.r.first_sweep * (T)1) : (T)0;
 }
 
-template <typename T, bool COMPACT>
-__global__ __launch_bounds__(kTileThreads) void k_resid_restrict_tile(ResidRestrictArgs<T> a)
+template <typename T, bool COMPACT, bool SMALL>
+__global__ __launch_bounds__(TileGeom<SMALL>::threads) void k_down_tile(DownTileArgs<T> a)
 {
-    resid_restrict_tile_body<T, COMPACT>(a, blockIdx.x);
+    down_tile_body<T, COMPACT, SMALL>(a, blockIdx.x);
 }
 
 template <typename T, bool COMPACT>
-__global__ __launch_bounds__(kTileThreads) void k_resid_restrict_tile_many(
-    const ResidRestrictArgs<T>* __restrict__ a, const unsigned* __restrict__ first, int n)
+__global__ __launch_bounds__(TileGeom<false>::threads) void k_down_tile_many(const DownTileArgs<T>* __restrict__ a,
+                                                                             const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
-    resid_restrict_tile_body<T, COMPACT>(a[i], blockIdx.x - first[i]);
+    down_tile_body<T, COMPACT, false>(a[i], blockIdx.x - first[i]);
 }
 
 // k_residual fused into k_restrict (2D): the restriction evaluates the fine
@@ -2038,8 +2184,8 @@ struct DevTransferBuf {
 namespace psum_hip {
 
 // kernel kinds of recorded ops (base + template variant bits)
-constexpr uint16_t kKindSmooth = 0;      // + (FP64 << 3 | compact << 2 | prolong << 1 | acc)
-constexpr uint16_t kKindRRTile = 16;     // + (FP64 << 1 | compact)
+constexpr uint16_t kKindSmooth = 0;      // + (FP64 << 3 | compact << 2 | prolong << 1 | acc), large tiles
+constexpr uint16_t kKindDown = 16;       // + (FP64 << 1 | compact), large tiles
 constexpr uint16_t kKindRR = 20;         // + (FP64 << 1 | compact)
 constexpr uint16_t kKindCoarse = 24;     // + (0 FP32 vectors with an FP64 operator, 1 FP64, 2 FP32)
 constexpr uint16_t kKindOuter = 27;      // + (norms << 2 | compact << 1 | emit FP32), 2D
@@ -2107,7 +2253,7 @@ public:
             else if (key == "line") line_ = v;
             else throw std::invalid_argument("hip_multigrid: unknown tuning option " + key);
         }
-        rr_fit_.clear();
+        tile_fit_.clear();
         drop_graphs();   // captured cycles hold the previous kernel shapes
     }
 
@@ -2120,7 +2266,7 @@ public:
             throw std::invalid_argument("hip_multigrid: smoothing sweeps need 0 <= pre, post <= 64, pre + post >= 1");
         pre_ = pre;
         post_ = post;
-        rr_fit_.clear();
+        tile_fit_.clear();
         drop_graphs();
         if (!host_.empty()) build_operator();
     }
@@ -2183,7 +2329,7 @@ public:
         dense_inverse(L.back(), cinv_host_, pin_ >= 0);
         host_ = std::move(L);
         tr_host_ = std::move(T);
-        rr_fit_.clear();
+        tile_fit_.clear();
         upload();
         build_operator();
     }
@@ -2407,18 +2553,26 @@ private:
     static constexpr int tbit() { return std::is_same<T, double>::value ? 1 : 0; }
 
     template <typename T, bool C, bool P, bool A>
-    void run_smooth_tile(unsigned nb, const SmoothTileArgs<T>& a)
+    void run_smooth_tile(bool small, unsigned nb, const SmoothTileArgs<T>& a)
     {
         if (rec_) { emit((uint16_t)(kKindSmooth + ((tbit<T>() << 3) | (C << 2) | (P << 1) | (A ? 1 : 0))), nb, a); return; }
-        hipLaunchKernelGGL((k_smooth_tile<T, C, P, A>), dim3(nb), dim3(kTileThreads), 0, stream_, a);
+        if (small) hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, true>), dim3(nb), dim3(TileGeom<true>::threads), 0, stream_, a);
+        else hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, false>), dim3(nb), dim3(TileGeom<false>::threads), 0, stream_, a);
     }
 
-    template <typename T, bool C, bool TILE>
+    template <typename T, bool C>
+    void run_down(bool small, unsigned nb, const DownTileArgs<T>& a)
+    {
+        if (rec_) { emit((uint16_t)(kKindDown + ((tbit<T>() << 1) | (C ? 1 : 0))), nb, a); return; }
+        if (small) hipLaunchKernelGGL((k_down_tile<T, C, true>), dim3(nb), dim3(TileGeom<true>::threads), 0, stream_, a);
+        else hipLaunchKernelGGL((k_down_tile<T, C, false>), dim3(nb), dim3(TileGeom<false>::threads), 0, stream_, a);
+    }
+
+    template <typename T, bool C>
     void run_rr(unsigned nb, const ResidRestrictArgs<T>& a)
     {
-        if (rec_) { emit((uint16_t)((TILE ? kKindRRTile : kKindRR) + ((tbit<T>() << 1) | (C ? 1 : 0))), nb, a); return; }
-        if (TILE) hipLaunchKernelGGL((k_resid_restrict_tile<T, C>), dim3(nb), dim3(kTileThreads), 0, stream_, a);
-        else hipLaunchKernelGGL((k_resid_restrict<T, C>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
+        if (rec_) { emit((uint16_t)(kKindRR + ((tbit<T>() << 1) | (C ? 1 : 0))), nb, a); return; }
+        hipLaunchKernelGGL((k_resid_restrict<T, C>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
     }
 
     template <typename T, typename M>
@@ -2464,7 +2618,7 @@ private:
     bool op_f32_ = false;
     void* op_ = nullptr;
     bool fixed_mode_ = false;          // set_fixed_cycles was called
-    std::vector<int> rr_fit_;
+    std::vector<int> tile_fit_;
     double tol_ = 0.0;
     int predicted_ = 1;                // cycles the previous solve needed
     int periodic_mode_ = 1;
@@ -2766,19 +2920,26 @@ private:
         const DevTransfer<T> tr = xc ? transfer<T>(l) : DevTransfer<T>{};
         const bool cmp = host_[l].compact;
         const int ncls = (int)host_[l].dinv.size();
+        const int half = xc && tile_steps(l, true) == 22 ? 1 : 0;
         bool accd = false;
         while (count > 0) {
             const int k = std::min(count, kMaxFuse);
             const int ostep = kTileX - 2 * k;
-            const unsigned nb = (unsigned)(((L.n[0] + kTileRows - 1) / kTileRows) * ((L.n[1] + ostep - 1) / ostep));
+            const int64_t ntc = (L.n[1] + ostep - 1) / ostep;
+            const bool small = small_tiles(((L.n[0] + TileGeom<false>::rows - 1) / TileGeom<false>::rows) * ntc);
+            const int rows = small ? TileGeom<true>::rows : TileGeom<false>::rows;
+            const unsigned nb = (unsigned)(((L.n[0] + rows - 1) / rows) * ntc);
             double* a = (k == count) ? acc : nullptr;
-            const SmoothTileArgs<T> ta{L, table<T>(l, true), ncls, x, b, buf, two3, k, C, tr, xc, a};
-#define TILE(CMP, PRO, ACC) run_smooth_tile<T, CMP, PRO, ACC>(nb, ta)
-            if (a) {
-                if (xc) { if (cmp) TILE(true, true, true); else TILE(false, true, true); }
-                else { if (cmp) TILE(true, false, true); else TILE(false, false, true); }
-                accd = true;
-            } else {
+            const SmoothTileArgs<T> ta{L, table<T>(l, true), ncls, x, b, buf, two3, k, C, tr, half, xc, a};
+#define TILE(CMP, PRO, ACC) run_smooth_tile<T, CMP, PRO, ACC>(small, nb, ta)
+            if constexpr (std::is_same<T, float>::value) {
+                if (a) {
+                    if (xc) { if (cmp) TILE(true, true, true); else TILE(false, true, true); }
+                    else { if (cmp) TILE(true, false, true); else TILE(false, false, true); }
+                    accd = true;
+                }
+            }
+            if (!accd) {
                 if (xc) { if (cmp) TILE(true, true, false); else TILE(false, true, false); }
                 else { if (cmp) TILE(true, false, false); else TILE(false, false, false); }
             }
@@ -2790,26 +2951,45 @@ private:
         return accd;
     }
 
-    // whether every coarse tile of level l+1 has its fine support within the
-    // tiled residual + restriction kernel's LDS tile (checked once per level)
-    bool rr_tile_fits(int l)
+    // Tiles of 256 threads and 8 rows where the large ones (1024 threads, 32
+    // rows) would cover the level with fewer than 128 blocks, half the compute
+    // units: V(2,1) cycles of 128^2 FP64 take 16 % less time with them (13.6
+    // against 16.0 ms per 20 steps of the Langmuir run), 641 x 385 17 % less,
+    // 1024^2 0.5-2 % more.  Recorded solves share their launches with other
+    // solvers, whose blocks fill the chip: always the large ones (12 instances
+    // of 64^2..256^2: 27.3 against 28.2 ms).
+    bool small_tiles(int64_t large_blocks) const { return !rec_ && large_blocks < 128; }
+
+    // How the transfers between levels l and l + 1 step along the two axes,
+    // 10 st[0] + st[1] with 2 for a halved axis and 1 for one kept as it is,
+    // or 0 where the tables go beyond what the tiles hold (k_down_tile,
+    // prolongation: the staged coarse values).  Checked once per level.
+    int tile_steps(int l, bool prolongation)
     {
-        if ((int)rr_fit_.size() != (int)host_.size()) rr_fit_.assign(host_.size(), -1);
-        if (rr_fit_[l] >= 0) return rr_fit_[l] == 1;
-        const HostLevel& C = host_[l + 1];
+        if (tile_fit_.size() != 2 * host_.size()) tile_fit_.assign(2 * host_.size(), -1);
+        int& fit = tile_fit_[2 * (size_t)l + (prolongation ? 1 : 0)];
+        if (fit >= 0) return fit;
+        int code = 0;
         bool ok = true;
-        const int lim[2] = {kRRFineRows, kRRFineCols}, step[2] = {kRRRows, kRRCols};
-        for (int d = 0; d < 2 && ok; ++d) {
+        for (int d = 0; d < 2; ++d) {
             const AxisTransfer& t = tr_host_[l][d];
-            for (int lo = 0; lo < C.n[d] && ok; lo += step[d]) {
-                const int hi = std::min(lo + step[d], C.n[d]) - 1;
-                for (int c = lo; c < hi; ++c)
-                    if (t.rf[c + 1] < t.rf[c] || t.rf[c + 1] + t.rn[c + 1] < t.rf[c] + t.rn[c]) ok = false;
-                if (t.rf[hi] + t.rn[hi] - t.rf[lo] > lim[d]) ok = false;
+            const int nf = host_[l].n[d], nc = host_[l + 1].n[d];
+            const int st = nf == nc ? 1 : 2;
+            code = 10 * code + st;
+            // a wrapped axis with transfers that do not wrap (periodic_mode 0):
+            // a halo node's coarse nodes are not next to its tile's
+            if (prolongation && (host_[l].wrap[d] != 0) != (t.wrap != 0)) ok = false;
+            for (int c = 0; c < nc && !prolongation; ++c)
+                if (t.rn[c] > 3 || t.rf[c] < st * c - (st - 1) || t.rf[c] + t.rn[c] > st * c + st) ok = false;
+            for (int i = 0; i < nf && prolongation; ++i) {
+                const int q = st == 2 ? i >> 1 : i;
+                // (the last node of an even count is a coarse node itself)
+                if (t.pc[i] != q && (t.wrap || t.pc[i] != q + 1 || t.pw[2 * i + 1] != 0.0)) ok = false;
+                if (t.wrap && st == 2 && nf % 2 != 0) ok = false;
             }
         }
-        rr_fit_[l] = ok ? 1 : 0;
-        return ok;
+        fit = ok ? code : 0;
+        return fit;
     }
 
     template <typename T>
@@ -2981,23 +3161,31 @@ private:
                 rec_phase(it, kStageDown, (uint32_t)l);
                 // coarse levels received their first sweep from the restriction
                 const bool swept = (l > 0 || (cyc == 0 && first_swept)) && pre_ > 0;
-                smooth_n<T>(l, xs[l], ts[l], bs[l], swept ? pre_ - 1 : pre_);
+                const int sweeps = swept ? pre_ - 1 : pre_;
                 const DevLevel F = dl(l), C = dl(l + 1);
                 const T fs = (l + 1 < ld && pre_ > 0) ? two3 : (T)0;
                 if (host_[l].D == 2 && fuse_) {
-                    if (rr_tile_fits(l)) {
-                        const unsigned nbt = (unsigned)(((C.n[0] + kRRRows - 1) / kRRRows) * ((C.n[1] + kRRCols - 1) / kRRCols));
-                        const int ncls = (int)host_[l].dinv.size();
-                        const ResidRestrictArgs<T> ra{F, C, transfer<T>(l), table<T>(l, false), ncls, table<T>(l + 1, false), xs[l], bs[l], bs[l + 1], xs[l + 1], fs};
-                        if (host_[l].compact) run_rr<T, true, true>(nbt, ra);
-                        else run_rr<T, false, true>(nbt, ra);
+                    const int steps = tile_steps(l, false);
+                    const int h = steps ? std::min(sweeps, kMaxFuse) : 0;
+                    smooth_n<T>(l, xs[l], ts[l], bs[l], sweeps - h);
+                    const ResidRestrictArgs<T> ra{F, C, transfer<T>(l), table<T>(l, false), (int)host_[l].dinv.size(), table<T>(l + 1, false), xs[l], bs[l], bs[l + 1], xs[l + 1], fs};
+                    if (steps) {
+                        const int st[2] = {steps / 10, steps % 10};
+                        const int64_t ntc = (C.n[1] + down_cols(h, st[1]) - 1) / down_cols(h, st[1]);
+                        const bool small = small_tiles(((C.n[0] + TileGeom<false>::crows - 1) / TileGeom<false>::crows) * ntc);
+                        const int rows = small ? TileGeom<true>::crows : TileGeom<false>::crows;
+                        const DownTileArgs<T> da{ra, table<T>(l, true), ts[l], two3, h, {st[0], st[1]}};
+                        const unsigned nb = (unsigned)(((C.n[0] + rows - 1) / rows) * ntc);
+                        if (host_[l].compact) run_down<T, true>(small, nb, da);
+                        else run_down<T, false>(small, nb, da);
+                        if (h > 0) std::swap(xs[l], ts[l]);
                     } else {
-                        const ResidRestrictArgs<T> ra{F, C, transfer<T>(l), table<T>(l, false), 0, table<T>(l + 1, false), xs[l], bs[l], bs[l + 1], xs[l + 1], fs};
-                        if (host_[l].compact) run_rr<T, true, false>(nblk(C.N), ra);
-                        else run_rr<T, false, false>(nblk(C.N), ra);
+                        if (host_[l].compact) run_rr<T, true>(nblk(C.N), ra);
+                        else run_rr<T, false>(nblk(C.N), ra);
                     }
                     continue;
                 }
+                smooth_n<T>(l, xs[l], ts[l], bs[l], sweeps);
                 residual<T>(l, xs[l], bs[l], ts[l]);
                 if (host_[l].D == 2)
                     hipLaunchKernelGGL((k_restrict<T, 2>), dim3(nblk(C.N)), dim3(kMgThreads), 0, stream_, F, C, transfer<T>(l), table<T>(l + 1, false), ts[l], bs[l + 1], xs[l + 1], fs);
@@ -3308,31 +3496,40 @@ void mg_batch_launch(const MgBatchPlan& plan, hipStream_t st)
         const unsigned* f = reinterpret_cast<const unsigned*>(base + g.first_off);
         const dim3 grid(g.blocks);
         const uint16_t k = g.kind;
-        if (k < kKindRRTile) {
-            const int v = k - kKindSmooth;
-#define SMT(T, C, P, A)                                                                             \
-    hipLaunchKernelGGL((k_smooth_tile_many<T, C, P, A>), grid, dim3(kTileThreads), 0, st,           \
+        if (k < kKindDown) {
+#define SMT(T, C, P, A)                                                                                                   \
+    hipLaunchKernelGGL((k_smooth_tile_many<T, C, P, A>), grid, dim3(TileGeom<false>::threads), 0, st,                     \
                        static_cast<const SmoothTileArgs<T>*>(a), f, g.n)
-#define SMT4(T, C)                                            \
-    switch (v & 3) {                                          \
-    case 0: SMT(T, C, false, false); break;                   \
-    case 1: SMT(T, C, false, true); break;                    \
-    case 2: SMT(T, C, true, false); break;                    \
-    default: SMT(T, C, true, true); break;                    \
-    }
-            if (v & 8) { if (v & 4) { SMT4(double, true) } else { SMT4(double, false) } }
-            else { if (v & 4) { SMT4(float, true) } else { SMT4(float, false) } }
-#undef SMT4
+            switch (k - kKindSmooth) {
+            case 0: SMT(float, false, false, false); break;
+            case 1: SMT(float, false, false, true); break;
+            case 2: SMT(float, false, true, false); break;
+            case 3: SMT(float, false, true, true); break;
+            case 4: SMT(float, true, false, false); break;
+            case 5: SMT(float, true, false, true); break;
+            case 6: SMT(float, true, true, false); break;
+            case 7: SMT(float, true, true, true); break;
+            case 8: SMT(double, false, false, false); break;
+            case 10: SMT(double, false, true, false); break;
+            case 12: SMT(double, true, false, false); break;
+            case 14: SMT(double, true, true, false); break;
+            default: throw std::logic_error("hip_multigrid: unknown recorded kind");
+            }
 #undef SMT
+        } else if (k < kKindRR) {
+#define DWN(T, C)                                                                                                         \
+    hipLaunchKernelGGL((k_down_tile_many<T, C>), grid, dim3(TileGeom<false>::threads), 0, st,                             \
+                       static_cast<const DownTileArgs<T>*>(a), f, g.n)
+            switch (k - kKindDown) {
+            case 0: DWN(float, false); break;
+            case 1: DWN(float, true); break;
+            case 2: DWN(double, false); break;
+            default: DWN(double, true); break;
+            }
+#undef DWN
         } else if (k < kKindCoarse) {
-            const bool tile = k < kKindRR;
-            const int v = k - (tile ? kKindRRTile : kKindRR);
-#define RRL(T, C)                                                                                   \
-    if (tile) hipLaunchKernelGGL((k_resid_restrict_tile_many<T, C>), grid, dim3(kTileThreads), 0, st, \
-                                 static_cast<const ResidRestrictArgs<T>*>(a), f, g.n);              \
-    else hipLaunchKernelGGL((k_resid_restrict_many<T, C>), grid, dim3(kMgThreads), 0, st,            \
-                            static_cast<const ResidRestrictArgs<T>*>(a), f, g.n)
-            switch (v) {
+#define RRL(T, C) hipLaunchKernelGGL((k_resid_restrict_many<T, C>), grid, dim3(kMgThreads), 0, st, static_cast<const ResidRestrictArgs<T>*>(a), f, g.n)
+            switch (k - kKindRR) {
             case 0: RRL(float, false); break;
             case 1: RRL(float, true); break;
             case 2: RRL(double, false); break;

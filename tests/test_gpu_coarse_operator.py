@@ -114,3 +114,32 @@ def test_switching_to_fixed_cycles_keeps_the_solution(dtype):
         phis.append(st.phi())
         st.close()
     assert np.max(np.abs(phis[0] - phis[1])) <= 1e-9 * np.max(np.abs(phis[0]))
+
+
+@pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
+@pytest.mark.parametrize("kind,nodes,depth", [
+    ("walls", (1100, 300), 6),       # large tiles (210 blocks) with remainders on both axes
+    ("walls", (301, 1153), 6),       # odd counts
+    ("periodic", (512, 464), 5),     # large tiles across the seam
+    ("walls", (199, 62), 3),         # small tiles, even last axis
+    ("periodic", (72, 40), 4),       # 9 x 5 at the end: axes kept as they are
+    ("periodic", (144, 6), 3),       # an axis shorter than a tile's halo
+])
+@pytest.mark.parametrize("prepost", [(1, 1), (2, 1), (4, 4), (7, 2), (0, 5)])
+def test_tile_kernels_match_the_unfused_kernels(backend, kind, nodes, depth, prepost):
+    """The tile kernels (sweeps, prolongation with staged coarse values, the
+    downward half in one launch; both tile sizes) against one launch per
+    sweep and transfer ("fuse 0"): equal bits."""
+    from psum_amd import engine as E
+    nn, r, c, v, b = (_walls if kind == "walls" else _periodic)(nodes, 7)
+    pre, post = prepost
+    out = []
+    for fuse in (0, 1):
+        s = E.SolverBackend(backend)
+        s.set_options(f"I {nodes[0]} J {nodes[1]} depth {depth} pre_relax {pre} post_relax {post} max_cycles 3 "
+                      f"correction_interval 1 fuse {fuse}")
+        s.set_matrix(nn, nn, r, c, v)
+        x = torch.zeros(nn, dtype=torch.float64, device="cuda")
+        s.solve(torch.from_numpy(b).cuda(), x)
+        out.append(x.cpu().numpy())
+    assert np.array_equal(out[0], out[1])
