@@ -74,11 +74,67 @@ __device__ __forceinline__ double wave_max_d(double v)
     return v;
 }
 
+// kAdjPPT consecutive particles per thread of k_adj_push and the nodes of its
+// deposit tile.  A block of 1024 particles in lattice or sorted order covers
+// at most ~64 cells of a row at 16 per cell, plus the drift since the order
+// was made; 4096 nodes (32 KB, 5 blocks per CU) also hold a block that
+// straddles the end of a 256-node row.
+constexpr int kAdjPPT = 4;
+constexpr int kAdjTile = 4096;
+
+// a thread's kAdjPPT values, from p0 on; vec: 16-byte accesses are allowed
+template <typename T>
+__device__ __forceinline__ void adj_load(const T* __restrict__ a, int64_t p0, int64_t n, bool vec, T* v)
+{
+    if (vec && p0 + kAdjPPT <= n) {
+        constexpr int per = 16 / (int)sizeof(T);
+        typedef T vec_t __attribute__((ext_vector_type(per)));
+#pragma unroll
+        for (int j = 0; j < kAdjPPT; j += per) {
+            const vec_t q = *reinterpret_cast<const vec_t*>(a + p0 + j);
+#pragma unroll
+            for (int k = 0; k < per; ++k) v[j + k] = q[k];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kAdjPPT; ++j) v[j] = p0 + j < n ? a[p0 + j] : (T)0;
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void adj_store(T* __restrict__ a, int64_t p0, int64_t n, bool vec, const T* v)
+{
+    if (vec && p0 + kAdjPPT <= n) {
+        constexpr int per = 16 / (int)sizeof(T);
+        typedef T vec_t __attribute__((ext_vector_type(per)));
+#pragma unroll
+        for (int j = 0; j < kAdjPPT; j += per) {
+            vec_t q;
+#pragma unroll
+            for (int k = 0; k < per; ++k) q[k] = v[j + k];
+            *reinterpret_cast<vec_t*>(a + p0 + j) = q;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kAdjPPT; ++j)
+            if (p0 + j < n) a[p0 + j] = v[j];
+    }
+}
+
 // Reverse of kick + drift + gather for one species (in place on lx, lv);
 // gradient-weight deposit of lvt into acc with the device-side scale.
 // T: precision of the positions (the forward state); A: precision of the
 // adjoint state lx, lv, of phi and of the arithmetic (A = double with FP32
 // positions keeps the reverse sweep's accumulations in FP64).
+//
+// One global atomic per support node of every particle (16.8M for 4.2M 2D
+// particles) bounded this kernel: 750 us at 256^2 nodes, 64 per cell, FP32
+// positions.  A block's terms are summed in an LDS tile over the box of its
+// particles' support and the tile is added to acc once: 70 us.  The sums are
+// integers, so the order does not matter.  A thread takes consecutive
+// particles so that the lanes of one LDS atomic lie in several cells.  A
+// block whose box is larger than the tile (unordered particles) adds to acc
+// directly.
 template <typename T, typename A, int D>
 __global__ __launch_bounds__(kA) void k_adj_push(DevGrid g, const T* __restrict__ x0,
                                                  const T* __restrict__ x1, const T* __restrict__ x2,
@@ -87,58 +143,174 @@ __global__ __launch_bounds__(kA) void k_adj_push(DevGrid g, const T* __restrict_
                                                  A* __restrict__ lv1, A* __restrict__ lv2,
                                                  int64_t n, const A* __restrict__ phi, A qm, A dt,
                                                  const double* __restrict__ scale_dev,
-                                                 unsigned long long* __restrict__ acc)
+                                                 unsigned long long* __restrict__ acc, int vec)
 {
-    const int64_t p = (int64_t)blockIdx.x * kA + threadIdx.x;
-    if (p >= n) return;
+    __shared__ unsigned long long tile[kAdjTile];
+    __shared__ int bmin[3], bmax[3], bref[3];
+    const int64_t p0 = ((int64_t)blockIdx.x * kA + threadIdx.x) * kAdjPPT;
     const T* xs[3] = {x0, x1, x2};
     A* lxs[3] = {lx0, lx1, lx2};
     A* lvs[3] = {lv0, lv1, lv2};
-    A x[D], lx[D], lvt[D];
+    T X[D][kAdjPPT];
 #pragma unroll
-    for (int d = 0; d < D; ++d) x[d] = (A)xs[d][p];
-    if (!isfinite((double)x[0])) return;
+    for (int d = 0; d < D; ++d) adj_load(xs[d], p0, n, vec, X[d]);
+    bool live[kAdjPPT], in[kAdjPPT];
+    int cell[kAdjPPT][D];
+#pragma unroll
+    for (int j = 0; j < kAdjPPT; ++j) {
+        live[j] = p0 + j < n && isfinite((double)X[0][j]);
+        in[j] = false;
+        if (live[j]) {
+            double xd[D], s[D];
+#pragma unroll
+            for (int d = 0; d < D; ++d) xd[d] = (double)X[d][j];
+            in[j] = base_cell<D>(g, xd, cell[j], s);
+        }
+    }
+    // box of the block's cells, unwrapped around its first particle's cell
+    // on periodic axes
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            bmin[d] = INT_MAX;
+            bmax[d] = INT_MIN;
+            bref[d] = -1;
+        }
+#pragma unroll
+        for (int j = kAdjPPT - 1; j >= 0; --j)
+            if (in[j])
+#pragma unroll
+                for (int d = 0; d < D; ++d) bref[d] = cell[j][d];
+    }
+    __syncthreads();
+    int uw[kAdjPPT][D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        lx[d] = lxs[d][p];
-        lvt[d] = lvs[d][p] + dt * lx[d];
-    }
-    int cw[D];
-    A W[D][2], G[D][2];
-    if (cic_factors<A, D>(g, x, cw, W, G)) {
-        A ph[1 << D];
+        const int ref = bref[d], w = g.w[d];
+        int lo = INT_MAX, hi = INT_MIN;
 #pragma unroll
-        for (int i = 0; i < (1 << D); ++i) ph[i] = phi[support_index<D>(g, cw, i)];
-        // lx_f -= qm dt sum_e lvt_e H_ef
-#pragma unroll
-        for (int f = 0; f < D; ++f) {
-            A acc_f = (A)0;
-#pragma unroll
-            for (int e = 0; e < D; ++e) {
-                if (e == f) continue;
-                A h = (A)0;
-#pragma unroll
-                for (int i = 0; i < (1 << D); ++i) h = h + ph[i] * cic_hess_coef<A, D>(W, G, i, e, f);
-                acc_f = acc_f + lvt[e] * h;
+        for (int j = 0; j < kAdjPPT; ++j)
+            if (in[j]) {
+                int u = cell[j][d];
+                if (g.periodic[d] && ref >= 0) {
+                    if (u - ref > w / 2) u -= w;
+                    else if (ref - u > w / 2) u += w;
+                }
+                uw[j][d] = u;
+                lo = min(lo, u);
+                hi = max(hi, u);
             }
-            lx[f] = lx[f] - (qm * dt) * acc_f;
+        lo = wave_min_full(lo);
+        hi = wave_max_full(hi);
+        if ((threadIdx.x & 63) == 0 && lo <= hi) {
+            atomicMin(&bmin[d], lo);
+            atomicMax(&bmax[d], hi);
         }
-        // lphi[idx_i] += -qm dt sum_e lvt_e d_e c_i
-        const double scale = scale_dev[0];
-        const double mqdt = -(double)qm * (double)dt;
+    }
+    __syncthreads();
+    // nodes of the box (support adds one per axis); 0: no particle inside
+    int64_t tsize = bmin[0] <= bmax[0] ? 1 : 0;
+    int e[D], lo[D];
 #pragma unroll
-        for (int i = 0; i < (1 << D); ++i) {
-            A t = (A)0;
+    for (int d = 0; d < D; ++d) {
+        lo[d] = bmin[d];
+        e[d] = tsize ? bmax[d] - bmin[d] + 2 : 1;
+        tsize *= e[d];
+    }
+    const bool use_tile = tsize <= kAdjTile;
+    if (use_tile)
+        for (int i = threadIdx.x; i < (int)tsize; i += kA) tile[i] = 0ull;
+    __syncthreads();
+    int st[D];
+    st[D - 1] = 1;
 #pragma unroll
-            for (int e = 0; e < D; ++e) t = t + lvt[e] * cic_grad_coef<A, D>(W, G, i, e);
-            const long long term = round_to_ll((mqdt * (double)t) * scale);
-            if (term) atomicAdd(&acc[support_index<D>(g, cw, i)], (unsigned long long)term);
+    for (int d = D - 2; d >= 0; --d) st[d] = st[d + 1] * e[d + 1];
+
+    A LX[D][kAdjPPT], LV[D][kAdjPPT];
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        adj_load(lxs[d], p0, n, vec, LX[d]);
+        adj_load(lvs[d], p0, n, vec, LV[d]);
+    }
+    const double scale = scale_dev[0];
+    const double mqdt = -(double)qm * (double)dt;
+#pragma unroll
+    for (int j = 0; j < kAdjPPT; ++j) {
+        if (!live[j]) continue;
+        A x[D], lx[D], lvt[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            x[d] = (A)X[d][j];
+            lx[d] = LX[d][j];
+            lvt[d] = LV[d][j] + dt * lx[d];
+        }
+        int cw[D];
+        A W[D][2], G[D][2];
+        if (cic_factors<A, D>(g, x, cw, W, G)) {
+            A ph[1 << D];
+#pragma unroll
+            for (int i = 0; i < (1 << D); ++i) ph[i] = phi[support_index<D>(g, cw, i)];
+            // lx_f -= qm dt sum_e lvt_e H_ef
+#pragma unroll
+            for (int f = 0; f < D; ++f) {
+                A acc_f = (A)0;
+#pragma unroll
+                for (int q = 0; q < D; ++q) {
+                    if (q == f) continue;
+                    A h = (A)0;
+#pragma unroll
+                    for (int i = 0; i < (1 << D); ++i) h = h + ph[i] * cic_hess_coef<A, D>(W, G, i, q, f);
+                    acc_f = acc_f + lvt[q] * h;
+                }
+                lx[f] = lx[f] - (qm * dt) * acc_f;
+            }
+            // lphi[idx_i] += -qm dt sum_e lvt_e d_e c_i
+            int li = 0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) li += (uw[j][d] - lo[d]) * st[d];
+#pragma unroll
+            for (int i = 0; i < (1 << D); ++i) {
+                A t = (A)0;
+#pragma unroll
+                for (int q = 0; q < D; ++q) t = t + lvt[q] * cic_grad_coef<A, D>(W, G, i, q);
+                const long long term = round_to_ll((mqdt * (double)t) * scale);
+                if (use_tile) {
+                    int o = li;
+#pragma unroll
+                    for (int d = 0; d < D; ++d) o += ((i >> (D - 1 - d)) & 1) * st[d];
+                    atomicAdd(&tile[o], (unsigned long long)term);
+                } else if (term) {
+                    atomicAdd(&acc[support_index<D>(g, cw, i)], (unsigned long long)term);
+                }
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            LX[d][j] = lx[d];
+            LV[d][j] = lvt[d];
         }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        lxs[d][p] = lx[d];
-        lvs[d][p] = lvt[d];
+        adj_store(lxs[d], p0, n, vec, LX[d]);
+        adj_store(lvs[d], p0, n, vec, LV[d]);
+    }
+    if (!use_tile) return;   // the same in every thread
+    __syncthreads();
+    for (int i = threadIdx.x; i < (int)tsize; i += kA) {
+        const unsigned long long t = tile[i];
+        if (!t) continue;
+        uint32_t lin = 0;
+        int rest = i;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            int c = lo[d] + rest / st[d];
+            rest %= st[d];
+            if (c < 0) c += g.w[d];
+            else if (c >= g.w[d]) c -= g.w[d];
+            lin = d == 0 ? (uint32_t)c : lin * (uint32_t)g.w[d] + (uint32_t)c;
+        }
+        atomicAdd(&acc[lin], t);
     }
 }
 
@@ -200,24 +372,27 @@ __global__ __launch_bounds__(kA) void k_adj_gather(DevGrid g, const T* __restric
     }
 }
 
+// one workgroup bound by the latency of its serial loads: 1024 threads, 8
+// loads in flight each (16384 maxima: 16.6 -> 4.7 us)
+constexpr int kScale = 1024;
+
 // max over nb block maxima, then scale = 2^(40 - e) with 2^(e-1) <= bound < 2^e,
 // bound = max |qm dt| * max_d delta_r * max sum_e |lvt_e| (the largest term);
 // scale_out[0] = scale, scale_out[1] = 1/scale
-__global__ __launch_bounds__(kA) void k_adj_scale(const double* __restrict__ bmax, int64_t nb,
-                                                  double factor, double* __restrict__ scale_out,
-                                                  int accumulate)
+__global__ __launch_bounds__(kScale) void k_adj_scale(const double* __restrict__ bmax, int64_t nb,
+                                                      double factor, double* __restrict__ scale_out,
+                                                      int accumulate)
 {
-    __shared__ double sh[kA];
+    __shared__ double sh[kScale / 64];
     double m = 0.0;
-    for (int64_t b = threadIdx.x; b < nb; b += kA) m = fmax(m, bmax[b]);
-    sh[threadIdx.x] = m;
+#pragma unroll 8
+    for (int64_t b = threadIdx.x; b < nb; b += kScale) m = fmax(m, bmax[b]);
+    m = wave_max_d(m);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
     __syncthreads();
-    for (int w = kA / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + w]);
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
-        double bound = sh[0] * factor;
+        for (int w = 1; w < kScale / 64; ++w) m = fmax(m, sh[w]);
+        double bound = m * factor;
         if (accumulate) bound = fmax(bound, scale_out[2]);
         scale_out[2] = bound;
         int e = 0;
@@ -342,10 +517,15 @@ psum_status launch_adj_push(const psum_grid* g, void* const* x, void* const* lx,
     const DevGrid dg = to_dev(*g);
     auto P = [&](void* const* a, int d) { return d < D ? static_cast<T*>(a[d]) : nullptr; };
     auto Q = [&](void* const* a, int d) { return d < D ? static_cast<A*>(a[d]) : nullptr; };
-    hipLaunchKernelGGL((k_adj_push<T, A, D>), dim3(nblk(n, kA)), dim3(kA), 0, st, dg, P(x, 0), P(x, 1),
-                       P(x, 2), Q(lx, 0), Q(lx, 1), Q(lx, 2), Q(lv, 0), Q(lv, 1), Q(lv, 2), n,
+    // 16-byte accesses where every component starts on 16 bytes
+    int vec = 1;
+    for (int d = 0; d < D; ++d)
+        for (const void* p : {(const void*)x[d], (const void*)lx[d], (const void*)lv[d]})
+            if ((uintptr_t)p & 15) vec = 0;
+    hipLaunchKernelGGL((k_adj_push<T, A, D>), dim3(nblk(n, kA * kAdjPPT)), dim3(kA), 0, st, dg, P(x, 0),
+                       P(x, 1), P(x, 2), Q(lx, 0), Q(lx, 1), Q(lx, 2), Q(lv, 0), Q(lv, 1), Q(lv, 2), n,
                        static_cast<const A*>(phi), (A)qm, (A)dt, scale_dev,
-                       reinterpret_cast<unsigned long long*>(acc));
+                       reinterpret_cast<unsigned long long*>(acc), vec);
     PSUM_HIP_TRY(hipGetLastError());
     return PSUM_OK;
 }
@@ -414,7 +594,7 @@ psum_status psum_hip_adjoint_gather(const psum_grid* g, int dtype, void* const* 
 psum_status psum_hip_adjoint_scale(const double* bmax, int64_t nb, double factor, double* scale_dev,
                                    int accumulate, void* stream)
 {
-    hipLaunchKernelGGL(k_adj_scale, dim3(1), dim3(kA), 0, S(stream), bmax, nb, factor, scale_dev,
+    hipLaunchKernelGGL(k_adj_scale, dim3(1), dim3(kScale), 0, S(stream), bmax, nb, factor, scale_dev,
                        accumulate);
     PSUM_HIP_TRY(hipGetLastError());
     return PSUM_OK;
