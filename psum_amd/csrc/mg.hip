@@ -703,9 +703,13 @@ __device__ __forceinline__ int batch_instance(const unsigned* __restrict__ first
 // beyond a non-wrapped edge are clamped copies: the stencils of real nodes
 // give them zero coefficients, as in k_smooth's clamped neighbour.
 //
-// Everything a block reads is asked for before its first barrier (transfer
-// tables, coarse values, weights of the restriction): on small levels a
-// launch is a chain of memory round trips, not bandwidth.  Two geometries:
+// Everything a block reads is asked for in one run of unconditional loads
+// before its first barrier (transfer tables, coarse values, weights of the
+// restriction): on small levels a launch is a chain of memory round trips and
+// of instruction fetches, not bandwidth.  128^2 and 64^2 FP64 levels of 256
+// threads a block: 6.7-7.9 us a launch with copy loops and conditional loads,
+// 5.7-6.7 us so; 1024^2 FP32: 19.7 and 20.0 -> 17.3 and 18.8 us.  Two
+// geometries:
 // 1024 threads over 32 rows (16 coarse rows), and 256 threads over 8 rows
 // (3 coarse rows) for levels whose large tiles would leave most compute units
 // idle (small_tiles()).
@@ -723,22 +727,52 @@ struct TileGeom {
     // one guard row on each side, one guard value before and after: tile row
     // i, column tx at at(i, tx)
     static constexpr int plane = (groups * rpt + 2) * kTileX + 2;
+    // values of a class table, and of the coarse values a prolongation reads
+    // (cw columns, ch rows), each thread brings into LDS
+    static constexpr int tab_per = (kMaxClsLds * 9 + threads - 1) / threads;
+    static constexpr int cw = kTileX / 2 + 2, ch = (groups * rpt) / 2 + 2;
+    static constexpr int xc_per = (cw * ch + threads - 1) / threads;
     static __device__ __forceinline__ int at(int i, int tx) { return (i + 1) * kTileX + tx + 1; }
     static_assert(rows + 2 * kMaxFuse <= groups * rpt, "smoothing tile exceeds its planes");
     static_assert(2 * crows + 1 + 2 + 2 * kMaxFuse <= groups * rpt, "k_down_tile tile exceeds its planes");
     static_assert(crows <= groups, "one coarse row per wave");
 };
 
-// wrapped (periodic axis) or clamped node coordinate; g is at most a few
-// nodes outside [0, n)
+// The thread's share of a class table, loaded to registers and stored to LDS
+// later: a loop that copies global to LDS waits for memory in every turn, so
+// the tile's other loads would only be asked for after it (a round trip is
+// 0.5-1 us on lines that another XCD wrote).
+template <bool SMALL, typename T>
+__device__ __forceinline__ void tab_load(const T* __restrict__ coef, int n, T* v)
+{
+#pragma unroll
+    for (int q = 0; q < TileGeom<SMALL>::tab_per; ++q) {
+        const int i = threadIdx.x + q * TileGeom<SMALL>::threads;
+        v[q] = coef[i < n ? i : 0];
+    }
+}
+template <bool SMALL, typename T>
+__device__ __forceinline__ void tab_store(T* lds, int n, const T* v)
+{
+#pragma unroll
+    for (int q = 0; q < TileGeom<SMALL>::tab_per; ++q) {
+        const int i = threadIdx.x + q * TileGeom<SMALL>::threads;
+        if (i < n) lds[i] = v[q];
+    }
+}
+
+// wrapped (periodic axis) or clamped node coordinate; g is less than two
+// tiles outside [0, n).  Without loops or branches (they were a third of the
+// tile kernels' code): the float quotient is off by at most one below 2^23
+// periods, which the selects mend.
 __device__ __forceinline__ int tile_coord(int g, int n, int wrap)
 {
-    if (wrap) {
-        while (g < 0) g += n;
-        while (g >= n) g -= n;
-        return g;
-    }
-    return g < 0 ? 0 : (g >= n ? n - 1 : g);
+    const int q = (int)floorf((float)g * __builtin_amdgcn_rcpf((float)n));
+    int m = g - q * n;
+    m = m < 0 ? m + n : m;
+    m = m >= n ? m - n : m;
+    const int w = wrap ? -1 : 0;
+    return (m & w) | (min(max(g, 0), n - 1) & ~w);
 }
 
 template <typename T, bool COMPACT>
@@ -850,7 +884,7 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
 {
     using G = TileGeom<SMALL>;
     constexpr int RPT = G::rpt;
-    constexpr int CW = kTileX / 2 + 2, CH = (G::groups * RPT) / 2 + 2;   // staged coarse values
+    constexpr int CW = G::cw, CH = G::ch;   // staged coarse values
     const DevLevel& L = A.L;
     const DevTable<T>& relax = A.relax;
     const int h = A.h;
@@ -867,18 +901,31 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
     const int t0 = (int)(bid / ntc) * G::rows, t1 = (int)(bid % ntc) * ostep;
     const int R = G::rows + 2 * h;
     const bool lds_tab = A.ncls <= kMaxClsLds;
-    if (lds_tab)
-        for (int i = threadIdx.x; i < A.ncls * 9; i += G::threads) ctab[i] = relax.coef[i];
+    // coordinates first, then every load in one straight run (a load under a
+    // condition is waited for where the paths join); rows beyond the tile
+    // repeat its last
     const int g1 = tile_coord(t1 - h + tx, n1, L.wrap[1]);
+    int g0[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) g0[k] = tile_coord(t0 - h + min(i0 + k, R - 1), n0, L.wrap[0]);
     // coarse rows and columns lo .. lo + CH - 1, CW - 1 hold every value the
     // tile interpolates from when both axes halve
     const int lo0 = (t0 - h) >> 1, lo1 = (t1 - h) >> 1;
     const bool staged = PROLONG && A.half;
+    int64_t ic[G::xc_per];
     if (staged)
-        for (int i = threadIdx.x; i < CW * CH; i += G::threads) {
+#pragma unroll
+        for (int k = 0; k < G::xc_per; ++k) {
+            const int i = threadIdx.x + k * G::threads;
             const int r = i / CW, q = i - r * CW;
-            sxc[i] = xc[(int64_t)tile_coord(lo0 + r, Cl.n[0], tr.wrap[0]) * Cl.n[1] + tile_coord(lo1 + q, Cl.n[1], tr.wrap[1])];
+            ic[k] = (int64_t)tile_coord(lo0 + min(r, CH - 1), Cl.n[0], tr.wrap[0]) * Cl.n[1] +
+                    tile_coord(lo1 + q, Cl.n[1], tr.wrap[1]);
         }
+    T tab[G::tab_per], cv[G::xc_per];
+    if (staged)
+#pragma unroll
+        for (int k = 0; k < G::xc_per; ++k) cv[k] = xc[ic[k]];
+    if (lds_tab) tab_load<SMALL>(relax.coef, A.ncls * 9, tab);
     T breg[RPT], xv[RPT];
     int creg[RPT];
     double xa[RPT];
@@ -893,29 +940,27 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
     const bool colout = tx >= h && tx < kTileX - h && g1o < n1;
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
-        const int i = i0 + k;
-        breg[k] = (T)0;
-        xv[k] = (T)0;
-        creg[k] = 0;
-        xa[k] = 0.0;
-        p0[k] = 0;
-        w0[k][0] = w0[k][1] = (T)0;
-        if (i < R) {
-            const int g0 = tile_coord(t0 - h + i, n0, L.wrap[0]);
-            const int64_t gi = (int64_t)g0 * n1 + g1;
-            xv[k] = A.xin[gi];
-            breg[k] = A.b[gi];
-            creg[k] = L.cls[gi];
-            if (PROLONG) {
-                p0[k] = tr.pc[0][g0];
-                w0[k][0] = tr.pw[0][2 * g0];
-                w0[k][1] = tr.pw[0][2 * g0 + 1];
-            }
-            if (ACC && colout && i >= h && i < h + G::rows && t0 + i - h < n0) xa[k] = A.xacc[gi];
+        const int64_t gi = (int64_t)g0[k] * n1 + g1;
+        xv[k] = A.xin[gi];
+        breg[k] = A.b[gi];
+        creg[k] = L.cls[gi];
+        if (PROLONG) {
+            p0[k] = tr.pc[0][g0[k]];
+            w0[k][0] = tr.pw[0][2 * g0[k]];
+            w0[k][1] = tr.pw[0][2 * g0[k] + 1];
         }
+        if (ACC) xa[k] = A.xacc[gi];
     }
+    if (lds_tab) tab_store<SMALL>(ctab, A.ncls * 9, tab);
     if (PROLONG) {
-        if (staged) __syncthreads();
+        if (staged) {
+#pragma unroll
+            for (int k = 0; k < G::xc_per; ++k) {
+                const int i = threadIdx.x + k * G::threads;
+                if (i < CW * CH) sxc[i] = cv[k];
+            }
+            __syncthreads();
+        }
         int q1[2];
         if (staged) {
             q1[0] = (tr.wrap[1] ? (t1 - h + tx) >> 1 : p1) - lo1;
@@ -1035,49 +1080,47 @@ __device__ __forceinline__ void down_tile_body(const DownTileArgs<T>& A, unsigne
     const int R = A.st[0] * (c0hi - c0lo) + (A.st[0] - 1) + 2 + 2 * h;
     const int W = A.st[1] * (c1hi - c1lo) + (A.st[1] - 1) + 2 + 2 * h;
     const bool lds_tab = A.r.ncls <= kMaxClsLds;
-    if (lds_tab)
-        for (int i = threadIdx.x; i < A.r.ncls * 9; i += G::threads) {
-            atab[i] = A.r.Af.coef[i];
-            rtab[i] = A.relax.coef[i];
-        }
     const int tx = threadIdx.x & (kTileX - 1), ty = threadIdx.x / kTileX, i0 = ty * RPT;
     const int n0 = F.n[0], n1 = F.n[1];
+    // as in smooth_tile_body: coordinates, then the loads in one run
     const int g1 = tile_coord(u1 + tx, n1, F.wrap[1]);
+    int g0[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) g0[k] = tile_coord(u0 + min(i0 + k, R - 1), n0, F.wrap[0]);
+    T ta[G::tab_per], tb[G::tab_per];
+    if (lds_tab) {
+        tab_load<SMALL>(A.r.Af.coef, A.r.ncls * 9, ta);
+        tab_load<SMALL>(A.relax.coef, A.r.ncls * 9, tb);
+    }
     T breg[RPT], xv[RPT];
     int creg[RPT];
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
-        const int i = i0 + k;
-        breg[k] = (T)0;
-        xv[k] = (T)0;
-        creg[k] = 0;
-        if (i < R && tx < W) {
-            const int64_t gi = (int64_t)tile_coord(u0 + i, n0, F.wrap[0]) * n1 + g1;
-            xv[k] = A.r.x[gi];
-            breg[k] = A.r.bf[gi];
-            creg[k] = F.cls[gi];
-        }
+        const int64_t gi = (int64_t)g0[k] * n1 + g1;
+        xv[k] = A.r.x[gi];
+        breg[k] = A.r.bf[gi];
+        creg[k] = F.cls[gi];
     }
     // the coarse node this thread sums: its support and weights
     const int c0 = c0lo + ty, c1 = c1lo + tx;
     const bool coarse = ty < G::crows && tx < CC && c0 < c0hi && c1 < c1hi;
-    int f0 = 0, m0 = 0, f1 = 0, m1 = 0;
-    T rw0[3] = {(T)0, (T)0, (T)0}, rw1[3] = {(T)0, (T)0, (T)0}, dinv = (T)0;
-    if (coarse) {
-        f0 = tr.rf[0][c0];
-        m0 = tr.rn[0][c0];
-        f1 = tr.rf[1][c1];
-        m1 = tr.rn[1][c1];
+    const int c0r = min(c0, Cl.n[0] - 1), c1r = min(c1, Cl.n[1] - 1);
+    const int f0 = tr.rf[0][c0r], m0 = tr.rn[0][c0r], f1 = tr.rf[1][c1r], m1 = tr.rn[1][c1r];
+    T rw0[3], rw1[3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            rw0[q] = tr.rw[0][3 * c0 + q];
-            rw1[q] = tr.rw[1][3 * c1 + q];
-        }
-        dinv = A.r.Ac.dinv[Cl.cls[(int64_t)c0 * Cl.n[1] + c1]];
+    for (int q = 0; q < 3; ++q) {
+        rw0[q] = tr.rw[0][3 * c0r + q];
+        rw1[q] = tr.rw[1][3 * c1r + q];
+    }
+    const int cc = Cl.cls[(int64_t)c0r * Cl.n[1] + c1r];
+    if (lds_tab) {
+        tab_store<SMALL>(atab, A.r.ncls * 9, ta);
+        tab_store<SMALL>(rtab, A.r.ncls * 9, tb);
     }
 #pragma unroll
     for (int k = 0; k < RPT; ++k)
         if (i0 + k < R) sx[0][G::at(i0 + k, tx)] = xv[k];
+    const T dinv = A.r.Ac.dinv[cc];
     __syncthreads();
     auto row_of = [&](const T* lds, const T* coef, int k) {
         TileRow<T, COMPACT> r;
@@ -2777,11 +2820,15 @@ private:
     float host_dinv32(int l, int k) const { return (float)host_[l].dinv[k]; }
 
     // 3D transfers writing level l over planes (k_prolong_add_plane,
-    // k_restrict_plane): levels of 2^15 nodes or more
+    // k_restrict_plane): planes of at least a wave, since a launch is a chain
+    // of memory round trips and the per-node kernels' are longer (a term's
+    // load waits for the one before).  Restriction to 26 x 23 x 31 and
+    // 14 x 12 x 16 nodes in FP64: 11.9 -> 4.9 us.
     bool planar(int l) const
     {
-        return line_ && host_[l].D == 3 && host_[l].N >= (1 << 15) && host_[l].N < (int64_t)0xffffffffll &&
-               (l == 0 || host_[l - 1].N < (int64_t)0xffffffffll);
+        const HostLevel& h = host_[l];
+        return line_ && h.D == 3 && (int64_t)h.n[1] * h.n[2] >= 64 && h.n[0] <= 65535 &&
+               h.N < (int64_t)0xffffffffll && (l == 0 || host_[l - 1].N < (int64_t)0xffffffffll);
     }
 
     LineList line_list(int l) const
