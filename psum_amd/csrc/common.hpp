@@ -24,6 +24,16 @@ psum_status bin_keys(const psum_grid* g, int dtype, void* const* pos, int64_t n,
                      int shift, void* stream, void* const* vel = nullptr);
 uint32_t bin_count(const psum_grid& g, int shift);
 
+// dst[c][i] = src[c][perm[i]] for particles whose order may be random: the
+// result is in dst (*far = 0) or in src (*far = 1, the permutation has no
+// order and the copy went through records in dst), *far a word of device
+// memory.  dst and perm are 16-byte aligned, n < 2^32; tail: at least 256
+// bytes of device memory, free during the call.  permute_either_applies()
+// says for which components and sizes.
+bool permute_either_applies(int dtype, int ncomp, int64_t n);
+psum_status permute_either(int dtype, int ncomp, void* const* src, void* const* dst, const uint32_t* perm, int64_t n,
+                           void* tail, uint32_t* far, void* stream);
+
 #define PSUM_HIP_TRY(expr)                                                              \
     do {                                                                                \
         hipError_t e_ = (expr);                                                         \

@@ -17,6 +17,7 @@
 // rounded operations in the order written (the CPU oracle does the same).
 
 #include <climits>
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -154,36 +155,68 @@ __global__ __launch_bounds__(kThreads) void k_scan_add(uint32_t* __restrict__ ou
 }
 
 // ------------------------------------------------------------- radix sort
-// Stable LSD radix sort, 8-bit digits.  A block owns a tile of 4096 keys;
-// wave w owns the contiguous quarter [w*1024, (w+1)*1024) and visits it in
-// 16 rows of 64 keys, so lane order within a row and row order within the
-// wave are index order.  Within-wave stable ranks come from 8 ballots per
-// key (lanes with equal digit), across waves from per-wave digit counts.
+// Stable LSD radix sort, digits of 8 to 10 bits: the fewest passes at 10 bits
+// a digit, the bits then dealt evenly (a pass reads and writes every key and
+// index, so 17..20-bit keys in two passes instead of three).  A block of W
+// waves owns a tile of W*1024 keys; wave w owns the contiguous part [w*1024,
+// (w+1)*1024) and visits it in 16 rows of 64 keys, so lane order within a row
+// and row order within the wave are index order.  Within-wave stable ranks
+// come from one ballot per digit bit and key (lanes with equal digit), across
+// waves from per-wave digit counts.  Tiles are dealt to the XCDs in
+// contiguous eighths: the next tile's keys of a digit follow this one's in
+// memory, and the partly written line is then completed in the same L2.
+// Between passes key and index travel as one 8-byte pair.  Bound by the
+// scattered writes.  67M random 19-bit keys: 2.4 ms (three passes of 8 bits)
+// -> 1.6 ms; 105M nearly sorted 23-bit keys: 2.7 -> 1.8 ms.
 
-constexpr int kSortWaveItems = 16;
-constexpr int kSortTile = kThreads * kSortWaveItems;
+constexpr int kSortItems = 16;
+constexpr int kSortWaveTile = 64 * kSortItems;
+constexpr int kSortMaxBits = 10;
+constexpr int kSortSmallTile = 4 * kSortWaveTile;   // tile of 4-wave blocks
 
-__device__ __forceinline__ uint32_t sort_digit(uint32_t key, uint32_t nkeys, int shift)
+// waves per block: 8 (fewer digit counts to scan per key) where that still
+// gives every compute unit two blocks
+inline int sort_waves(int64_t n) { return n >= (int64_t)512 * 8 * kSortWaveTile ? 8 : 4; }
+
+__device__ __forceinline__ uint32_t sort_digit(uint32_t key, uint32_t nkeys, int shift, uint32_t mask)
 {
     const uint32_t k = key == PSUM_KEY_INVALID ? nkeys : key;
-    return (k >> shift) & 255u;
+    return (k >> shift) & mask;
 }
 
-__global__ __launch_bounds__(kThreads) void k_sort_hist(const uint32_t* __restrict__ keys,
-                                                        int64_t n, uint32_t nkeys, int shift,
-                                                        uint32_t* __restrict__ ghist, int nb)
+// tile of this block: XCD b % 8 works through one contiguous eighth (a
+// bijection for any block count: blocks beyond the last multiple of 8 keep
+// their index)
+__device__ __forceinline__ int64_t sort_block()
 {
-    __shared__ uint32_t hist[256];
-    hist[threadIdx.x] = 0;
+    const unsigned g = gridDim.x, b = blockIdx.x, full = g / 8u * 8u;
+    return b >= full ? b : (int64_t)(b % 8u) * (full / 8u) + b / 8u;
+}
+
+template <int W, bool PAIRS>
+__global__ __launch_bounds__(64 * W) void k_sort_hist(const uint32_t* __restrict__ keys,
+                                                      int64_t n, uint32_t nkeys, int shift, int bits,
+                                                      uint32_t* __restrict__ ghist, int nb)
+{
+    __shared__ uint32_t hist[1 << kSortMaxBits];
+    const int R = 1 << bits;
+    for (int d = threadIdx.x; d < R; d += 64 * W) hist[d] = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t base = (int64_t)blockIdx.x * kSortTile + wave * (64 * kSortWaveItems);
+    const int64_t tile = sort_block();
+    const int64_t base = (tile * W + wave) * kSortWaveTile;
+    uint32_t key[kSortItems];
 #pragma unroll
-    for (int j = 0; j < kSortWaveItems; ++j) {
+    for (int j = 0; j < kSortItems; ++j) {
+        const int64_t p = base + j * 64 + lane;
+        key[j] = p < n ? keys[PAIRS ? 2 * p : p] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kSortItems; ++j) {
         const int64_t p = base + j * 64 + lane;
         if (base + j * 64 >= n) break;   // no active key in this row (uniform)
         const bool act = p < n;
-        const uint32_t d = act ? sort_digit(keys[p], nkeys, shift) : 0u;
+        const uint32_t d = sort_digit(key[j], nkeys, shift, (uint32_t)R - 1u);
         // a row whose keys share one digit (nearly sorted keys) counts them
         // with one add; the counts are the same
         const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
@@ -195,38 +228,53 @@ __global__ __launch_bounds__(kThreads) void k_sort_hist(const uint32_t* __restri
         }
     }
     __syncthreads();
-    ghist[(int64_t)threadIdx.x * nb + blockIdx.x] = hist[threadIdx.x];
+    for (int d = threadIdx.x; d < R; d += 64 * W) ghist[(int64_t)d * nb + tile] = hist[d];
 }
 
-__global__ __launch_bounds__(kThreads) void k_sort_scatter(
+// vin: the indices (null: identity); PIN / POUT: keys and indices as 8-byte
+// pairs in kin / kout
+template <int W, bool PIN, bool POUT>
+__global__ __launch_bounds__(64 * W) void k_sort_scatter(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, int64_t n,
-    uint32_t nkeys, int shift, const uint32_t* __restrict__ goff, int nb,
+    uint32_t nkeys, int shift, int bits, const uint32_t* __restrict__ goff, int nb,
     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout)
 {
-    __shared__ uint32_t off[256];
-    __shared__ uint32_t whist[kThreads / 64][256];
+    __shared__ uint32_t whist[W][1 << kSortMaxBits];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    off[threadIdx.x] = goff[(int64_t)threadIdx.x * nb + blockIdx.x];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) whist[wave][lane + 64 * q] = 0;
-    __syncthreads();
-
-    const int64_t base = (int64_t)blockIdx.x * kSortTile + wave * (64 * kSortWaveItems);
+    const int R = 1 << bits;
+    const int64_t tile = sort_block();
+    for (int d = lane; d < R; d += 64) whist[wave][d] = 0;
+    __builtin_amdgcn_wave_barrier();
+    const int64_t base = (tile * W + wave) * kSortWaveTile;
     const uint64_t lt = __lanemask_lt();
-    uint32_t key[kSortWaveItems], val[kSortWaveItems], rank[kSortWaveItems];
+    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
 #pragma unroll
-    for (int j = 0; j < kSortWaveItems; ++j) {
+    for (int j = 0; j < kSortItems; ++j) {
         const int64_t p = base + j * 64 + lane;
         const bool act = p < n;
-        key[j] = act ? kin[p] : 0u;
-        val[j] = act ? (vin ? vin[p] : (uint32_t)p) : 0u;
-        const uint32_t d = sort_digit(key[j], nkeys, shift);
+        if constexpr (PIN) {
+            const uint2 q = act ? reinterpret_cast<const uint2*>(kin)[p] : make_uint2(0u, 0u);
+            key[j] = q.x;
+            val[j] = q.y;
+        } else {
+            key[j] = act ? kin[p] : 0u;
+            val[j] = act ? (vin ? vin[p] : (uint32_t)p) : 0u;
+        }
+    }
+    // (each wave counts in its own row of whist: no barrier needed before)
+#pragma unroll
+    for (int j = 0; j < kSortItems; ++j) {
+        const int64_t p = base + j * 64 + lane;
+        const bool act = p < n;
+        const uint32_t d = sort_digit(key[j], nkeys, shift, (uint32_t)R - 1u);
         uint64_t peers = __ballot(act);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < kSortMaxBits; ++b) {
+            if (b >= bits) break;            // uniform
             const uint64_t bal = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? bal : ~bal;
         }
+        rank[j] = 0u;
         if (act) {
             const uint32_t before = whist[wave][d];
             rank[j] = before + (uint32_t)__popcll(peers & lt);
@@ -234,15 +282,28 @@ __global__ __launch_bounds__(kThreads) void k_sort_scatter(
         }
     }
     __syncthreads();
+    // counts -> where each wave's keys of the digit start
+    for (int d = threadIdx.x; d < R; d += 64 * W) {
+        uint32_t run = goff[(int64_t)d * nb + tile];
 #pragma unroll
-    for (int j = 0; j < kSortWaveItems; ++j) {
+        for (int w = 0; w < W; ++w) {
+            const uint32_t c = whist[w][d];
+            whist[w][d] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSortItems; ++j) {
         const int64_t p = base + j * 64 + lane;
         if (p < n) {
-            const uint32_t d = sort_digit(key[j], nkeys, shift);
-            uint32_t dst = off[d] + rank[j];
-            for (int w = 0; w < wave; ++w) dst += whist[w][d];
-            kout[dst] = key[j];
-            vout[dst] = val[j];
+            const uint32_t dst = whist[wave][sort_digit(key[j], nkeys, shift, (uint32_t)R - 1u)] + rank[j];
+            if constexpr (POUT) {
+                reinterpret_cast<uint2*>(kout)[dst] = make_uint2(key[j], val[j]);
+            } else {
+                kout[dst] = key[j];
+                vout[dst] = val[j];
+            }
         }
     }
 }
@@ -284,8 +345,10 @@ struct PtrPack {
 // for all but the last thread, which goes one by one)
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_permute4(PtrPack pk, int ncomp,
-                                                       const uint32_t* __restrict__ perm, int64_t n)
+                                                       const uint32_t* __restrict__ perm, int64_t n,
+                                                       const uint32_t* __restrict__ far = nullptr)
 {
+    if (far && *far) return;      // taken by k_gather_records
     const int64_t i0 = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * 4;
     if (i0 >= n) return;
     if (i0 + 4 <= n) {
@@ -313,6 +376,109 @@ __global__ __launch_bounds__(kThreads) void k_permute(PtrPack pk, int ncomp,
     const uint32_t s = perm[i];
     for (int c = 0; c < ncomp; ++c)
         static_cast<T*>(pk.dst[c])[i] = static_cast<const T*>(pk.src[c])[s];
+}
+
+// ---- permutation of unordered particles through records ------------------
+// A gather of C component arrays through a random permutation fetches a
+// 128-byte line per value: 6 FP32 components of 67M particles took 8.9 ms,
+// 5.8 TB/s of lines of which 1/32 is used.  Copied into records of C values
+// first, a particle costs one line (sometimes two): 0.7 ms of copy, 2.1 ms of gather.  An ordered
+// permutation (particles sorted before) reads whole lines as it is and the
+// copy would only add to it, so k_perm_far samples the permutation and the
+// kernels of the route not taken return at once.
+//
+// The records take no memory of their own: with m = n / C, particles
+// [k m, (k + 1) m) of all components lie in scratch array k (n values), the
+// n % C last ones in `tail`; the gather then writes the source arrays, which
+// the copy left free.
+
+// *far = 1 where most neighbours in the permuted order come from more than
+// kFarStep particles apart (n >= 2 * kFarSamples)
+constexpr int kFarSamples = 4096, kFarStep = 1024;
+__global__ __launch_bounds__(1024) void k_perm_far(const uint32_t* __restrict__ perm, int64_t n,
+                                                   uint32_t* __restrict__ far)
+{
+    __shared__ int cnt;
+    if (threadIdx.x == 0) cnt = 0;
+    __syncthreads();
+    const int64_t step = (n - 1) / kFarSamples;
+    int c = 0;
+#pragma unroll
+    for (int q = 0; q < kFarSamples / 1024; ++q) {
+        const int64_t i = (int64_t)(threadIdx.x + q * 1024) * step;
+        const uint32_t a = perm[i], b = perm[i + 1];
+        c += (a > b ? a - b : b - a) > (uint32_t)kFarStep;
+    }
+    atomicAdd(&cnt, c);
+    __syncthreads();
+    if (threadIdx.x == 0) *far = cnt > kFarSamples / 2 ? 1u : 0u;
+}
+
+// the record of particle p
+template <typename T, int C>
+__device__ __forceinline__ T* record_of(const PtrPack& pk, T* tail, uint32_t p, uint32_t m)
+{
+    uint32_t k = 0;
+#pragma unroll
+    for (int j = 1; j <= C; ++j) k += p >= (uint32_t)j * m ? 1u : 0u;
+    T* base = k < (uint32_t)C ? static_cast<T*>(pk.dst[k]) : tail;
+    return base + (size_t)(p - k * m) * C;
+}
+
+template <typename T, int C>
+__global__ __launch_bounds__(kThreads) void k_pack_records(PtrPack pk, T* __restrict__ tail, uint32_t n, uint32_t m,
+                                                           const uint32_t* __restrict__ far)
+{
+    if (!*far) return;
+    for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < n; p += (int64_t)gridDim.x * kThreads) {
+        T* r = record_of<T, C>(pk, tail, (uint32_t)p, m);
+        T v[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) v[c] = static_cast<const T*>(pk.src[c])[p];
+        // (records of 4 or 6 values start on two values)
+#pragma unroll
+        for (int c = 0; c < C; c += 2) {
+            typedef T vec2 __attribute__((ext_vector_type(2)));
+            vec2 q;
+            q.x = v[c];
+            q.y = v[c + 1];
+            *reinterpret_cast<vec2*>(r + c) = q;
+        }
+    }
+}
+
+template <typename T, int C>
+__global__ __launch_bounds__(kThreads) void k_gather_records(PtrPack pk, T* __restrict__ tail, uint32_t n, uint32_t m,
+                                                             const uint32_t* __restrict__ perm,
+                                                             const uint32_t* __restrict__ far)
+{
+    if (!*far) return;
+    typedef T vec2 __attribute__((ext_vector_type(2)));
+    // four outputs a thread at a time, a block apart: stores are whole lines
+    for (int64_t i0 = (int64_t)blockIdx.x * (4 * kThreads) + threadIdx.x; i0 < n;
+         i0 += (int64_t)gridDim.x * (4 * kThreads)) {
+        vec2 v[4][C / 2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t i = i0 + q * kThreads;
+            if (i < n) {
+                const T* r = record_of<T, C>(pk, tail, perm[i], m);
+#pragma unroll
+                for (int c = 0; c < C / 2; ++c) v[q][c] = *reinterpret_cast<const vec2*>(r + 2 * c);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t i = i0 + q * kThreads;
+            if (i < n) {
+#pragma unroll
+                for (int c = 0; c < C / 2; ++c) {
+                    static_cast<T*>(const_cast<void*>(pk.src[2 * c]))[i] = v[q][c].x;
+                    static_cast<T*>(const_cast<void*>(pk.src[2 * c + 1]))[i] = v[q][c].y;
+                }
+            }
+        }
+    }
 }
 
 // ------------------------------------------------------------ compaction
@@ -1292,8 +1458,7 @@ static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 size_t psum_hip_sort_workspace(int64_t n)
 {
     if (n <= 0) return 256;
-    const int64_t nb = (n + kSortTile - 1) / kSortTile;
-    const int64_t nh = nb * 256;
+    const int64_t nh = (n + kSortSmallTile - 1) / kSortSmallTile << kSortMaxBits;
     return 2 * align256((size_t)n * 4) + align256((size_t)nh * 4) + scan_workspace(nh);
 }
 
@@ -1306,35 +1471,48 @@ psum_status psum_hip_sort(const uint32_t* keys, int64_t n, uint32_t nkeys, uint3
     PSUM_ARG_CHECK(work_bytes >= psum_hip_sort_workspace(n), "psum_hip_sort: workspace too small");
     PSUM_ARG_CHECK(nkeys >= 1 && nkeys < PSUM_KEY_INVALID, "psum_hip_sort: bad nkeys");
     hipStream_t st = S(stream);
-    const int nb = (int)((n + kSortTile - 1) / kSortTile);
+    const int W = sort_waves(n);
+    const int nb = (int)((n + (int64_t)W * kSortWaveTile - 1) / ((int64_t)W * kSortWaveTile));
     char* w = static_cast<char*>(work);
-    uint32_t* k1 = reinterpret_cast<uint32_t*>(w);
-    w += align256((size_t)n * 4);
-    uint32_t* v1 = reinterpret_cast<uint32_t*>(w);
-    w += align256((size_t)n * 4);
+    uint32_t* pairs = reinterpret_cast<uint32_t*>(w);     // n (key, index) pairs
+    w += 2 * align256((size_t)n * 4);
     uint32_t* gh = reinterpret_cast<uint32_t*>(w);
-    w += align256((size_t)nb * 256 * 4);
+    const int bits = 32 - __builtin_clz(nkeys);           // INVALID maps to nkeys
+    const int passes = (bits + kSortMaxBits - 1) / kSortMaxBits;
+    const int width = (bits + passes - 1) / passes;
+    w += align256(((size_t)nb << width) * 4);
     void* scan_work = w;
 
-    int bits = 32 - __builtin_clz(nkeys);   // INVALID maps to nkeys
-    const int passes = (bits + 7) / 8;
-    const uint32_t* kin = keys;
-    const uint32_t* vin = nullptr;
+    bool in_pairs = false;
     for (int p = 0; p < passes; ++p) {
-        // the last pass lands in (keys_out, perm)
-        const bool to_out = ((passes - 1 - p) % 2) == 0;
-        uint32_t* kout = to_out ? keys_out : k1;
-        uint32_t* vout = to_out ? perm : v1;
-        hipLaunchKernelGGL(k_sort_hist, dim3(nb), dim3(kThreads), 0, st, kin, n, nkeys, 8 * p, gh,
-                           nb);
-        PSUM_HIP_TRY(hipGetLastError());
-        psum_status s = exclusive_scan_u32(gh, gh, (int64_t)nb * 256, scan_work, st);
-        if (s != PSUM_OK) return s;
-        hipLaunchKernelGGL(k_sort_scatter, dim3(nb), dim3(kThreads), 0, st, kin, vin, n, nkeys,
-                           8 * p, gh, nb, kout, vout);
-        PSUM_HIP_TRY(hipGetLastError());
-        kin = kout;
-        vin = vout;
+        // the last pass lands in (keys_out, perm), the one before in the pairs
+        const bool to_pairs = ((passes - 1 - p) % 2) != 0;
+        const int shift = p * width;
+        const uint32_t* kin = p == 0 ? keys : (in_pairs ? pairs : keys_out);
+        const uint32_t* vin = p == 0 || in_pairs ? nullptr : perm;
+        const dim3 gr(nb), bl(64 * W);
+#define PSUM_SORT(WW)                                                                                                  \
+    do {                                                                                                               \
+        if (in_pairs) hipLaunchKernelGGL((k_sort_hist<WW, true>), gr, bl, 0, st, kin, n, nkeys, shift, width, gh, nb); \
+        else hipLaunchKernelGGL((k_sort_hist<WW, false>), gr, bl, 0, st, kin, n, nkeys, shift, width, gh, nb);         \
+        PSUM_HIP_TRY(hipGetLastError());                                                                               \
+        const psum_status s_ = exclusive_scan_u32(gh, gh, (int64_t)nb << width, scan_work, st);                        \
+        if (s_ != PSUM_OK) return s_;                                                                                  \
+        if (in_pairs)                                                                                                  \
+            hipLaunchKernelGGL((k_sort_scatter<WW, true, false>), gr, bl, 0, st, kin, vin, n, nkeys, shift, width, gh, \
+                               nb, keys_out, perm);                                                                    \
+        else if (to_pairs)                                                                                             \
+            hipLaunchKernelGGL((k_sort_scatter<WW, false, true>), gr, bl, 0, st, kin, vin, n, nkeys, shift, width, gh, \
+                               nb, pairs, nullptr);                                                                    \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_sort_scatter<WW, false, false>), gr, bl, 0, st, kin, vin, n, nkeys, shift, width,    \
+                               gh, nb, keys_out, perm);                                                                \
+        PSUM_HIP_TRY(hipGetLastError());                                                                               \
+    } while (0)
+        if (W == 8) PSUM_SORT(8);
+        else PSUM_SORT(4);
+#undef PSUM_SORT
+        in_pairs = to_pairs;
     }
     return PSUM_OK;
 }
@@ -1367,6 +1545,59 @@ psum_status psum_hip_permute(int dtype, int ncomp, void* const* src, void* const
     PSUM_HIP_TRY(hipGetLastError());
     return PSUM_OK;
 }
+
+}  // extern "C"
+
+namespace psum_hip {
+
+// Permutes src into dst like psum_hip_permute, or, where the permutation has
+// no order, back into src through records in dst and tail: *far says on the
+// device which (1: the result is in src).  At most kRecordBlocks blocks walk
+// the particles, so that the launches of the route not taken are short.
+static constexpr unsigned kRecordBlocks = 8192;
+template <typename T, int C>
+static psum_status permute_records(const PtrPack& pk, int64_t n, const uint32_t* perm, void* tail, uint32_t* far,
+                                   hipStream_t st)
+{
+    const uint32_t un = (uint32_t)n, m = un / (uint32_t)C;
+    hipLaunchKernelGGL(k_perm_far, dim3(1), dim3(1024), 0, st, perm, n, far);
+    hipLaunchKernelGGL((k_pack_records<T, C>), dim3(std::min(grid_blocks(n, kThreads), kRecordBlocks)), dim3(kThreads), 0,
+                       st, pk, static_cast<T*>(tail), un, m, far);
+    hipLaunchKernelGGL((k_gather_records<T, C>), dim3(std::min(grid_blocks(n, 4 * kThreads), kRecordBlocks)),
+                       dim3(kThreads), 0, st, pk, static_cast<T*>(tail), un, m, perm, far);
+    hipLaunchKernelGGL(k_permute4<T>, dim3(grid_blocks((n + 3) / 4, kThreads)), dim3(kThreads), 0, st, pk, C, perm, n,
+                       far);
+    PSUM_HIP_TRY(hipGetLastError());
+    return PSUM_OK;
+}
+
+bool permute_either_applies(int dtype, int ncomp, int64_t n)
+{
+    // below 16 MB the arrays stay in the caches and a line fetched for one
+    // value is still there for its others
+    const size_t esz = dtype == PSUM_F64 ? 8 : 4;
+    return (ncomp == 4 || ncomp == 6) && (size_t)n * ncomp * esz >= ((size_t)16 << 20);
+}
+
+psum_status permute_either(int dtype, int ncomp, void* const* src, void* const* dst, const uint32_t* perm, int64_t n,
+                           void* tail, uint32_t* far, void* stream)
+{
+    PtrPack pk{};
+    for (int c = 0; c < ncomp; ++c) {
+        pk.src[c] = src[c];
+        pk.dst[c] = dst[c];
+    }
+    hipStream_t st = S(stream);
+    if (dtype == PSUM_F64)
+        return ncomp == 4 ? permute_records<double, 4>(pk, n, perm, tail, far, st)
+                          : permute_records<double, 6>(pk, n, perm, tail, far, st);
+    return ncomp == 4 ? permute_records<float, 4>(pk, n, perm, tail, far, st)
+                      : permute_records<float, 6>(pk, n, perm, tail, far, st);
+}
+
+}  // namespace psum_hip
+
+extern "C" {
 
 size_t psum_hip_compact_workspace(int64_t n)
 {

@@ -312,7 +312,7 @@ public:
         S_TRY(hipMalloc(&perm_, (size_t)max_cap_ * 4 + 4));
         sort_bytes_ = psum_hip_sort_workspace(max_cap_);
         S_TRY(hipMalloc(&sort_work_, sort_bytes_));
-        S_TRY(hipMalloc(&nvalid_, sizeof(unsigned long long)));
+        S_TRY(hipMalloc(&nvalid_, 2 * sizeof(unsigned long long)));   // valid count, permute_either's flag
     }
 
     ~Stepper()
@@ -1362,26 +1362,39 @@ public:
             int nc = 0;
             for (int d = 0; d < D; ++d) { src[nc] = sp.pos[d]; dst[nc] = sp.pos2[d]; ++nc; }
             for (int d = 0; d < D; ++d) { src[nc] = sp.vel[d]; dst[nc] = sp.vel2[d]; ++nc; }
-            CHK(psum_hip_permute(cfg_.dtype, nc, src, dst, perm_, sp.n, st_));
-            if (stable_buffers_) {
-                // keep the arrays a captured graph points at
+            // a particle load may be in random order: the permutation then
+            // leaves its result in the source arrays (permute_either; the
+            // unsorted keys are free by now)
+            const bool either = permute_either_applies(cfg_.dtype, nc, sp.n);
+            if (either)
+                CHK(permute_either(cfg_.dtype, nc, src, dst, perm_, sp.n, keys_,
+                                   reinterpret_cast<uint32_t*>(nvalid_ + 1), st_));
+            else
+                CHK(psum_hip_permute(cfg_.dtype, nc, src, dst, perm_, sp.n, st_));
+            auto take_sorted = [&]() {
                 for (int d = 0; d < D; ++d) {
-                    S_TRY(hipMemcpyAsync(sp.pos[d], sp.pos2[d], (size_t)sp.n * esz_, hipMemcpyDeviceToDevice, st_));
-                    S_TRY(hipMemcpyAsync(sp.vel[d], sp.vel2[d], (size_t)sp.n * esz_, hipMemcpyDeviceToDevice, st_));
+                    if (stable_buffers_) {
+                        // keep the arrays a captured graph points at
+                        S_TRY(hipMemcpyAsync(sp.pos[d], sp.pos2[d], (size_t)sp.n * esz_, hipMemcpyDeviceToDevice, st_));
+                        S_TRY(hipMemcpyAsync(sp.vel[d], sp.vel2[d], (size_t)sp.n * esz_, hipMemcpyDeviceToDevice, st_));
+                    } else {
+                        std::swap(sp.pos[d], sp.pos2[d]);
+                        std::swap(sp.vel[d], sp.vel2[d]);
+                    }
                 }
-            } else {
-                for (int d = 0; d < D; ++d) {
-                    std::swap(sp.pos[d], sp.pos2[d]);
-                    std::swap(sp.vel[d], sp.vel2[d]);
-                }
-            }
+            };
+            if (!either) take_sorted();
             // drop particles whose key is invalid (absorbed): they sort last
-            unsigned long long nv = (unsigned long long)sp.n;
-            S_TRY(hipMemcpyAsync(nvalid_, &nv, sizeof nv, hipMemcpyHostToDevice, st_));
+            unsigned long long nv[2] = {(unsigned long long)sp.n, 0ull};
+            S_TRY(hipMemcpyAsync(nvalid_, nv, sizeof nv[0], hipMemcpyHostToDevice, st_));
             hipLaunchKernelGGL(k_count_valid, dim3(1), dim3(64), 0, st_, skeys_, sp.n, nvalid_);
-            S_TRY(hipMemcpyAsync(&nv, nvalid_, sizeof nv, hipMemcpyDeviceToHost, st_));
+            S_TRY(hipMemcpyAsync(nv, nvalid_, sizeof nv, hipMemcpyDeviceToHost, st_));
             S_TRY(hipStreamSynchronize(st_));
-            sp.n = (int64_t)nv;
+            if (either && (uint32_t)nv[1] == 0) {
+                take_sorted();
+                if (stable_buffers_) S_TRY(hipStreamSynchronize(st_));
+            }
+            sp.n = (int64_t)nv[0];
         }
     }
 };
