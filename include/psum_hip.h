@@ -144,6 +144,15 @@ psum_status psum_hip_gather_push(const psum_grid* g, int dtype, void* const* pos
                                  void* const* vel, int64_t n, const void* phi, double qm,
                                  double dt, double mass, double w_dep, double scale, int64_t* acc,
                                  double* diag, int64_t* counters, void* stream);
+/* psum_hip_gather_push with device workspace for particles in no order (their
+ * deposit then runs apart, summed per domain of the grid; the same result).
+ * psum_hip_gather_push_workspace: the bytes it takes, 0 where it would not
+ * be used (work may always be NULL).  No reference counterpart. */
+size_t psum_hip_gather_push_workspace(const psum_grid* g, int64_t n);
+psum_status psum_hip_gather_push_ws(const psum_grid* g, int dtype, void* const* pos, void* const* vel, int64_t n,
+                                    const void* phi, double qm, double dt, double mass, double w_dep, double scale,
+                                    int64_t* acc, double* diag, int64_t* counters, void* work, size_t work_bytes,
+                                    void* stream);
 
 /* Higher-order coupling (interp_B_spline / add_back_B_spline of
  * higher_order_interp.hpp:196-248, selected by TSI's interp_order,

@@ -175,6 +175,9 @@ SIGNATURES = [
     ("psum_hip_gather_push", ST, [_GP, C.c_int, P, P, I64, P, C.c_double, C.c_double, C.c_double,
                                   C.c_double, C.c_double, P, P, P, P]),
     ("psum_hip_deposit_bspline", ST, [_GP, C.c_int, C.c_int, P, I64, C.c_double, C.c_double, P, P, P]),
+    ("psum_hip_gather_push_workspace", C.c_size_t, [_GP, I64]),
+    ("psum_hip_gather_push_ws", ST, [_GP, C.c_int, P, P, I64, P, C.c_double, C.c_double, C.c_double,
+                                     C.c_double, C.c_double, P, P, P, P, C.c_size_t, P]),
     ("psum_hip_gather_push_bspline", ST, [_GP, C.c_int, C.c_int, P, P, I64, P, C.c_double, C.c_double,
                                           C.c_double, P, P, P]),
     ("psum_hip_mcc_workspace", C.c_size_t, [I64, C.c_int]),

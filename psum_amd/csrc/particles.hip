@@ -753,17 +753,21 @@ __device__ __forceinline__ bool push_one(const DevGrid& g, const T* __restrict__
 template <int D>
 constexpr int push_min_waves() { return D == 2 ? 5 : 1; }
 
-template <typename T, int D, bool PUSH, bool DEPOSIT, int UNIT = kGridAny>
+// DEFER (2D and 3D): a block most of whose particles lie outside its clipped
+// box deposits nothing and says so in defer[block]; k_deposit_domains takes
+// its particles.
+template <typename T, int D, bool PUSH, bool DEPOSIT, int UNIT = kGridAny, bool DEFER = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(push_min_waves<D>(), 8))) void k_push_deposit(
     DevGrid g, T* __restrict__ x0, T* __restrict__ x1, T* __restrict__ x2, T* __restrict__ v0,
     T* __restrict__ v1, T* __restrict__ v2, int64_t n, const T* __restrict__ phi, T qm, T dt,
     double mass, double w_dep, double scale, unsigned long long* __restrict__ acc,
-    double* __restrict__ diag, unsigned long long* __restrict__ counters)
+    double* __restrict__ diag, unsigned long long* __restrict__ counters, uint32_t* __restrict__ defer = nullptr)
 {
     __shared__ unsigned long long tile[DEPOSIT ? tile_nodes<D>() : 1];
     __shared__ int bmin[3], bmax[3], bref[3];
     __shared__ long long bsum[3];
     __shared__ int bcnt;
+    __shared__ int bin;          // DEFER: particles inside the clipped box
     __shared__ double wdiag[kThreads / 16][4];   // per 16-lane row
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // wraps of the global int64 sums; an LDS tile entry holds at most
@@ -774,6 +778,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(push_m
         bmax[threadIdx.x] = INT_MIN;
         bsum[threadIdx.x] = 0;
         if (threadIdx.x == 0) bcnt = 0;
+        if (DEFER && threadIdx.x == 0) bin = 0;
     }
     T* const xs[3] = {x0, x1, x2};
     T* const vs[3] = {v0, v1, v2};
@@ -970,7 +975,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(push_m
                 tsize *= c;
             }
         }
-        const bool use_lds = any;
+        bool use_lds = any;
+        if constexpr (DEFER) {
+            bool scattered = false;
+            if (clipped) {
+                int in = 0;
+#pragma unroll
+                for (int j = 0; j < kPPT; ++j)
+                    if (ok[j]) {
+                        bool inside = true;
+#pragma unroll
+                        for (int d = 0; d < D; ++d) inside = inside && uw[j][d] >= lo[d] && uw[j][d] + 1 < lo[d] + e[d];
+                        in += inside ? 1 : 0;
+                    }
+                in = wave_isum_full(in);
+                if (lane == 0) atomicAdd(&bin, in);
+                __syncthreads();
+                scattered = 2 * bin < bcnt;
+            }
+            if (threadIdx.x == 0) defer[blockIdx.x] = scattered ? 1u : 0u;
+            if (scattered) {           // the same in every thread
+                use_lds = false;
+#pragma unroll
+                for (int j = 0; j < kPPT; ++j) ok[j] = false;
+            }
+        }
         if (use_lds)
             for (int i = threadIdx.x; i < (int)tsize; i += kThreads) tile[i] = 0ull;
         __syncthreads();
@@ -1196,6 +1225,163 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(push_m
     }
 }
 
+// ---- deposit of unordered particles ----------------------------------------
+// Particles without order cost 2^D global int64 atomics each, which run at
+// the memory side (23 G/s measured, whatever the grid's size: 5M particles on
+// 512 x 384 nodes, 20M atomics, 860 us).  Here each block owns a domain of
+// consecutive cells (linear index) whose nodes, with the support of its last
+// cells, fit an LDS tile; it walks its share of the blocks that k_push_deposit
+// deferred, keeps the particles of its domain and adds their terms in LDS, so
+// every particle is read once per domain (8..24 bytes, mostly from cache)
+// and only tiles reach memory: push 68 us, domains 216 us.  A wave queues the particles it keeps
+// and works them off 64 at a time, all lanes busy.  Terms and cells are
+// k_push_deposit's and sums are integers: the same result.
+constexpr int kDomThreads = 1024;
+constexpr int kDomTile = 17408;            // nodes, 136 KB
+constexpr int kDomMax = 64;                // domains: each reads every particle
+constexpr int64_t kDomMinParticles = (int64_t)1 << 19;   // below, the atomics take less than ~100 us
+
+struct Domains {
+    uint32_t cells, count, up, splits;     // cells a domain, domains, nodes above, blocks per domain
+};
+
+template <typename T, int D>
+__global__ __launch_bounds__(kDomThreads) void k_deposit_domains(
+    DevGrid g, const T* __restrict__ x0, const T* __restrict__ x1, const T* __restrict__ x2, int64_t n,
+    const uint32_t* __restrict__ defer, uint32_t nchunks, Domains dm, uint32_t nn, double w_dep, double scale,
+    unsigned long long* __restrict__ acc, unsigned long long* __restrict__ counters)
+{
+    __shared__ unsigned long long tile[kDomTile];
+    __shared__ uint32_t queue[kDomThreads / 64][128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t dom = blockIdx.x % dm.count, part = blockIdx.x / dm.count;
+    int some = 0;
+    for (uint32_t c = part + threadIdx.x * dm.splits; c < nchunks; c += kDomThreads * dm.splits) some |= defer[c] != 0;
+    if (!__syncthreads_or(some)) return;
+    unsigned long long* const ovf = counters ? counters + 3 : nullptr;
+    const uint32_t lo = dom * dm.cells, hi = min(lo + dm.cells, nn);
+    const uint32_t ext = min(hi - lo + dm.up, nn - lo);
+    for (uint32_t i = threadIdx.x; i < ext; i += kDomThreads) tile[i] = 0ull;
+    __syncthreads();
+    const T* const xs[3] = {x0, x1, x2};
+    const double wsc = w_dep * scale;
+    const uint64_t lt = __lanemask_lt();
+    constexpr int NS = 1 << D, ROWS = kPushTile / kDomThreads;
+
+    auto add = [&](uint32_t p) {
+        T x[D], sd[D], W[D][2];
+        int cw[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) x[d] = xs[d][p];
+        if (!cell_of<T, D, kGridAny>(g, x, cw, sd)) return;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            W[d][0] = (T)1 - sd[d];
+            W[d][1] = sd[d];
+        }
+        uint32_t node[NS];
+        support_indices<D>(g, cw, node);
+        bool wr = false;
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const T c0 = cic_coef<T, D>(W, i);
+            const T cf = coef_kept<T>(c0) ? c0 : (T)0;
+            const unsigned long long t = (unsigned long long)round_to_ll((double)cf * wsc);
+            const uint32_t o = node[i] - lo;
+            if (ovf) {
+                // (a tile entry takes more terms than k_push_deposit's and may wrap)
+                if (t) wr |= add_wraps(o < ext ? atomicAdd(&tile[o], t) : atomicAdd(&acc[node[i]], t), t);
+            } else if (o < ext) {
+                atomicAdd(&tile[o], t);
+            } else if (t) {
+                atomicAdd(&acc[node[i]], t);
+            }
+        }
+        if (wr) atomicAdd(ovf, 1ull);
+    };
+
+    uint32_t qn = 0;                       // queued particles of the wave
+    T X[2][ROWS][D];
+    auto fetch = [&](uint32_t c, T (*v)[D]) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const int64_t p = (int64_t)c * kPushTile + r * kDomThreads + threadIdx.x;
+#pragma unroll
+            for (int d = 0; d < D; ++d) v[r][d] = p < n ? xs[d][p] : (T)NAN;
+        }
+    };
+    auto next = [&](uint32_t c) {          // the first deferred chunk from c on (uniform)
+        while (c < nchunks && !defer[c]) c += dm.splits;
+        return c;
+    };
+    auto work = [&](uint32_t c, T (*v)[D]) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            T sd[D];
+            int cw[D];
+            bool in = false;
+            if (isfinite((double)v[r][0]) && cell_of<T, D, kGridAny>(g, v[r], cw, sd)) {
+                uint32_t lc = (uint32_t)cw[0];
+#pragma unroll
+                for (int d = 1; d < D; ++d) lc = lc * (uint32_t)g.w[d] + (uint32_t)cw[d];
+                in = lc >= lo && lc < hi;
+            }
+            const uint64_t m = __ballot(in);
+            if (in) queue[wave][qn + (uint32_t)__popcll(m & lt)] = c * (uint32_t)kPushTile + r * kDomThreads + threadIdx.x;
+            qn += (uint32_t)__popcll(m);
+            if (qn >= 64) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                qn -= 64;
+                add(queue[wave][qn + lane]);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+        }
+    };
+    // the next chunk's positions are on their way while one is worked on
+    uint32_t c = next(part);
+    if (c < nchunks) fetch(c, X[0]);
+    while (c < nchunks) {
+        uint32_t c2 = next(c + dm.splits);
+        if (c2 < nchunks) fetch(c2, X[1]);
+        work(c, X[0]);
+        if (c2 >= nchunks) break;
+        c = next(c2 + dm.splits);
+        if (c < nchunks) fetch(c, X[0]);
+        work(c2, X[1]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if ((uint32_t)lane < qn) add(queue[wave][lane]);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < ext; i += kDomThreads) {
+        const unsigned long long t = tile[i];
+        if (t) acc_add(&acc[lo + i], t, ovf);
+    }
+}
+
+// the domains of a grid, or count 0 where they do not apply
+static Domains plan_domains(const psum_grid* g, int64_t n)
+{
+    Domains dm{0, 0, 0, 0};
+    const int64_t nn = grid_nodes(*g);
+    if (g->dim < 2 || n < kDomMinParticles || n >= (int64_t)0xFFFFFFFF - 2 * kPushTile) return dm;
+    // a cell's support reaches one node further along every axis
+    int64_t up = 0, stride = 1;
+    for (int d = g->dim - 1; d >= 0; --d) {
+        up += stride;
+        stride *= g->cells[d] + 1;
+    }
+    const int64_t room = kDomTile - up;
+    if (room < kDomTile / 4) return dm;
+    const int64_t count = (nn + room - 1) / room;
+    if (count > kDomMax) return dm;
+    dm.count = (uint32_t)count;
+    dm.cells = (uint32_t)((nn + count - 1) / count);
+    dm.up = (uint32_t)up;
+    // one block a compute unit (the tile fills its LDS), at least 16k particles each
+    dm.splits = (uint32_t)std::max<int64_t>(1, std::min<int64_t>(256 / count, n / 16384));
+    return dm;
+}
+
 // -------------------------------------------------------- small kernels
 
 __global__ __launch_bounds__(kThreads) void k_fixed_to_double(const long long* __restrict__ acc,
@@ -1303,7 +1489,7 @@ template <typename T>
 psum_status launch_push(const psum_grid* g, void* const* pos, void* const* vel, int64_t n,
                         const void* phi, double qm, double dt, double mass, double w_dep,
                         double scale, int64_t* acc, double* diag, int64_t* counters, bool push,
-                        hipStream_t st)
+                        hipStream_t st, uint32_t* defer = nullptr)
 {
     const DevGrid dg = to_dev(*g);
     const unsigned nb = grid_blocks(n, kPushTile);
@@ -1323,6 +1509,27 @@ psum_status launch_push(const psum_grid* g, void* const* pos, void* const* vel, 
     bool unit = true;
     for (int d = 0; d < g->dim; ++d) unit = unit && g->delta_r[d] == 1.0 && g->delta[d] == 1.0;
     const bool unit0 = unit && dg.origin0 && sizeof(T) == 4;
+    const Domains dm = defer && push && acc ? plan_domains(g, n) : Domains{0, 0, 0, 0};
+    if (dm.count) {
+#define PSUM_DEFER(DIM, UN)                                                                                      \
+    hipLaunchKernelGGL((k_push_deposit<T, DIM, true, true, UN, true>), dim3(nb), dim3(kThreads), 0, st, dg, p[0], \
+                       p[1], p[2], v[0], v[1], v[2], n, ph, (T)qm, (T)dt, mass, w_dep, scale, a, diag, c, defer)
+#define PSUM_DOMAINS(DIM)                                                                                          \
+    do {                                                                                                           \
+        if (unit0) PSUM_DEFER(DIM, kGridUnit0);                                                                    \
+        else if (unit) PSUM_DEFER(DIM, kGridUnit);                                                                 \
+        else PSUM_DEFER(DIM, kGridAny);                                                                            \
+        PSUM_HIP_TRY(hipGetLastError());                                                                           \
+        hipLaunchKernelGGL((k_deposit_domains<T, DIM>), dim3(dm.count * dm.splits), dim3(kDomThreads), 0, st, dg,  \
+                           p[0], p[1], p[2], n, defer, nb, dm, (uint32_t)grid_nodes(*g), w_dep, scale, a, c);      \
+    } while (0)
+        if (g->dim == 2) PSUM_DOMAINS(2);
+        else PSUM_DOMAINS(3);
+#undef PSUM_DOMAINS
+#undef PSUM_DEFER
+        PSUM_HIP_TRY(hipGetLastError());
+        return PSUM_OK;
+    }
 #define PSUM_LAUNCH(DIM, PU, DE, UN)                                                          \
     hipLaunchKernelGGL((k_push_deposit<T, DIM, PU, DE, UN>), dim3(nb), dim3(kThreads), 0, st, \
                        dg, p[0], p[1], p[2], v[0], v[1], v[2], n, ph, (T)qm, (T)dt, mass,      \
@@ -1750,17 +1957,35 @@ psum_status psum_hip_gather_push(const psum_grid* g, int dtype, void* const* pos
                                  double dt, double mass, double w_dep, double scale, int64_t* acc,
                                  double* diag, int64_t* counters, void* stream)
 {
+    return psum_hip_gather_push_ws(g, dtype, pos, vel, n, phi, qm, dt, mass, w_dep, scale, acc, diag, counters,
+                                   nullptr, 0, stream);
+}
+
+size_t psum_hip_gather_push_workspace(const psum_grid* g, int64_t n)
+{
+    if (!grid_ok(g) || n < 0 || !plan_domains(g, n).count) return 0;
+    return (size_t)psum_hip_push_blocks(n) * sizeof(uint32_t);
+}
+
+psum_status psum_hip_gather_push_ws(const psum_grid* g, int dtype, void* const* pos, void* const* vel, int64_t n,
+                                    const void* phi, double qm, double dt, double mass, double w_dep, double scale,
+                                    int64_t* acc, double* diag, int64_t* counters, void* work, size_t work_bytes,
+                                    void* stream)
+{
     PSUM_ARG_CHECK(grid_ok(g), "psum_hip_gather_push: invalid grid");
     PSUM_ARG_CHECK(n == 0 || (pos && vel && phi), "psum_hip_gather_push: null pointer");
     PSUM_ARG_CHECK(!acc || pow2(scale), "psum_hip_gather_push: scale must be a power of two");
     PSUM_ARG_CHECK(!acc || std::fabs(w_dep) * scale <= 0x1p50,
                    "psum_hip_gather_push: |w_dep| * scale must not exceed 2^50");
+    PSUM_ARG_CHECK(!work || work_bytes >= psum_hip_gather_push_workspace(g, n),
+                   "psum_hip_gather_push_ws: workspace too small");
+    uint32_t* defer = static_cast<uint32_t*>(work);
     if (dtype == PSUM_F64)
         return launch_push<double>(g, pos, vel, n, phi, qm, dt, mass, w_dep, scale, acc, diag,
-                                   counters, true, S(stream));
+                                   counters, true, S(stream), defer);
     if (dtype == PSUM_F32)
         return launch_push<float>(g, pos, vel, n, phi, qm, dt, mass, w_dep, scale, acc, diag,
-                                  counters, true, S(stream));
+                                  counters, true, S(stream), defer);
     set_error("psum_hip_gather_push: bad dtype");
     return PSUM_ERR_ARG;
 }

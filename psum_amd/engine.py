@@ -204,9 +204,12 @@ def gather_push(g, pos, vel, phi, qm, dt, mass=1.0, w_dep=None, scale=None, coun
         if scale is None:
             scale = float(np.ldexp(1.0, fx_shift(w_dep)))
         acc = torch.zeros(num_nodes(g), dtype=torch.int64, device=dev)
-    check(lib().psum_hip_gather_push(C.byref(g), _dtype_code(pos[0]), _ptrs(pos), _ptrs(vel), n,
-                                     _p(phi), qm, dt, mass, w_dep or 0.0, scale or 1.0, _p(acc),
-                                     _p(diag), _p(counters), _stream()), "psum_hip_gather_push")
+    # one word per block where unordered particles would be deposited apart
+    wb = lib().psum_hip_gather_push_workspace(C.byref(g), n) if acc is not None else 0
+    work = torch.empty(wb, dtype=torch.uint8, device=dev) if wb else None
+    check(lib().psum_hip_gather_push_ws(C.byref(g), _dtype_code(pos[0]), _ptrs(pos), _ptrs(vel), n,
+                                        _p(phi), qm, dt, mass, w_dep or 0.0, scale or 1.0, _p(acc),
+                                        _p(diag), _p(counters), _p(work), wb, _stream()), "psum_hip_gather_push")
     out = torch.zeros(4, dtype=torch.float64, device=dev)
     if nb > 0:
         work = torch.empty(lib().psum_hip_reduce_workspace() // 8, dtype=torch.float64, device=dev)
