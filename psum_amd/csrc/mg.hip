@@ -1579,9 +1579,13 @@ __global__ __launch_bounds__(kMgThreads) void k_outer_line(LineGeom G, LineList 
     if (A.e0) st_line(A.e0 + i, e);
 }
 
+// (x non-null: also shift = x_pin - bn_pin, the gauge of a pinned system)
 __global__ __launch_bounds__(kMgThreads) void k_reduce2(const double* __restrict__ part, int64_t nb,
-                                                        double* __restrict__ out)
+                                                        double* __restrict__ out, const double* __restrict__ x,
+                                                        const double* __restrict__ bn, int64_t pin,
+                                                        double* __restrict__ shift)
 {
+    if (x && threadIdx.x == 2) shift[0] = x[pin] - bn[pin];
     __shared__ double sh[2][kMgThreads];
     double s0 = 0.0, s1 = 0.0;
     // thread t sums pairs 8t .. 8t+7, then 8(t + 256) .., in order; the eight
@@ -1630,8 +1634,8 @@ __global__ __launch_bounds__(kMgThreads) void k_psum(const double* __restrict__ 
     }
 }
 
-__global__ __launch_bounds__(kMgThreads) void k_fsum(const double* __restrict__ part, int64_t nb,
-                                                     double* __restrict__ out)
+// the total of the block sums, in every thread of the block
+__device__ __forceinline__ double block_fsum(const double* __restrict__ part, int64_t nb)
 {
     __shared__ double sh[kMgThreads];
     double s = 0.0;
@@ -1642,7 +1646,79 @@ __global__ __launch_bounds__(kMgThreads) void k_fsum(const double* __restrict__ 
         if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[0] = sh[0];
+    return sh[0];
+}
+
+__global__ __launch_bounds__(kMgThreads) void k_fsum(const double* __restrict__ part, int64_t nb,
+                                                     double* __restrict__ out)
+{
+    const double s = block_fsum(part, nb);
+    if (threadIdx.x == 0) out[0] = s;
+}
+
+// The right-hand side of a pinned system in two launches: between the solves
+// of small problems every launch costs its 5 us, and the eight that subtract
+// the mean, replace, copy, sum (twice), set the pin and scale took a tenth of
+// a 128^2 step.  k_pin_rhs: b (less the mean whose block sums are mean_part),
+// replaced nodes set, copied to bp and, scaled by dinv, to b0 (FP64 cycles;
+// null in the mixed solve), summed per block.  Every block adds the mean's
+// sums itself, so there are at most kPinBlocks.  k_pin_set: the total, and the
+// pin's entries.  Operations and orders are those of the single kernels.
+constexpr unsigned kPinBlocks = 512;
+constexpr int kPinReplace = 4;
+struct PinArgs {
+    double* b;
+    int64_t n;
+    const double* mean_part;
+    const unsigned long long* idx;
+    const double* val;
+    int nrep, zero;
+    double *bp, *part, *b0;
+    const double* dinv;
+    const uint16_t* cls;
+    int64_t pin;
+    double* sum;
+};
+
+__global__ __launch_bounds__(kMgThreads) void k_pin_rhs(PinArgs a)
+{
+    __shared__ double ws[kMgThreads / 64];
+    const int64_t i = (int64_t)blockIdx.x * kMgThreads + threadIdx.x;
+    double v = 0.0, dinv = 0.0;
+    if (i < a.n) {
+        v = a.b[i];
+        if (a.b0) dinv = a.dinv[a.cls[i]];
+    }
+    if (a.mean_part) {
+        const double mean = block_fsum(a.mean_part, gridDim.x) / (double)a.n;
+        if (i < a.n) v = v - mean;
+    }
+    if (i < a.n) {
+        for (int r = 0; r < a.nrep; ++r)
+            if ((int64_t)a.idx[r] == i) v = a.zero ? 0.0 : a.val[r];
+        a.b[i] = v;
+        a.bp[i] = v;
+        if (a.b0) a.b0[i] = v * dinv;
+    }
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int w = 0; w < kMgThreads / 64; ++w) s += ws[w];
+        a.part[blockIdx.x] = s;
+    }
+}
+
+__global__ __launch_bounds__(kMgThreads) void k_pin_set(PinArgs a, int64_t nb)
+{
+    const double s = block_fsum(a.part, nb);
+    if (threadIdx.x == 0) {
+        const double v = a.b[a.pin] - s;
+        a.sum[0] = s;
+        a.bp[a.pin] = v;
+        if (a.b0) a.b0[a.pin] = v * a.dinv[a.cls[a.pin]];
+    }
 }
 
 // b'_p = b_p - sum(b): the consistent right-hand side of the singular system
@@ -2406,10 +2482,27 @@ public:
     // The three parts of solve(): begin (addback, replace, the consistent
     // right-hand side of a pinned periodic system; returns the right-hand
     // side the V-cycles see), core (the cycles) and end (gauge, sync).
-    const double* solve_begin(double* b, bool homogeneous = false)
+    //
+    // mean_part: b still holds the charge whose block sums (kMgThreads nodes
+    // each) these are; its mean is taken off first (takes_mean() only).
+    bool takes_mean() const
+    {
+        return pin_ >= 0 && nblk(N0()) <= kPinBlocks && add_n_ == 0 && rep_n_ <= kPinReplace;
+    }
+    const double* solve_begin(double* b, bool homogeneous = false, const double* mean_part = nullptr)
     {
         if (host_.empty()) throw std::runtime_error("hip_multigrid: solve before set_matrix");
         hipStream_t st = stream_;
+        scaled_ = false;
+        if (takes_mean()) {
+            const PinArgs a{b, N0(), mean_part, rep_idx_, rep_val_, (int)rep_n_, homogeneous ? 1 : 0, bprime_, part_,
+                            mixed_ ? nullptr : dev_[0].b, table<double>(0, false).dinv, dl(0).cls, pin_, shift_};
+            hipLaunchKernelGGL(k_pin_rhs, dim3(nblk(N0())), dim3(kMgThreads), 0, st, a);
+            hipLaunchKernelGGL(k_pin_set, dim3(1), dim3(kMgThreads), 0, st, a, (int64_t)nblk(N0()));
+            MG_HIP(hipGetLastError());
+            scaled_ = !mixed_;
+            return bprime_;
+        }
         if (add_n_ && !homogeneous) hipLaunchKernelGGL(k_addback, dim3(nblk(add_n_)), dim3(kMgThreads), 0, st, b, add_idx_, add_val_, add_n_);
         if (rep_n_) hipLaunchKernelGGL(k_replace, dim3(nblk(rep_n_)), dim3(kMgThreads), 0, st, b, rep_idx_, rep_val_, rep_n_, homogeneous ? 1 : 0);
         MG_HIP(hipGetLastError());
@@ -2439,7 +2532,7 @@ public:
         const int first_check = std::max(1, std::min(max_cycles_, predicted_ - 1));
         if (!mixed_) {
             rec_phase(0, kStageOuter, 0);
-            scale_rhs_f64(bs);
+            if (!scaled_ || rec_) scale_rhs_f64(bs);
             if (!use_tol) {
                 vcycles_f64(x, max_cycles_);
                 last_cycles_ = max_cycles_;
@@ -2505,12 +2598,22 @@ public:
     void solve_end(const double* b, double* x, bool sync)
     {
         hipStream_t st = stream_;
-        if (pin_ >= 0) {
-            hipLaunchKernelGGL(k_gauge_read, dim3(1), dim3(64), 0, st, x, b, pin_, shift_ + 1);
-            hipLaunchKernelGGL(k_gauge_apply, dim3(nblk(N0())), dim3(kMgThreads), 0, st, x, N0(), shift_ + 1);
+        if (const double* shift = gauge(b, x)) {
+            hipLaunchKernelGGL(k_gauge_apply, dim3(nblk(N0())), dim3(kMgThreads), 0, st, x, N0(), shift);
             MG_HIP(hipGetLastError());
         }
         if (sync) MG_HIP(hipStreamSynchronize(st));
+    }
+    // the device value to take off x after the cycles, or null
+    const double* gauge(const double* b, const double* x)
+    {
+        if (pin_ < 0) return nullptr;
+        // (with a tolerance, the last check has left it)
+        if (!(tol_ > 0.0)) {
+            hipLaunchKernelGGL(k_gauge_read, dim3(1), dim3(64), 0, stream_, x, b, pin_, shift_ + 1);
+            MG_HIP(hipGetLastError());
+        }
+        return shift_ + 1;
     }
 
     // ---- batched fixed-cycle solves --------------------------------------
@@ -2674,6 +2777,7 @@ private:
     int periodic_mode_ = 1;
     int64_t pin_ = -1;                 // pinned node of a pinned-periodic matrix
     double* bprime_ = nullptr;         // consistent singular right-hand side
+    bool scaled_ = false;              // dev_[0].b holds the scaled right-hand side
     double* shift_ = nullptr;          // device scalar for the gauge shift / sums
     hipStream_t stream_ = nullptr;
     std::vector<HostLevel> host_;
@@ -3501,7 +3605,8 @@ private:
 #undef OUTER
         MG_HIP(hipGetLastError());
         if (!norms) return;
-        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kMgThreads), 0, stream_, part_, (int64_t)nb, red_);
+        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kMgThreads), 0, stream_, part_, (int64_t)nb, red_,
+                           pin_ >= 0 ? x : nullptr, bn, pin_, shift_ + 1);
         MG_HIP(hipGetLastError());
         MG_HIP(hipMemcpyAsync(red_host_, red_, 2 * sizeof(double), hipMemcpyDeviceToHost, stream_));
         if (wait) read_norms(rr, bb);
@@ -3785,9 +3890,13 @@ void mg_set_fixed_cycles(HipMultigrid* h, int cycles) { h->set_fixed_cycles(cycl
 void mg_set_predicted(HipMultigrid* h, int p) { h->set_predicted(p); }
 int mg_last_cycles(HipMultigrid* h) { return h->last_cycles(); }
 double mg_last_rel(HipMultigrid* h) { return h->last_rel(); }
-const double* mg_solve_begin(HipMultigrid* h, double* b) { return h->solve_begin(b); }
+const double* mg_solve_begin(HipMultigrid* h, double* b, const double* mean_part)
+{
+    return h->solve_begin(b, false, mean_part);
+}
+bool mg_takes_mean(HipMultigrid* h) { return h->takes_mean(); }
 void mg_solve_core(HipMultigrid* h, const double* b, const double* bs, double* x) { h->solve_core(b, bs, x); }
-void mg_solve_end(HipMultigrid* h, const double* b, double* x) { h->solve_end(b, x, false); }
+const double* mg_gauge(HipMultigrid* h, const double* b, const double* x) { return h->gauge(b, x); }
 bool mg_recordable(HipMultigrid* h) { return h->recordable(); }
 const double* mg_core_rhs(HipMultigrid* h, double* b)
 {

@@ -26,10 +26,13 @@ struct MgRecOp {
 struct MgBatchPlan;
 
 // solve() in parts: begin (replace, pin; returns the cycles' right-hand
-// side), core (the cycles), end (gauge; no sync)
-const double* mg_solve_begin(HipMultigrid* h, double* b);
+// side), core (the cycles), gauge (the device value to take off x, or null).
+// mean_part (only if mg_takes_mean()): the sums of b over blocks of 256 nodes,
+// whose mean is taken off b first.
+bool mg_takes_mean(HipMultigrid* h);
+const double* mg_solve_begin(HipMultigrid* h, double* b, const double* mean_part = nullptr);
 void mg_solve_core(HipMultigrid* h, const double* b, const double* bs, double* x);
-void mg_solve_end(HipMultigrid* h, const double* b, double* x);
+const double* mg_gauge(HipMultigrid* h, const double* b, const double* x);
 // whether the core can be recorded (2D fused hierarchy, fixed cycle count),
 // the right-hand side the core reads, and its ops
 bool mg_recordable(HipMultigrid* h);

@@ -1404,7 +1404,8 @@ __global__ __launch_bounds__(kThreads) void k_f64_to_f32(const double* __restric
 // contiguous chunk [b*chunk, (b+1)*chunk) (lane-strided, then a tree), pass 2
 // sums the per-chunk results the same way in one block.
 __global__ __launch_bounds__(kThreads) void k_reduce4(const double* __restrict__ part, int64_t nb,
-                                                      int64_t chunk, double* __restrict__ out)
+                                                      int64_t chunk, double* __restrict__ out, double f = 0.0,
+                                                      double vol = 0.0)
 {
     __shared__ double sh[4][kThreads];
     double s[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1422,7 +1423,12 @@ __global__ __launch_bounds__(kThreads) void k_reduce4(const double* __restrict__
             for (int q = 0; q < 4; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x < 4) out[(int64_t)blockIdx.x * 4 + threadIdx.x] = sh[threadIdx.x][0];
+    if (threadIdx.x < 4) {
+        double v = sh[threadIdx.x][0];
+        // (f * v) * vol of the first sum, the order of orc_field_energy
+        if (f != 0.0 && threadIdx.x == 0) v = (f * v) * vol;
+        out[(int64_t)blockIdx.x * 4 + threadIdx.x] = v;
+    }
 }
 
 // Field energy partials: one value per block (written to part[b*4]).
@@ -1475,12 +1481,6 @@ __global__ __launch_bounds__(kThreads) void k_field_energy(DevGrid g, const doub
         part[blockIdx.x * 4 + 2] = 0.0;
         part[blockIdx.x * 4 + 3] = 0.0;
     }
-}
-
-// v[0] = (f * v[0]) * vol, the order of orc_field_energy
-__global__ void k_scale_first(double* v, double f, double vol)
-{
-    if (threadIdx.x == 0) v[0] = (f * v[0]) * vol;
 }
 
 // ------------------------------------------------------ launch helpers
@@ -1992,16 +1992,17 @@ psum_status psum_hip_gather_push_ws(const psum_grid* g, int dtype, void* const* 
 
 size_t psum_hip_reduce_workspace(void) { return (size_t)kReduceBlocks * 4 * sizeof(double); }
 
+// f != 0: the first sum as (f * sum) * vol
 static psum_status reduce4(const double* part, int64_t nb, double* out, double* work,
-                           hipStream_t st)
+                           hipStream_t st, double f = 0.0, double vol = 0.0)
 {
     if (nb <= 4 * kThreads) {
-        hipLaunchKernelGGL(k_reduce4, dim3(1), dim3(kThreads), 0, st, part, nb, nb, out);
+        hipLaunchKernelGGL(k_reduce4, dim3(1), dim3(kThreads), 0, st, part, nb, nb, out, f, vol);
     } else {
         const int64_t chunk = (nb + kReduceBlocks - 1) / kReduceBlocks;
         const int64_t nr = (nb + chunk - 1) / chunk;
-        hipLaunchKernelGGL(k_reduce4, dim3((unsigned)nr), dim3(kThreads), 0, st, part, nb, chunk, work);
-        hipLaunchKernelGGL(k_reduce4, dim3(1), dim3(kThreads), 0, st, work, nr, nr, out);
+        hipLaunchKernelGGL(k_reduce4, dim3((unsigned)nr), dim3(kThreads), 0, st, part, nb, chunk, work, 0.0, 0.0);
+        hipLaunchKernelGGL(k_reduce4, dim3(1), dim3(kThreads), 0, st, work, nr, nr, out, f, vol);
     }
     PSUM_HIP_TRY(hipGetLastError());
     return PSUM_OK;
@@ -2040,13 +2041,10 @@ psum_status psum_hip_field_energy(const psum_grid* g, const double* phi, double 
     else
         hipLaunchKernelGGL(k_field_energy<3>, dim3(nb), dim3(kThreads), 0, st, dg, phi, nn, part);
     PSUM_HIP_TRY(hipGetLastError());
-    psum_status rs = reduce4(part, nb, out, part + nb * 4, st);
-    if (rs != PSUM_OK) return rs;
     double vol = 1.0;
     for (int d = 0; d < g->dim; ++d) vol *= g->delta[d];
-    hipLaunchKernelGGL(k_scale_first, dim3(1), dim3(64), 0, st, out, 0.5 * eps, vol);
-    PSUM_HIP_TRY(hipGetLastError());
-    return PSUM_OK;
+    if (eps == 0.0) vol = 0.0;   // (0 * sum: the reduction's f of 0 means no scaling)
+    return reduce4(part, nb, out, part + nb * 4, st, eps == 0.0 ? 1.0 : 0.5 * eps, vol);
 }
 
 psum_status psum_hip_f64_to_f32(const double* in, float* out, int64_t n, void* stream)

@@ -97,6 +97,47 @@ __global__ __launch_bounds__(kT) void k_sum_part(const double* __restrict__ x, i
     }
 }
 
+// rho from the integer deposit (psum_hip_fixed_to_double's arithmetic) and its
+// block sums (k_sum_part's)
+__global__ __launch_bounds__(kT) void k_rho_part(const long long* __restrict__ acc, int64_t n, double inv_scale,
+                                                 double offset, double* __restrict__ out,
+                                                 double* __restrict__ part)
+{
+    __shared__ double ws[kT / 64];
+    const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+    double v = 0.0;
+    if (i < n) {
+        v = (double)acc[i] * inv_scale + offset;
+        out[i] = v;
+    }
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int w = 0; w < kT / 64; ++w) s += ws[w];
+        part[blockIdx.x] = s;
+    }
+}
+
+// the end of a solve in one launch: phi less its gauge, its FP32 copy, and
+// the deposit cleared for the push (each where its pointer is given)
+__global__ __launch_bounds__(kT) void k_finish(double* __restrict__ phi, int64_t n, const double* __restrict__ shift,
+                                               float* __restrict__ phi32, long long* __restrict__ acc)
+{
+    const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
+    if (i >= n) return;
+    if (shift || phi32) {
+        double v = phi[i];
+        if (shift) {
+            v = v - shift[0];
+            phi[i] = v;
+        }
+        if (phi32) phi32[i] = (float)v;
+    }
+    if (acc) acc[i] = 0;
+}
+
 __global__ __launch_bounds__(kT) void k_sum_final(const double* __restrict__ part, int64_t nb,
                                                   double* __restrict__ out)
 {
@@ -418,18 +459,18 @@ public:
     // go to the device-side row counter.
     void step_body(bool diagnostics)
     {
-        solve_field();
+        solve_field(true);
         step_after_solve(diagnostics);
     }
 
-    // the rest of a step once phi is solved: field energy, gather + push +
-    // deposit of every species, diagnostics
+    // the rest of a step once phi is solved and the deposit cleared
+    // (solve_field_end(true)): field energy, gather + push + deposit of every
+    // species, diagnostics
     void step_after_solve(bool diagnostics)
     {
         {
             if (diagnostics) CHK(psum_hip_field_energy(&cfg_.grid, phi_, cfg_.eps, fe_, few_, few_bytes_, st_));
             const void* ph = cfg_.dtype == PSUM_F32 ? (const void*)phi32_ : (const void*)phi_;
-            hipLaunchKernelGGL(k_zero_i64, dim3(nblk(nn_)), dim3(kT), 0, st_, (long long*)acc_, nn_);
             for (int q = 0; q < cfg_.nspecies; ++q) {
                 Species& sp = sp_[q];
                 const double qm = sp.sp.q / sp.sp.m;
@@ -488,11 +529,13 @@ public:
 
     // rho from the exact deposit of the current positions, neutralised,
     // then phi by the multigrid (warm start); phi32 refreshed in FP32 mode
-    void solve_field()
+    // stepping: the push follows and deposits anew (the current deposit is
+    // cleared)
+    void solve_field(bool stepping = false)
     {
         const double* bs = solve_field_begin();
         mg_solve_core(mg_, b_, bs, phi_);
-        solve_field_end();
+        solve_field_end(stepping);
     }
 
     // solve_field in three parts, so that a batch can run the solver cores of
@@ -502,20 +545,30 @@ public:
     const double* solve_field_begin()
     {
         if (!acc_valid_) deposit_all();
-        CHK(psum_hip_fixed_to_double(acc_, nn_, 1.0 / scale_, cfg_.rho_bg, b_, st_));
-        if (all_periodic_) {
+        const bool mean_in_mg = all_periodic_ && mg_takes_mean(mg_);
+        if (mean_in_mg)
+            hipLaunchKernelGGL(k_rho_part, dim3(nblk(nn_)), dim3(kT), 0, st_, (const long long*)acc_, nn_, 1.0 / scale_,
+                               cfg_.rho_bg, b_, sum_part_);
+        else
+            CHK(psum_hip_fixed_to_double(acc_, nn_, 1.0 / scale_, cfg_.rho_bg, b_, st_));
+        if (all_periodic_ && !mean_in_mg) {
             hipLaunchKernelGGL(k_sum_part, dim3(nblk(nn_)), dim3(kT), 0, st_, b_, nn_, sum_part_);
             hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kT), 0, st_, sum_part_, (int64_t)nblk(nn_), sum_);
             hipLaunchKernelGGL(k_sub_mean, dim3(nblk(nn_)), dim3(kT), 0, st_, b_, nn_, sum_);
         }
         if (cfg_.extrapolate && have_prev_)
             hipLaunchKernelGGL(k_extrapolate, dim3(nblk(nn_)), dim3(kT), 0, st_, phi_, phi_prev_, nn_);
-        return mg_solve_begin(mg_, b_);
+        return mg_solve_begin(mg_, b_, mean_in_mg ? sum_part_ : nullptr);
     }
 
-    void solve_field_end()
+    void solve_field_end(bool stepping)
     {
-        mg_solve_end(mg_, b_, phi_);
+        const double* shift = mg_gauge(mg_, b_, phi_);
+        float* p32 = cfg_.dtype == PSUM_F32 ? phi32_ : nullptr;
+        if (shift || p32 || stepping)
+            hipLaunchKernelGGL(k_finish, dim3(nblk(nn_)), dim3(kT), 0, st_, phi_, nn_, shift, p32,
+                               stepping ? (long long*)acc_ : nullptr);
+        S_TRY(hipGetLastError());
         if (cfg_.extrapolate && !have_prev_) {
             S_TRY(hipMemcpyAsync(phi_prev_, phi_, nn_ * sizeof(double), hipMemcpyDeviceToDevice, st_));
             have_prev_ = true;
@@ -523,7 +576,6 @@ public:
         cycles_ += mg_last_cycles(mg_);
         max_cyc_seen_ = std::max(max_cyc_seen_, mg_last_cycles(mg_));
         last_rel_ = mg_last_rel(mg_);
-        if (cfg_.dtype == PSUM_F32) CHK(psum_hip_f64_to_f32(phi_, phi32_, nn_, st_));
     }
 
     // batch hooks: whether the solve's core can be recorded, and its ops
@@ -1685,7 +1737,7 @@ private:
         for (size_t i = 0; i < inst_.size(); ++i) {
             Stepper& st = *inst_[i];
             S_TRY(hipStreamWaitEvent(st.stream(), fork2_, 0));
-            st.solve_field_end();
+            st.solve_field_end(true);
             st.step_after_solve(true);
             S_TRY(hipEventRecord(join2_[i], st.stream()));
             S_TRY(hipStreamWaitEvent(ls, join2_[i], 0));
