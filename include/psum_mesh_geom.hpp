@@ -245,23 +245,13 @@ __device__ inline int64_t fast_cell(const View& m, const double* g)
     return ((int64_t)f[0] * m.J + (int64_t)f[1]) * m.K + (int64_t)f[2];
 }
 
-// triangle_mesh_trigger_acc::detect (:54-101): the first cell along the
-// segment with a hit (restrict mode) or the end cells only (fast mode)
-__device__ inline bool detect(const View& m, const double* p1, const double* p2, double& k, double* nrm,
-                              int32_t& id)
+// the traversal's end points in grid coordinates; false when the distance
+// field rules a hit out
+__device__ inline bool traverse_from(const View& m, const double* p1, const double* p2, double* g1, double* g2)
 {
-    double g1[3], g2[3];
     for (int c = 0; c < 3; ++c) {
         g1[c] = (p1[c] - m.box[c]) * m.rd[c];
         g2[c] = (p2[c] - m.box[c]) * m.rd[c];
-    }
-    if (m.fast) {
-        const bool in1 = g1[0] >= 0 && g1[0] < m.I && g1[1] >= 0 && g1[1] < m.J && g1[2] >= 0 && g1[2] < m.K;
-        const bool in2 = g2[0] >= 0 && g2[0] < m.I && g2[1] >= 0 && g2[1] < m.J && g2[2] >= 0 && g2[2] < m.K;
-        const int64_t c1 = fast_cell(m, g1), c2 = fast_cell(m, g2);
-        if (in1 && detect_cell(m, (int)c1, p1, p2, k, nrm, id)) return true;
-        if (in2 && c1 != c2) return detect_cell(m, (int)c2, p1, p2, k, nrm, id);
-        return false;
     }
     if (m.udf) {
         // distance-field skip (:66-92): from a start cell whose field
@@ -286,11 +276,33 @@ __device__ inline bool detect(const View& m, const double* p1, const double* p2,
             }
         }
     }
-    Trace s;
-    const int first = s.begin(m.I, m.J, m.K, g1, g2);
-    if (first < 0) return false;
-    for (int idx = first; !s.finished; idx = s.next())
-        if (detect_cell(m, idx, p1, p2, k, nrm, id)) return true;
+    return true;
+}
+
+// triangle_mesh_trigger_acc::detect (:54-101): the first cell along the
+// segment with a hit (restrict mode) or the end cells only (fast mode)
+__device__ inline bool detect(const View& m, const double* p1, const double* p2, double& k, double* nrm,
+                              int32_t& id)
+{
+    double g1[3], g2[3];
+    if (!m.fast) {
+        if (!traverse_from(m, p1, p2, g1, g2)) return false;
+        Trace s;
+        const int first = s.begin(m.I, m.J, m.K, g1, g2);
+        if (first < 0) return false;
+        for (int idx = first; !s.finished; idx = s.next())
+            if (detect_cell(m, idx, p1, p2, k, nrm, id)) return true;
+        return false;
+    }
+    for (int c = 0; c < 3; ++c) {
+        g1[c] = (p1[c] - m.box[c]) * m.rd[c];
+        g2[c] = (p2[c] - m.box[c]) * m.rd[c];
+    }
+    const bool in1 = g1[0] >= 0 && g1[0] < m.I && g1[1] >= 0 && g1[1] < m.J && g1[2] >= 0 && g1[2] < m.K;
+    const bool in2 = g2[0] >= 0 && g2[0] < m.I && g2[1] >= 0 && g2[1] < m.J && g2[2] >= 0 && g2[2] < m.K;
+    const int64_t c1 = fast_cell(m, g1), c2 = fast_cell(m, g2);
+    if (in1 && detect_cell(m, (int)c1, p1, p2, k, nrm, id)) return true;
+    if (in2 && c1 != c2) return detect_cell(m, (int)c2, p1, p2, k, nrm, id);
     return false;
 }
 
