@@ -26,6 +26,7 @@
 #include <array>
 #include <type_traits>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -1579,9 +1580,21 @@ __global__ __launch_bounds__(kMgThreads) void k_outer_line(LineGeom G, LineList 
     if (A.e0) st_line(A.e0 + i, e);
 }
 
+// Squared norms of a residual and its right-hand side in pinned host memory.
+// The kernel that sums them stores them there and then, at system scope, the
+// number of norms stored so far (kept in *count on the device), which the host
+// waits for: a copy and a stream synchronisation after it left the GPU idle
+// for 25 us per check of a small problem.
+struct NormBox {
+    double rr, bb;
+    unsigned long long seq;
+};
+
 // (x non-null: also shift = x_pin - bn_pin, the gauge of a pinned system)
 __global__ __launch_bounds__(kMgThreads) void k_reduce2(const double* __restrict__ part, int64_t nb,
-                                                        double* __restrict__ out, const double* __restrict__ x,
+                                                        NormBox* __restrict__ box,
+                                                        unsigned long long* __restrict__ count,
+                                                        const double* __restrict__ x,
                                                         const double* __restrict__ bn, int64_t pin,
                                                         double* __restrict__ shift)
 {
@@ -1615,7 +1628,14 @@ __global__ __launch_bounds__(kMgThreads) void k_reduce2(const double* __restrict
         }
         __syncthreads();
     }
-    if (threadIdx.x < 2) out[threadIdx.x] = sh[threadIdx.x][0];
+    if (threadIdx.x == 0) {
+        const unsigned long long c = *count + 1;
+        *count = c;
+        box->rr = sh[0][0];
+        box->bb = sh[1][0];
+        __threadfence_system();
+        __hip_atomic_store(&box->seq, c, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // per-block sums of x (part[b]), then a fixed-order single-block total
@@ -2553,7 +2573,7 @@ public:
             double rr, bb;
             const bool fm = fused_mixed();
             rec_phase(0, kStageOuter, 0);
-            outer_residual(bs, b, x, true, fm, false, false, &rr, &bb);
+            outer_residual(bs, b, x, true, fm, false);
             int cycle = 0;
             if (use_tol) {
                 // the iterations before the first whose norms are read
@@ -2583,11 +2603,14 @@ public:
                 last_cycles_ += batch;
                 if (cycle < max_cycles_) {
                     rec_phase(rec_iter_ - 1, kStageOuter, 0);
-                    outer_residual(bs, b, x, true, fm, false, false, &rr, &bb);
+                    outer_residual(bs, b, x, true, fm, false);
                 }
             }
             if (use_tol) {
-                if (last_cycles_ == 0) outer_residual(bs, b, x, false, false, true, false, &rr, &bb);
+                if (last_cycles_ == 0) {
+                    outer_residual(bs, b, x, false, false, true);
+                    ++norm_seq_;
+                }
                 read_norms(&rr, &bb);
                 last_rel_ = bb > 0 ? std::sqrt(rr / bb) : 0.0;
             }
@@ -2786,8 +2809,9 @@ private:
     std::vector<DevLevelBuf> dev_;
     std::vector<DevTransferBuf> dtr_;
     double* part_ = nullptr;
-    double* red_ = nullptr;
-    double* red_host_ = nullptr;
+    unsigned long long* norm_count_ = nullptr;   // norms stored, on the device
+    NormBox* norms_ = nullptr;                   // pinned host memory
+    unsigned long long norm_seq_ = 0;            // norms asked for
     unsigned long long *rep_idx_ = nullptr, *add_idx_ = nullptr;
     double *rep_val_ = nullptr, *add_val_ = nullptr;
     int64_t rep_n_ = 0, add_n_ = 0, rep_cap_ = 0, add_cap_ = 0;
@@ -2835,15 +2859,16 @@ private:
         dtr_.clear();
         release_operator();
         if (part_) (void)hipFree(part_);
-        if (red_) (void)hipFree(red_);
-        if (red_host_) (void)hipHostFree(red_host_);
+        if (norm_count_) (void)hipFree(norm_count_);
+        if (norms_) (void)hipHostFree(norms_);
         if (shift_) (void)hipFree(shift_);
         if (bprime_) (void)hipFree(bprime_);
         shift_ = nullptr;
         bprime_ = nullptr;
         part_ = nullptr;
-        red_ = nullptr;
-        red_host_ = nullptr;
+        norm_count_ = nullptr;
+        norms_ = nullptr;
+        norm_seq_ = 0;
     }
 
     void upload()
@@ -2889,10 +2914,12 @@ private:
             }
         const int64_t nb = (int64_t)nblk(host_[0].N);
         MG_HIP(hipMalloc(&part_, (size_t)nb * 2 * sizeof(double)));
-        MG_HIP(hipMalloc(&red_, 2 * sizeof(double)));
+        MG_HIP(hipMalloc(&norm_count_, sizeof *norm_count_));
+        MG_HIP(hipMemset(norm_count_, 0, sizeof *norm_count_));
         MG_HIP(hipMalloc(&shift_, 4 * sizeof(double)));
         if (pin_ >= 0) MG_HIP(hipMalloc(&bprime_, (size_t)host_[0].N * sizeof(double)));
-        MG_HIP(hipHostMalloc(&red_host_, 2 * sizeof(double), hipHostMallocDefault));
+        MG_HIP(hipHostMalloc(&norms_, sizeof *norms_, hipHostMallocCoherent));
+        *norms_ = NormBox{0.0, 0.0, 0};
         MG_HIP(hipStreamSynchronize(nullptr));   // the clears above, before work on other streams
     }
 
@@ -3478,7 +3505,11 @@ private:
 
     void drop_graph(Captured& c)
     {
-        if (c.exec) (void)hipGraphExecDestroy(c.exec);
+        if (c.exec) {
+            // (the host saw its norms, not yet its end)
+            (void)hipStreamSynchronize(stream_);
+            (void)hipGraphExecDestroy(c.exec);
+        }
         c = Captured{};
     }
     void drop_graphs()
@@ -3532,7 +3563,7 @@ private:
     // one V-cycle, ||b - A x||^2 and ||b||^2 on their way to the host
     void checked_cycle_f64(const double* bs, const double* b, double* x, bool chain)
     {
-        auto check = [&]() { outer_residual(bs, b, x, false, false, true, false, nullptr, nullptr); };
+        auto check = [&]() { outer_residual(bs, b, x, false, false, true); };
         if (chain) {
             replay(cap64_, b, x, 1 | kChecked, [&]() {
                 vcycles_f64(x, 1);
@@ -3542,6 +3573,7 @@ private:
             cycles_f64(b, x, 1, false);
             check();
         }
+        ++norm_seq_;
     }
 
     // refinement iterations: FP32 V-cycle on A e = r, x += e, next residual
@@ -3550,7 +3582,7 @@ private:
     {
         const bool fm = fused_mixed();
         vcycles_f32(1, fm, x);
-        outer_residual(bs, b, x, true, fm, norms, false, nullptr, nullptr);
+        outer_residual(bs, b, x, true, fm, norms);
     }
     void iterations_f32(const double* bs, const double* b, double* x, int n, bool chain)
     {
@@ -3561,15 +3593,15 @@ private:
     void iteration_f32(const double* bs, const double* b, double* x)
     {
         replay(cap32_, b, x, 1 | kChecked, [&]() { iterate_f32(bs, b, x, true); });
+        ++norm_seq_;
     }
 
-    // ||b - A x||^2 and ||bn||^2 into red_ (device) and, asynchronously, into
-    // pinned host memory; `wait` synchronises and returns them.
-    // emit_f32: also the scaled FP32 residual into dev_[0].bf; first_sweep:
-    // and the first sweep of e from zero into dev_[0].xf; norms: reduce the
-    // norms and start their copy to the host.
+    // The residual b - A x.  emit_f32: scaled and in FP32 into dev_[0].bf;
+    // first_sweep: and the first sweep of e from zero into dev_[0].xf; norms:
+    // ||b - A x||^2 and ||bn||^2 into norms_ (the caller counts them in
+    // norm_seq_ once per launch or replay, read_norms waits).
     void outer_residual(const double* b, const double* bn, const double* x, bool emit_f32,
-                        bool first_sweep, bool norms, bool wait, double* rr, double* bb)
+                        bool first_sweep, bool norms)
     {
         const DevLevel L = dl(0);
         const unsigned nb = nblk(L.N);
@@ -3605,18 +3637,25 @@ private:
 #undef OUTER
         MG_HIP(hipGetLastError());
         if (!norms) return;
-        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kMgThreads), 0, stream_, part_, (int64_t)nb, red_,
+        hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(kMgThreads), 0, stream_, part_, (int64_t)nb, norms_, norm_count_,
                            pin_ >= 0 ? x : nullptr, bn, pin_, shift_ + 1);
         MG_HIP(hipGetLastError());
-        MG_HIP(hipMemcpyAsync(red_host_, red_, 2 * sizeof(double), hipMemcpyDeviceToHost, stream_));
-        if (wait) read_norms(rr, bb);
     }
 
     void read_norms(double* rr, double* bb)
     {
-        MG_HIP(hipStreamSynchronize(stream_));
-        *rr = red_host_[0];
-        *bb = red_host_[1];
+        // a short wait watches the box; a longer one, and one for norms that
+        // a failed launch never stored, synchronises
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(2000);
+        while (__atomic_load_n(&norms_->seq, __ATOMIC_ACQUIRE) < norm_seq_) {
+            if (std::chrono::steady_clock::now() > until) {
+                MG_HIP(hipStreamSynchronize(stream_));
+                norm_seq_ = __atomic_load_n(&norms_->seq, __ATOMIC_ACQUIRE);
+                break;
+            }
+        }
+        *rr = norms_->rr;
+        *bb = norms_->bb;
     }
 };
 
