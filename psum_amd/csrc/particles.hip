@@ -1233,12 +1233,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(push_m
 // cells, fit an LDS tile; it walks its share of the blocks that k_push_deposit
 // deferred, keeps the particles of its domain and adds their terms in LDS, so
 // every particle is read once per domain (8..24 bytes, mostly from cache)
-// and only tiles reach memory: push 68 us, domains 216 us.  A wave queues the particles it keeps
+// and only tiles reach memory: push 68 us, domains 188 us.  A wave queues the particles it keeps
 // and works them off 64 at a time, all lanes busy.  Terms and cells are
 // k_push_deposit's and sums are integers: the same result.
 constexpr int kDomThreads = 1024;
 constexpr int kDomTile = 17408;            // nodes, 136 KB
 constexpr int kDomMax = 64;                // domains: each reads every particle
+constexpr int kDomAhead = 4;               // chunks in flight
 constexpr int64_t kDomMinParticles = (int64_t)1 << 19;   // below, the atomics take less than ~100 us
 
 struct Domains {
@@ -1301,53 +1302,81 @@ __global__ __launch_bounds__(kDomThreads) void k_deposit_domains(
     };
 
     uint32_t qn = 0;                       // queued particles of the wave
-    T X[2][ROWS][D];
-    auto fetch = [&](uint32_t c, T (*v)[D]) {
+    // The block's chunks part, part + splits, ..: the flags of 64 of them are
+    // read at once (one at a time, each chunk waited for its flag), and the
+    // positions of the next kDomAhead deferred ones are on their way while
+    // the last ones are worked on.
+    uint32_t first = part;                 // chunk of bit 0 of `flags`
+    uint64_t flags = 0;
+    auto load_flags = [&]() {
+        const uint64_t c = (uint64_t)first + (uint64_t)lane * dm.splits;
+        flags = __ballot(c < nchunks && defer[c] != 0);
+    };
+    auto next = [&]() -> uint32_t {        // the next deferred chunk, or nchunks (uniform)
+        while (!flags) {
+            const uint64_t f = (uint64_t)first + 64ull * dm.splits;
+            if (f >= nchunks) return nchunks;
+            first = (uint32_t)f;
+            load_flags();
+        }
+        const int b = __builtin_ctzll(flags);
+        flags &= flags - 1;
+        return first + (uint32_t)b * dm.splits;
+    };
+    struct Batch {
+        uint32_t c[kDomAhead];
+        T x[kDomAhead][ROWS][D];
+    };
+    auto fetch = [&](Batch& q) {
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const int64_t p = (int64_t)c * kPushTile + r * kDomThreads + threadIdx.x;
+        for (int u = 0; u < kDomAhead; ++u) {
+            q.c[u] = next();
 #pragma unroll
-            for (int d = 0; d < D; ++d) v[r][d] = p < n ? xs[d][p] : (T)NAN;
+            for (int r = 0; r < ROWS; ++r) {
+                const int64_t p = (int64_t)q.c[u] * kPushTile + r * kDomThreads + threadIdx.x;
+#pragma unroll
+                for (int d = 0; d < D; ++d) q.x[u][r][d] = p < n ? xs[d][p] : (T)NAN;
+            }
         }
     };
-    auto next = [&](uint32_t c) {          // the first deferred chunk from c on (uniform)
-        while (c < nchunks && !defer[c]) c += dm.splits;
-        return c;
-    };
-    auto work = [&](uint32_t c, T (*v)[D]) {
+    auto work = [&](const Batch& q) {
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            T sd[D];
-            int cw[D];
-            bool in = false;
-            if (isfinite((double)v[r][0]) && cell_of<T, D, kGridAny>(g, v[r], cw, sd)) {
-                uint32_t lc = (uint32_t)cw[0];
+        for (int u = 0; u < kDomAhead; ++u) {
+            if (q.c[u] >= nchunks) continue;
 #pragma unroll
-                for (int d = 1; d < D; ++d) lc = lc * (uint32_t)g.w[d] + (uint32_t)cw[d];
-                in = lc >= lo && lc < hi;
-            }
-            const uint64_t m = __ballot(in);
-            if (in) queue[wave][qn + (uint32_t)__popcll(m & lt)] = c * (uint32_t)kPushTile + r * kDomThreads + threadIdx.x;
-            qn += (uint32_t)__popcll(m);
-            if (qn >= 64) {
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                qn -= 64;
-                add(queue[wave][qn + lane]);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            for (int r = 0; r < ROWS; ++r) {
+                T sd[D];
+                int cw[D];
+                bool in = false;
+                if (isfinite((double)q.x[u][r][0]) && cell_of<T, D, kGridAny>(g, q.x[u][r], cw, sd)) {
+                    uint32_t lc = (uint32_t)cw[0];
+#pragma unroll
+                    for (int d = 1; d < D; ++d) lc = lc * (uint32_t)g.w[d] + (uint32_t)cw[d];
+                    in = lc >= lo && lc < hi;
+                }
+                const uint64_t m = __ballot(in);
+                if (in)
+                    queue[wave][qn + (uint32_t)__popcll(m & lt)] =
+                        q.c[u] * (uint32_t)kPushTile + r * kDomThreads + threadIdx.x;
+                qn += (uint32_t)__popcll(m);
+                if (qn >= 64) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    qn -= 64;
+                    add(queue[wave][qn + lane]);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
             }
         }
     };
-    // the next chunk's positions are on their way while one is worked on
-    uint32_t c = next(part);
-    if (c < nchunks) fetch(c, X[0]);
-    while (c < nchunks) {
-        uint32_t c2 = next(c + dm.splits);
-        if (c2 < nchunks) fetch(c2, X[1]);
-        work(c, X[0]);
-        if (c2 >= nchunks) break;
-        c = next(c2 + dm.splits);
-        if (c < nchunks) fetch(c, X[0]);
-        work(c2, X[1]);
+    load_flags();
+    Batch qa, qb;
+    fetch(qa);
+    while (qa.c[0] < nchunks) {
+        fetch(qb);
+        work(qa);
+        if (qb.c[0] >= nchunks) break;
+        fetch(qa);
+        work(qb);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if ((uint32_t)lane < qn) add(queue[wave][lane]);
