@@ -50,7 +50,7 @@ namespace {
 constexpr int kMgThreads = 256;
 // right-hand sides hold this many zeros beyond their nodes (the dense product
 // reads whole 16-byte vectors of its operator's rows)
-constexpr int kOpPad = 4;
+constexpr int kOpPad = 2;
 
 #define MG_HIP(expr)                                                                        \
     do {                                                                                    \
@@ -1275,51 +1275,54 @@ __global__ __launch_bounds__(kMgThreads) void k_hadamard_many(const HadamardArgs
 // wave per row, 16-byte loads of the row, products summed in FP64 in a fixed
 // order (lane partials, then a butterfly).  Bound by reading M: up to the
 // 32 MB of the eight L2s (a block's rows stay on its XCD from launch to
-// launch) n = 1024 takes 2.6 us and 2025 4.3 us in FP64, launch included;
-// beyond it the Infinity Cache gives about 6 TB/s (FP64 2856: 11 us, FP32
-// 4096: 12 us).  Two or four rows per wave, or a block per row pair, were no
-// faster.  b holds ld values (zeros beyond n).
-template <typename T, typename M>
+// launch) n = 1024 takes 2.6 us and 2025 4.3 us, launch included; beyond it
+// the Infinity Cache gives about 6 TB/s (2856: 11 us, 4913: 28 us).  Two or
+// four rows per wave, or a block per row pair, were no faster.  M is FP64 for
+// FP32 vectors too, as the coarsest inverse is: in FP32 it would be read in
+// half the time, but where the terms of a row cancel (the singular system of
+// a periodic box, a pair of far charges) a V-cycle's error grew from 1.0e-7
+// to 3.7e-7.  b holds ld values (zeros beyond n).
+template <typename T>
 struct CoarseArgs {
-    const M* op;
+    const double* op;
     int n, ld;
     const T* b;
     T* x;
 };
 
-template <typename T, typename M>
-__device__ __forceinline__ void coarse_solve_body(const CoarseArgs<T, M>& a, unsigned bid)
+template <typename T>
+__device__ __forceinline__ void coarse_solve_body(const CoarseArgs<T>& a, unsigned bid)
 {
-    constexpr int V = 16 / (int)sizeof(M);
-    using vec = M __attribute__((ext_vector_type(16 / sizeof(M))));
+    constexpr int V = 2;
+    typedef double vec __attribute__((ext_vector_type(2)));
     const int row = (int)(((int64_t)bid * kMgThreads + threadIdx.x) >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= a.n) return;
-    const M* __restrict__ m = a.op + (int64_t)row * a.ld;
+    const double* __restrict__ m = a.op + (int64_t)row * a.ld;
     const T* __restrict__ b = a.b;
     double s = 0.0;
 #pragma unroll 4
     for (int j = lane * V; j < a.ld; j += 64 * V) {
         const vec v = *reinterpret_cast<const vec*>(m + j);
 #pragma unroll
-        for (int k = 0; k < V; ++k) s += (double)v[k] * (double)b[j + k];
+        for (int k = 0; k < V; ++k) s += v[k] * (double)b[j + k];
     }
     s = wave_sum_full(s);
     if (lane == 0) a.x[row] = (T)s;
 }
 
-template <typename T, typename M>
-__global__ __launch_bounds__(kMgThreads) void k_coarse_solve(CoarseArgs<T, M> a)
+template <typename T>
+__global__ __launch_bounds__(kMgThreads) void k_coarse_solve(CoarseArgs<T> a)
 {
-    coarse_solve_body<T, M>(a, blockIdx.x);
+    coarse_solve_body<T>(a, blockIdx.x);
 }
 
-template <typename T, typename M>
-__global__ __launch_bounds__(kMgThreads) void k_coarse_solve_many(const CoarseArgs<T, M>* __restrict__ a,
+template <typename T>
+__global__ __launch_bounds__(kMgThreads) void k_coarse_solve_many(const CoarseArgs<T>* __restrict__ a,
                                                                   const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
-    coarse_solve_body<T, M>(a[i], blockIdx.x - first[i]);
+    coarse_solve_body<T>(a[i], blockIdx.x - first[i]);
 }
 
 // ---- building the dense coarse-end operator --------------------------------
@@ -1435,12 +1438,11 @@ __global__ __launch_bounds__(kMgThreads) void k_dense_product(int m, int n, cons
         if (r0 + ty + 8 * q < m && c0 + tx < n) E[(int64_t)(r0 + ty + 8 * q) * n + c0 + tx] = s[q];
 }
 
-// rows of n values -> rows of ld values of type M, zeros beyond n
-template <typename M>
-__global__ __launch_bounds__(kMgThreads) void k_dense_pad(int n, int ld, const double* __restrict__ A, M* __restrict__ out)
+// rows of n values -> rows of ld values, zeros beyond n
+__global__ __launch_bounds__(kMgThreads) void k_dense_pad(int n, int ld, const double* __restrict__ A, double* __restrict__ out)
 {
     const int j = (int)(blockIdx.x * kMgThreads + threadIdx.x);
-    if (j < ld) out[(int64_t)blockIdx.y * ld + j] = j < n ? (M)A[(int64_t)blockIdx.y * n + j] : (M)0;
+    if (j < ld) out[(int64_t)blockIdx.y * ld + j] = j < n ? A[(int64_t)blockIdx.y * n + j] : 0.0;
 }
 
 // FP64 residual of the unscaled operator: r = b - A x, partial sums of r^2
@@ -2326,11 +2328,11 @@ namespace psum_hip {
 constexpr uint16_t kKindSmooth = 0;      // + (FP64 << 3 | compact << 2 | prolong << 1 | acc), large tiles
 constexpr uint16_t kKindDown = 16;       // + (FP64 << 1 | compact), large tiles
 constexpr uint16_t kKindRR = 20;         // + (FP64 << 1 | compact)
-constexpr uint16_t kKindCoarse = 24;     // + (0 FP32 vectors with an FP64 operator, 1 FP64, 2 FP32)
-constexpr uint16_t kKindOuter = 27;      // + (norms << 2 | compact << 1 | emit FP32), 2D
-constexpr uint16_t kKindVec = 35;        // + op (0 zero, 1 add correction, 2 copy)
-constexpr uint16_t kKindHadamard = 38;   // FP64
-constexpr uint16_t kKindCount = 39;
+constexpr uint16_t kKindCoarse = 24;     // + FP64
+constexpr uint16_t kKindOuter = 26;      // + (norms << 2 | compact << 1 | emit FP32), 2D
+constexpr uint16_t kKindVec = 34;        // + op (0 zero, 1 add correction, 2 copy)
+constexpr uint16_t kKindHadamard = 37;   // FP64
+constexpr uint16_t kKindCount = 38;
 
 class HipMultigrid {
 public:
@@ -2751,11 +2753,11 @@ private:
         hipLaunchKernelGGL((k_resid_restrict<T, C>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
     }
 
-    template <typename T, typename M>
-    void run_coarse(unsigned nb, const CoarseArgs<T, M>& a)
+    template <typename T>
+    void run_coarse(unsigned nb, const CoarseArgs<T>& a)
     {
-        if (rec_) { emit((uint16_t)(kKindCoarse + (tbit<T>() ? 1 : (tbit<M>() ? 0 : 2))), nb, a); return; }
-        hipLaunchKernelGGL((k_coarse_solve<T, M>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
+        if (rec_) { emit((uint16_t)(kKindCoarse + tbit<T>()), nb, a); return; }
+        hipLaunchKernelGGL((k_coarse_solve<T>), dim3(nb), dim3(kMgThreads), 0, stream_, a);
     }
 
     template <int D, bool C, bool F32, bool NORMS>
@@ -2791,8 +2793,7 @@ private:
     // the coarse end as one dense operator: levels op_level_ and below
     int op_level_ = 0;                 // the coarsest level when nothing is merged
     int op_ld_ = 0, op_pre_ = -1, op_post_ = -1;
-    bool op_f32_ = false;
-    void* op_ = nullptr;
+    double* op_ = nullptr;
     bool fixed_mode_ = false;          // set_fixed_cycles was called
     std::vector<int> tile_fit_;
     double tol_ = 0.0;
@@ -3196,21 +3197,18 @@ private:
     // launch of the levels it covers: 3 per 2D level (5-7 us each), 2 + pre +
     // post per 3D level (3.7-11 us each).  The level taken is the finest whose
     // matrix is small enough to beat those launches:
-    //   2D  33 MB: FP64 2048 nodes 4.3 us (16-18 us for the level's launches),
-    //       4096 nodes 21 us, no faster than the launches; FP32 to 67 MB,
-    //       4096 nodes 12 us against 17 + 2.8 us
-    //   3D  200 MB: 17^3 nodes 28 us (FP64) / 17 us (FP32) against 45-60 us
+    //   2D  33 MB: 2048 nodes 4.3 us (16-18 us for the level's launches), 4096
+    //       nodes 21 us, no faster than the launches
+    //   3D  200 MB: 17^3 nodes 28 us against 45-60 us
     // Fixed-cycle solves (batches of many solvers, whose matrices share the
     // caches) take at most 1089 nodes.
-    // FP32 V-cycles take the matrix in FP32 (built in FP64, products summed in
-    // FP64) where levels are merged, and the coarsest inverse alone in FP64.
     int operator_level() const
     {
         const int Lc = (int)host_.size() - 1;
-        const int64_t limit = host_[0].D == 3 ? 200000000 : (mixed_ ? 67200000 : 33600000);
+        const int64_t limit = host_[0].D == 3 ? 200000000 : 33600000;
         for (int l = 1; l < Lc; ++l) {
             const int64_t n = host_[l].N;
-            if (fixed_mode_ ? n <= 1089 : (n < 32768 && n * n * (mixed_ ? 4 : 8) <= limit)) return l;
+            if (fixed_mode_ ? n <= 1089 : (n < 32768 && n * n * 8 <= limit)) return l;
         }
         return Lc;
     }
@@ -3280,13 +3278,9 @@ private:
             M = X;
         }
         const int n = (int)host_[target].N;
-        op_f32_ = mixed_ && target < Lc;
-        const int v = op_f32_ ? 4 : 2;
-        op_ld_ = (n + v - 1) / v * v;
-        MG_HIP(hipMalloc(&op_, (size_t)n * op_ld_ * (op_f32_ ? sizeof(float) : sizeof(double))));
-        const dim3 grid(nblk(op_ld_), n);
-        if (op_f32_) hipLaunchKernelGGL(k_dense_pad<float>, grid, dim3(kMgThreads), 0, st, n, op_ld_, M, static_cast<float*>(op_));
-        else hipLaunchKernelGGL(k_dense_pad<double>, grid, dim3(kMgThreads), 0, st, n, op_ld_, M, static_cast<double*>(op_));
+        op_ld_ = (n + 1) / 2 * 2;
+        MG_HIP(hipMalloc(&op_, (size_t)n * op_ld_ * sizeof(double)));
+        hipLaunchKernelGGL(k_dense_pad, dim3(nblk(op_ld_), n), dim3(kMgThreads), 0, st, n, op_ld_, M, op_);
         MG_HIP(hipGetLastError());
         MG_HIP(hipStreamSynchronize(st));
         op_level_ = target;
@@ -3382,12 +3376,7 @@ private:
             rec_phase(it, kStageCoarse, 0);
             const int n = (int)host_[ld].N;
             const unsigned nb = (unsigned)(((int64_t)n * 64 + kMgThreads - 1) / kMgThreads);
-            if constexpr (std::is_same<T, float>::value) {
-                if (op_f32_) run_coarse<T, float>(nb, CoarseArgs<T, float>{static_cast<const float*>(op_), n, op_ld_, bs[ld], xs[ld]});
-                else run_coarse<T, double>(nb, CoarseArgs<T, double>{static_cast<const double*>(op_), n, op_ld_, bs[ld], xs[ld]});
-            } else {
-                run_coarse<T, double>(nb, CoarseArgs<T, double>{static_cast<const double*>(op_), n, op_ld_, bs[ld], xs[ld]});
-            }
+            run_coarse<T>(nb, CoarseArgs<T>{op_, n, op_ld_, bs[ld], xs[ld]});
             for (int l = ld - 1; l >= 0; --l) {
                 rec_phase(it, kStageUp, 255u - (uint32_t)l);
                 if (post_ > 0) {
@@ -3792,13 +3781,12 @@ void mg_batch_launch(const MgBatchPlan& plan, hipStream_t st)
             }
 #undef RRL
         } else if (k < kKindOuter) {
-#define COARSE(T, M) hipLaunchKernelGGL((k_coarse_solve_many<T, M>), grid, dim3(kMgThreads), 0, st, static_cast<const CoarseArgs<T, M>*>(a), f, g.n)
-            switch (k - kKindCoarse) {
-            case 0: COARSE(float, double); break;
-            case 1: COARSE(double, double); break;
-            default: COARSE(float, float); break;
-            }
-#undef COARSE
+            if (k - kKindCoarse)
+                hipLaunchKernelGGL((k_coarse_solve_many<double>), grid, dim3(kMgThreads), 0, st,
+                                   static_cast<const CoarseArgs<double>*>(a), f, g.n);
+            else
+                hipLaunchKernelGGL((k_coarse_solve_many<float>), grid, dim3(kMgThreads), 0, st,
+                                   static_cast<const CoarseArgs<float>*>(a), f, g.n);
         } else if (k < kKindVec) {
             const OuterArgs* oa = static_cast<const OuterArgs*>(a);
 #define OUT(C, F, N) hipLaunchKernelGGL((k_outer_residual_many<2, C, F, N>), grid, dim3(kMgThreads), 0, st, oa, f, g.n)

@@ -39,7 +39,7 @@ def _periodic(nodes, seed):
     return nn, r, c, v, b
 
 
-# second level of 2025, 2070 (FP64 limit 2049), 4096 and 64, 49 nodes in 2D;
+# second level of 2025, 2070 (limit 2049), 4096 and 64, 49 nodes in 2D;
 # 4913, 5832 (limit 5000) and 1100 in 3D
 CASES = [("walls", (89, 89), 3), ("walls", (89, 90), 3), ("periodic", (128, 128), 3), ("periodic", (16, 16), 2),
          ("walls", (13, 14), 2), ("walls", (33, 33, 33), 3), ("walls", (35, 35, 35), 3), ("walls", (17, 20, 23), 2)]
@@ -93,6 +93,31 @@ def test_merged_levels_in_the_mixed_solver(kind, nodes, depth):
     x64, _ = solve("hip_multigrid_gpu", "max_cycles 60 tol 1e-11")
     assert rel <= 1e-10
     assert np.max(np.abs(x32 - x64)) <= 1e-8 * np.max(np.abs(x64))
+
+
+@pytest.mark.parametrize("n", [32, 64])
+def test_merged_levels_lose_no_precision_in_the_mixed_solver(n):
+    """A pair of far charges in a periodic box: the rows of the merged matrix
+    cancel against each other, so the matrix itself has to be held in FP64
+    (held in FP32: 3.7e-7).  What FP32 vectors round is the scaled and the
+    restricted right-hand side, the coarse values and the sweep: 2^-24 each."""
+    from psum_amd import engine as E
+    nodes = (n, n, n)
+    nn, r, c, v, _ = _periodic(nodes, 1)
+    b = np.zeros(nodes)
+    b[n // 4, n // 4, n // 4], b[3 * n // 4, 3 * n // 4, 3 * n // 4] = 1.0, -1.0
+    x = []
+    for backend in ("hip_multigrid_gpu", "hip_multigrid32f_gpu"):
+        s = E.SolverBackend(backend)
+        s.set_options(f"I {n} J {n} K {n} depth {n.bit_length() - 4} pre_relax 0 post_relax 1 max_cycles 1 "
+                      "correction_interval 1")
+        s.set_matrix(nn, nn, r, c, v)
+        xd = torch.zeros(nn, dtype=torch.float64, device="cuda")
+        s.solve(torch.from_numpy(b.ravel().copy()).cuda(), xd)
+        x.append(xd.cpu().numpy())
+    e = x[1] - x[0]
+    e -= e[0]            # the gauge is the pinned node's
+    assert np.linalg.norm(e) <= 4 * 2.0 ** -24 * np.linalg.norm(x[0])
 
 
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
