@@ -2686,10 +2686,7 @@ public:
         corr_ = 1;
         use_graph_ = 0;
         drop_graphs();
-        if (!fixed_mode_) {
-            fixed_mode_ = true;
-            if (!host_.empty()) build_operator();
-        }
+        fixed_mode_ = true;
     }
 
     int last_cycles() const { return last_cycles_; }
@@ -2790,10 +2787,14 @@ private:
     int I_ = 0, J_ = 0, K_ = 0, depth_ = 3, pre_ = 2, post_ = 1, max_cycles_ = 10, corr_ = 4;
     int fuse_ = 1;   // 2D: fused multi-sweep tile smoothing and residual+restriction
     int line_ = 1;   // 3D 7-point levels: chunk kernels (k_smooth_line, k_residual_line)
-    // the coarse end as one dense operator: levels op_level_ and below
-    int op_level_ = 0;                 // the coarsest level when nothing is merged
-    int op_ld_ = 0, op_pre_ = -1, op_post_ = -1;
-    double* op_ = nullptr;
+    // the coarse end as one dense operator: levels `level` and below (the
+    // coarsest alone when nothing is merged)
+    struct Operator {
+        double* m = nullptr;
+        int level = 0, ld = 0;
+    };
+    Operator op_, op_fixed_;           // op_fixed_: fixed-cycle solves (may be op_'s matrix)
+    int op_pre_ = -1, op_post_ = -1;   // sweeps they were built for
     bool fixed_mode_ = false;          // set_fixed_cycles was called
     std::vector<int> tile_fit_;
     double tol_ = 0.0;
@@ -3201,105 +3202,107 @@ private:
     //       nodes 21 us, no faster than the launches
     //   3D  200 MB: 17^3 nodes 28 us against 45-60 us
     // Fixed-cycle solves (batches of many solvers, whose matrices share the
-    // caches) take at most 1089 nodes.
-    int operator_level() const
+    // caches) take at most 1089 nodes.  Their matrix is one of those that the
+    // other is built from, so both are kept and a solver that switches to a
+    // fixed cycle count builds nothing again.
+    int operator_level(bool fixed) const
     {
         const int Lc = (int)host_.size() - 1;
         const int64_t limit = host_[0].D == 3 ? 200000000 : 33600000;
         for (int l = 1; l < Lc; ++l) {
             const int64_t n = host_[l].N;
-            if (fixed_mode_ ? n <= 1089 : (n < 32768 && n * n * 8 <= limit)) return l;
+            if (fixed ? n <= 1089 : (n < 32768 && n * n * 8 <= limit)) return l;
         }
         return Lc;
     }
 
     void release_operator()
     {
-        if (op_) (void)hipFree(op_);
-        op_ = nullptr;
-        op_level_ = (int)host_.size() - 1;
+        if (op_.m) (void)hipFree(op_.m);
+        if (op_fixed_.m && op_fixed_.m != op_.m) (void)hipFree(op_fixed_.m);
+        op_ = op_fixed_ = Operator{};
         op_pre_ = op_post_ = -1;
     }
 
-    // device memory released when the scope is left
-    struct Scratch {
-        std::vector<void*> p;
-        ~Scratch() { for (void* q : p) (void)hipFree(q); }
-        double* take(size_t n)
-        {
-            void* q = nullptr;
-            MG_HIP(hipMalloc(&q, std::max<size_t>(1, n) * sizeof(double)));
-            p.push_back(q);
-            return static_cast<double*>(q);
-        }
-        void drop(double* q)
-        {
-            p.erase(std::find(p.begin(), p.end(), (void*)q));
-            (void)hipFree(q);
-        }
-    };
-
-    // the operator for the current hierarchy, smoothing counts and cycle mode;
-    // without memory for a merged one, the coarsest inverse alone
+    // the operators for the current hierarchy and smoothing counts; without
+    // memory for a merged one, the coarsest inverse alone
     void build_operator()
     {
-        const int l = operator_level();
-        const bool merged = l < (int)host_.size() - 1;
-        if (op_ && l == op_level_ && (!merged || (pre_ == op_pre_ && post_ == op_post_))) return;
+        if (op_.m && pre_ == op_pre_ && post_ == op_post_) return;
+        const int Lc = (int)host_.size() - 1;
         drop_graphs();
         release_operator();
-        if (merged) {
-            try {
-                build_operator_at(l);
-                return;
-            } catch (const std::runtime_error&) {
-                (void)hipGetLastError();
-                release_operator();
-            }
+        try {
+            build_operators_at(operator_level(false), operator_level(true));
+        } catch (const std::runtime_error&) {
+            (void)hipGetLastError();
+            release_operator();
+            build_operators_at(Lc, Lc);
         }
-        build_operator_at((int)host_.size() - 1);
-    }
-
-    void build_operator_at(int target)
-    {
-        const int Lc = (int)host_.size() - 1;
-        struct Stream {
-            hipStream_t s = nullptr;
-            ~Stream() { if (s) (void)hipStreamDestroy(s); }
-        } own;
-        MG_HIP(hipStreamCreateWithFlags(&own.s, hipStreamNonBlocking));
-        hipStream_t st = own.s;
-        Scratch mem;
-        double* M = mem.take(cinv_host_.size());
-        MG_HIP(hipMemcpy(M, cinv_host_.data(), cinv_host_.size() * sizeof(double), hipMemcpyHostToDevice));
-        for (int l = Lc - 1; l >= target; --l) {
-            double* X = host_[l].D == 2 ? operator_columns<2>(l, M, mem, st) : operator_columns<3>(l, M, mem, st);
-            mem.drop(M);
-            M = X;
-        }
-        const int n = (int)host_[target].N;
-        op_ld_ = (n + 1) / 2 * 2;
-        MG_HIP(hipMalloc(&op_, (size_t)n * op_ld_ * sizeof(double)));
-        hipLaunchKernelGGL(k_dense_pad, dim3(nblk(op_ld_), n), dim3(kMgThreads), 0, st, n, op_ld_, M, op_);
-        MG_HIP(hipGetLastError());
-        MG_HIP(hipStreamSynchronize(st));
-        op_level_ = target;
         op_pre_ = pre_;
         op_post_ = post_;
     }
 
-    // the V-cycle from level l down applied to every unit vector: pre-sweeps
-    // from zero, residual, restriction, the next level's operator M,
-    // prolongation, post-sweeps
+    // op_ at level `target`, op_fixed_ at `fixed` (target <= fixed).  One
+    // allocation for everything but the results: a hipMalloc and a hipFree of
+    // their own for each matrix of each level were most of the set-up's time
+    // on small grids.
+    void build_operators_at(int target, int fixed)
+    {
+        const int Lc = (int)host_.size() - 1;
+        struct Scope {
+            hipStream_t st = nullptr;
+            double* mem = nullptr;
+            ~Scope()
+            {
+                if (mem) (void)hipFree(mem);
+                if (st) (void)hipStreamDestroy(st);
+            }
+        } own;
+        MG_HIP(hipStreamCreateWithFlags(&own.st, hipStreamNonBlocking));
+        hipStream_t st = own.st;
+        size_t sq = (size_t)host_[Lc].N * host_[Lc].N, rect = 0;
+        for (int l = target; l < Lc; ++l) {
+            sq = std::max(sq, (size_t)host_[l].N * host_[l].N);
+            rect = std::max(rect, (size_t)host_[l].N * host_[l + 1].N);
+        }
+        // the next level's operator and two n x n matrices, two m x n ones
+        MG_HIP(hipMalloc(&own.mem, ((target < Lc ? 3 : 1) * sq + 2 * rect) * sizeof(double)));
+        double *M = own.mem, *X = M + sq, *Y = X + sq, *B = Y + sq, *E = B + rect;
+        MG_HIP(hipMemcpy(M, cinv_host_.data(), cinv_host_.size() * sizeof(double), hipMemcpyHostToDevice));
+        for (int l = Lc;; --l) {
+            if (l == fixed && l != target) keep_operator(op_fixed_, l, M, st);
+            if (l == target) break;
+            if (host_[l - 1].D == 2) operator_columns<2>(l - 1, M, X, Y, B, E, st);
+            else operator_columns<3>(l - 1, M, X, Y, B, E, st);
+            std::swap(M, X);
+        }
+        keep_operator(op_, target, M, st);
+        if (fixed == target) op_fixed_ = op_;
+        MG_HIP(hipStreamSynchronize(st));
+    }
+
+    void keep_operator(Operator& op, int level, const double* M, hipStream_t st)
+    {
+        const int n = (int)host_[level].N;
+        op.level = level;
+        op.ld = (n + 1) / 2 * 2;
+        MG_HIP(hipMalloc(&op.m, (size_t)n * op.ld * sizeof(double)));
+        hipLaunchKernelGGL(k_dense_pad, dim3(nblk(op.ld), n), dim3(kMgThreads), 0, st, n, op.ld, M, op.m);
+        MG_HIP(hipGetLastError());
+    }
+
+    // X = the V-cycle from level l down applied to every unit vector:
+    // pre-sweeps from zero, residual, restriction, the next level's operator M,
+    // prolongation, post-sweeps (X and Y are exchanged as the sweeps go)
     template <int D>
-    double* operator_columns(int l, const double* M, Scratch& mem, hipStream_t st)
+    void operator_columns(int l, const double* M, double*& X, double*& Y, double* B, double* E, hipStream_t st)
     {
         const DevLevel F = dl(l), C = dl(l + 1);
-        const size_t n = (size_t)F.N, m = (size_t)C.N;
+        const int n = (int)F.N, m = (int)C.N;
         const double two3 = 2.0 / 3;
         const DevTable<double> rx{dev_[l].Rx, dev_[l].dinv}, ah{dev_[l].Ah, dev_[l].dinv};
-        double *X = mem.take(n * n), *Y = mem.take(n * n), *B = mem.take(m * n), *E = mem.take(m * n);
-        const dim3 th(kMgThreads), gf(nblk(F.N), (unsigned)n), gc(nblk(F.N), (unsigned)m);
+        const dim3 th(kMgThreads), gf(nblk(n), n), gc(nblk(n), m);
         // sweep from zero: (2/3) I; no pre-sweeps: 0
         hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, rx.coef, (const double*)nullptr, X, 0.0, pre_ > 0 ? two3 : 0.0);
         for (int k = 1; k < pre_; ++k) {
@@ -3308,18 +3311,13 @@ private:
         }
         hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, ah.coef, X, Y, -1.0, 1.0);
         hipLaunchKernelGGL(k_dense_restrict<D>, gc, th, 0, st, F, C, transfer<double>(l), dev_[l + 1].dinv, Y, B);
-        hipLaunchKernelGGL(k_dense_product, dim3((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32)), th, 0, st, (int)m, (int)n, M, B, E);
+        hipLaunchKernelGGL(k_dense_product, dim3((n + 31) / 32, (m + 31) / 32), th, 0, st, m, n, M, B, E);
         hipLaunchKernelGGL(k_dense_prolong<D>, gf, th, 0, st, F, C, transfer<double>(l), E, X);
         for (int k = 0; k < post_; ++k) {
             hipLaunchKernelGGL(k_dense_stencil<D>, gf, th, 0, st, F, rx.coef, X, Y, 1.0, two3);
             std::swap(X, Y);
         }
         MG_HIP(hipGetLastError());
-        MG_HIP(hipStreamSynchronize(st));
-        mem.drop(Y);
-        mem.drop(B);
-        mem.drop(E);
-        return X;
     }
 
     // One or more V-cycles on level-0 arrays (b0 scaled, x0 warm start).
@@ -3333,7 +3331,8 @@ private:
     {
         const T two3 = (T)(2.0 / 3);
         bool accd = false;
-        const int ld = op_level_;                // this level and those below: one dense product
+        const Operator& op = fixed_mode_ ? op_fixed_ : op_;
+        const int ld = op.level;                 // this level and those below: one dense product
         for (int cyc = 0; cyc < cycles; ++cyc) {
             const uint32_t it = rec_iter_ + (uint32_t)cyc;
             for (int l = 0; l < ld; ++l) {
@@ -3376,7 +3375,7 @@ private:
             rec_phase(it, kStageCoarse, 0);
             const int n = (int)host_[ld].N;
             const unsigned nb = (unsigned)(((int64_t)n * 64 + kMgThreads - 1) / kMgThreads);
-            run_coarse<T>(nb, CoarseArgs<T>{op_, n, op_ld_, bs[ld], xs[ld]});
+            run_coarse<T>(nb, CoarseArgs<T>{op.m, n, op.ld, bs[ld], xs[ld]});
             for (int l = ld - 1; l >= 0; --l) {
                 rec_phase(it, kStageUp, 255u - (uint32_t)l);
                 if (post_ > 0) {

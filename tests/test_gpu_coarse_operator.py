@@ -141,6 +141,24 @@ def test_switching_to_fixed_cycles_keeps_the_solution(dtype):
     assert np.max(np.abs(phis[0] - phis[1])) <= 1e-9 * np.max(np.abs(phis[0]))
 
 
+def test_switching_to_fixed_cycles_builds_nothing():
+    """44 x 46 nodes are merged with a tolerance and 22 x 23 in a fixed-cycle
+    solver: both matrices are there from the set-up on, so the switch neither
+    allocates nor frees."""
+    from psum_amd import engine as E
+    from psum_amd.workloads import langmuir_2d
+    wl = langmuir_2d(n=88, ppc=4, seed=3)
+    g = E.periodic_grid([88, 92])
+    st = E.Stepper(g, wl["species"], depth=3, pre=2, post=2, max_cycles=40, tol=1e-12, dt=wl["dt"], rho_bg=1.0)
+    st.run(1)
+    free = torch.cuda.mem_get_info()[0]
+    st.set_schedule(25, 0, 0)
+    assert torch.cuda.mem_get_info()[0] == free
+    st.run(1)
+    assert torch.cuda.mem_get_info()[0] == free
+    st.close()
+
+
 @pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
 @pytest.mark.parametrize("kind,nodes,depth", [
     ("walls", (1100, 300), 6),       # large tiles (210 blocks) with remainders on both axes
