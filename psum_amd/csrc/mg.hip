@@ -2514,6 +2514,7 @@ public:
     const double* solve_begin(double* b, bool homogeneous = false, const double* mean_part = nullptr)
     {
         if (host_.empty()) throw std::runtime_error("hip_multigrid: solve before set_matrix");
+        build_operator();     // nothing to do, unless a call that set the sweeps failed
         hipStream_t st = stream_;
         scaled_ = false;
         if (takes_mean()) {
@@ -2663,6 +2664,7 @@ public:
     void record_core(const double* b, const double* bs, double* x, std::vector<RecOp>& ops)
     {
         if (!recordable()) throw std::logic_error("hip_multigrid: this solve cannot be batched");
+        build_operator();
         ops.clear();
         rec_ = &ops;
         try {

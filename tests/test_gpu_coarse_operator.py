@@ -141,6 +141,26 @@ def test_switching_to_fixed_cycles_keeps_the_solution(dtype):
     assert np.max(np.abs(phis[0] - phis[1])) <= 1e-9 * np.max(np.abs(phis[0]))
 
 
+def test_operator_follows_the_sweeps_of_a_refused_option_list():
+    """An option list that is refused half-way has set the sweeps before the
+    value it is refused for: the next solve runs with them on every level,
+    merged ones included, like a solver set up with them."""
+    from psum_amd import engine as E
+    nn, r, c, v, b = _walls((65, 49), 4)
+    out = []
+    for late in (False, True):
+        s = E.SolverBackend("hip_multigrid_gpu")
+        s.set_options(f"I 65 J 49 depth 3 pre_relax {1 if late else 3} post_relax 1 max_cycles 2")
+        s.set_matrix(nn, nn, r, c, v)
+        if late:
+            with pytest.raises(E.PsumError):
+                s.set_options("I 65 J 49 pre_relax 3 correction_interval 0")
+        x = torch.zeros(nn, dtype=torch.float64, device="cuda")
+        s.solve(torch.from_numpy(b).cuda(), x)
+        out.append(x.cpu().numpy())
+    assert np.array_equal(out[0], out[1])
+
+
 def test_switching_to_fixed_cycles_builds_nothing():
     """44 x 46 nodes are merged with a tolerance and 22 x 23 in a fixed-cycle
     solver: both matrices are there from the set-up on, so the switch neither
