@@ -710,21 +710,25 @@ __device__ __forceinline__ int batch_instance(const unsigned* __restrict__ first
 // of instruction fetches, not bandwidth.  128^2 and 64^2 FP64 levels of 256
 // threads a block: 6.7-7.9 us a launch with copy loops and conditional loads,
 // 5.7-6.7 us so; 1024^2 FP32: 19.7 and 20.0 -> 17.3 and 18.8 us.  Two
-// geometries:
-// 1024 threads over 32 rows (16 coarse rows), and 256 threads over 8 rows
-// (3 coarse rows) for levels whose large tiles would leave most compute units
-// idle (small_tiles()).
+// geometries per precision: large tiles, 1024 threads over 32 rows (16 coarse
+// rows) in FP32 and 512 threads over 16 rows (7 coarse rows) in FP64, and 256
+// threads over 8 rows (3 coarse rows) for levels that large tiles would leave
+// mostly idle (small_tiles()).  All of a block's waves wait for the same
+// barriers, so a compute unit with two blocks of 1024 threads moves nothing
+// meanwhile: on large FP64 levels, which are bound by bandwidth, four blocks
+// of 512 threads are faster (walls, 2049^2: prolongation and sweep 58 -> 45
+// us, downward half 78 -> 71 us; 1025^2: 20 -> 15 and 25 -> 23 us).
 constexpr int kTileX = 64;
 constexpr int kMaxFuse = 3;
 constexpr int kMaxClsLds = 32;
 
-template <bool SMALL>
+template <typename T, bool SMALL>
 struct TileGeom {
-    static constexpr int threads = SMALL ? 256 : 1024;
+    static constexpr int threads = SMALL ? 256 : (sizeof(T) == 8 ? 512 : 1024);
     static constexpr int groups = threads / kTileX;     // waves, one row group each
     static constexpr int rpt = SMALL ? 4 : 3;           // consecutive rows per thread
-    static constexpr int rows = SMALL ? 8 : 32;         // output rows of a smoothing tile
-    static constexpr int crows = SMALL ? 3 : 16;        // coarse rows of a k_down_tile tile
+    static constexpr int rows = SMALL ? 8 : (sizeof(T) == 8 ? 16 : 32);   // output rows of a smoothing tile
+    static constexpr int crows = SMALL ? 3 : (sizeof(T) == 8 ? 7 : 16);   // coarse rows of a k_down_tile tile
     // one guard row on each side, one guard value before and after: tile row
     // i, column tx at at(i, tx)
     static constexpr int plane = (groups * rpt + 2) * kTileX + 2;
@@ -747,8 +751,8 @@ template <bool SMALL, typename T>
 __device__ __forceinline__ void tab_load(const T* __restrict__ coef, int n, T* v)
 {
 #pragma unroll
-    for (int q = 0; q < TileGeom<SMALL>::tab_per; ++q) {
-        const int i = threadIdx.x + q * TileGeom<SMALL>::threads;
+    for (int q = 0; q < TileGeom<T, SMALL>::tab_per; ++q) {
+        const int i = threadIdx.x + q * TileGeom<T, SMALL>::threads;
         v[q] = coef[i < n ? i : 0];
     }
 }
@@ -756,8 +760,8 @@ template <bool SMALL, typename T>
 __device__ __forceinline__ void tab_store(T* lds, int n, const T* v)
 {
 #pragma unroll
-    for (int q = 0; q < TileGeom<SMALL>::tab_per; ++q) {
-        const int i = threadIdx.x + q * TileGeom<SMALL>::threads;
+    for (int q = 0; q < TileGeom<T, SMALL>::tab_per; ++q) {
+        const int i = threadIdx.x + q * TileGeom<T, SMALL>::threads;
         if (i < n) lds[i] = v[q];
     }
 }
@@ -816,7 +820,7 @@ struct TileRow {
 template <typename T, bool COMPACT, bool SMALL, typename R, typename F>
 __device__ __forceinline__ void tile_stencil(const T* p, R&& row, F&& f)
 {
-    constexpr int RPT = TileGeom<SMALL>::rpt;
+    constexpr int RPT = TileGeom<T, SMALL>::rpt;
     T w[3][3];
     // a compact row reads only column 0 of the rows above and below
     auto get = [&](int r, T* q, bool side) {
@@ -846,8 +850,8 @@ __device__ __forceinline__ int tile_sweeps(P& sx, int tx, int i0, int nrows, int
 {
     int cur = 0;
     for (int sw = 1; sw <= h; ++sw) {
-        const T* xs = &sx[cur][TileGeom<SMALL>::at(i0 - 1, tx)];
-        T* xn = &sx[cur ^ 1][TileGeom<SMALL>::at(i0, tx)];
+        const T* xs = &sx[cur][TileGeom<T, SMALL>::at(i0 - 1, tx)];
+        T* xn = &sx[cur ^ 1][TileGeom<T, SMALL>::at(i0, tx)];
         const bool colok = tx >= sw && tx < kTileX - sw;
         tile_stencil<T, COMPACT, SMALL>(xs, row, [&](int k, T t) {
             const int i = i0 + k;
@@ -883,7 +887,7 @@ struct SmoothTileArgs {
 template <typename T, bool COMPACT, bool PROLONG, bool ACC, bool SMALL>
 __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, unsigned bid)
 {
-    using G = TileGeom<SMALL>;
+    using G = TileGeom<T, SMALL>;
     constexpr int RPT = G::rpt;
     constexpr int CW = G::cw, CH = G::ch;   // staged coarse values
     const DevLevel& L = A.L;
@@ -904,7 +908,10 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
     const bool lds_tab = A.ncls <= kMaxClsLds;
     // coordinates first, then every load in one straight run (a load under a
     // condition is waited for where the paths join); rows beyond the tile
-    // repeat its last
+    // repeat its last.  Waves of large FP64 tiles without a row (2 of 8 with
+    // one sweep) load none: those launches are bound by these loads (walls,
+    // 2049^2: 237 -> 230 us a cycle).  In FP32 and in small tiles they are
+    // not, and the branch costs more (1024^2 FP32 3 us a cycle)
     const int g1 = tile_coord(t1 - h + tx, n1, L.wrap[1]);
     int g0[RPT];
 #pragma unroll
@@ -928,7 +935,7 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
         for (int k = 0; k < G::xc_per; ++k) cv[k] = xc[ic[k]];
     if (lds_tab) tab_load<SMALL>(relax.coef, A.ncls * 9, tab);
     T breg[RPT], xv[RPT];
-    int creg[RPT];
+    int creg[RPT] = {};      // (waves that load no row index the tables with it)
     double xa[RPT];
     int p0[RPT], p1 = 0;
     T w0[RPT][2], w1[2] = {(T)0, (T)0};
@@ -939,19 +946,20 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
     }
     const int g1o = t1 + tx - h;
     const bool colout = tx >= h && tx < kTileX - h && g1o < n1;
+    if (SMALL || sizeof(T) == 4 || i0 < R)
 #pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-        const int64_t gi = (int64_t)g0[k] * n1 + g1;
-        xv[k] = A.xin[gi];
-        breg[k] = A.b[gi];
-        creg[k] = L.cls[gi];
-        if (PROLONG) {
-            p0[k] = tr.pc[0][g0[k]];
-            w0[k][0] = tr.pw[0][2 * g0[k]];
-            w0[k][1] = tr.pw[0][2 * g0[k] + 1];
+        for (int k = 0; k < RPT; ++k) {
+            const int64_t gi = (int64_t)g0[k] * n1 + g1;
+            xv[k] = A.xin[gi];
+            breg[k] = A.b[gi];
+            creg[k] = L.cls[gi];
+            if (PROLONG) {
+                p0[k] = tr.pc[0][g0[k]];
+                w0[k][0] = tr.pw[0][2 * g0[k]];
+                w0[k][1] = tr.pw[0][2 * g0[k] + 1];
+            }
+            if (ACC) xa[k] = A.xacc[gi];
         }
-        if (ACC) xa[k] = A.xacc[gi];
-    }
     if (lds_tab) tab_store<SMALL>(ctab, A.ncls * 9, tab);
     if (PROLONG) {
         if (staged) {
@@ -1013,13 +1021,13 @@ __device__ __forceinline__ void smooth_tile_body(const SmoothTileArgs<T>& A, uns
 }
 
 template <typename T, bool COMPACT, bool PROLONG, bool ACC, bool SMALL>
-__global__ __launch_bounds__(TileGeom<SMALL>::threads) void k_smooth_tile(SmoothTileArgs<T> a)
+__global__ __launch_bounds__((TileGeom<T, SMALL>::threads)) void k_smooth_tile(SmoothTileArgs<T> a)
 {
     smooth_tile_body<T, COMPACT, PROLONG, ACC, SMALL>(a, blockIdx.x);
 }
 
 template <typename T, bool COMPACT, bool PROLONG, bool ACC>
-__global__ __launch_bounds__(TileGeom<false>::threads) void k_smooth_tile_many(const SmoothTileArgs<T>* __restrict__ a,
+__global__ __launch_bounds__((TileGeom<T, false>::threads)) void k_smooth_tile_many(const SmoothTileArgs<T>* __restrict__ a,
                                                                                const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
@@ -1064,7 +1072,7 @@ __host__ __device__ inline int down_cols(int h, int st) { return (kTileX - 2 - 2
 template <typename T, bool COMPACT, bool SMALL>
 __device__ __forceinline__ void down_tile_body(const DownTileArgs<T>& A, unsigned bid)
 {
-    using G = TileGeom<SMALL>;
+    using G = TileGeom<T, SMALL>;
     constexpr int RPT = G::rpt;
     const DevLevel& F = A.r.F;
     const DevLevel& Cl = A.r.Cl;
@@ -1094,14 +1102,15 @@ __device__ __forceinline__ void down_tile_body(const DownTileArgs<T>& A, unsigne
         tab_load<SMALL>(A.relax.coef, A.r.ncls * 9, tb);
     }
     T breg[RPT], xv[RPT];
-    int creg[RPT];
+    int creg[RPT] = {};      // (waves that load no row index the tables with it)
+    if (SMALL || sizeof(T) == 4 || i0 < R)
 #pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-        const int64_t gi = (int64_t)g0[k] * n1 + g1;
-        xv[k] = A.r.x[gi];
-        breg[k] = A.r.bf[gi];
-        creg[k] = F.cls[gi];
-    }
+        for (int k = 0; k < RPT; ++k) {
+            const int64_t gi = (int64_t)g0[k] * n1 + g1;
+            xv[k] = A.r.x[gi];
+            breg[k] = A.r.bf[gi];
+            creg[k] = F.cls[gi];
+        }
     // the coarse node this thread sums: its support and weights
     const int c0 = c0lo + ty, c1 = c1lo + tx;
     const bool coarse = ty < G::crows && tx < CC && c0 < c0hi && c1 < c1hi;
@@ -1172,13 +1181,13 @@ __device__ __forceinline__ void down_tile_body(const DownTileArgs<T>& A, unsigne
 }
 
 template <typename T, bool COMPACT, bool SMALL>
-__global__ __launch_bounds__(TileGeom<SMALL>::threads) void k_down_tile(DownTileArgs<T> a)
+__global__ __launch_bounds__((TileGeom<T, SMALL>::threads)) void k_down_tile(DownTileArgs<T> a)
 {
     down_tile_body<T, COMPACT, SMALL>(a, blockIdx.x);
 }
 
 template <typename T, bool COMPACT>
-__global__ __launch_bounds__(TileGeom<false>::threads) void k_down_tile_many(const DownTileArgs<T>* __restrict__ a,
+__global__ __launch_bounds__((TileGeom<T, false>::threads)) void k_down_tile_many(const DownTileArgs<T>* __restrict__ a,
                                                                              const unsigned* __restrict__ first, int n)
 {
     const int i = batch_instance(first, n);
@@ -2733,16 +2742,16 @@ private:
     void run_smooth_tile(bool small, unsigned nb, const SmoothTileArgs<T>& a)
     {
         if (rec_) { emit((uint16_t)(kKindSmooth + ((tbit<T>() << 3) | (C << 2) | (P << 1) | (A ? 1 : 0))), nb, a); return; }
-        if (small) hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, true>), dim3(nb), dim3(TileGeom<true>::threads), 0, stream_, a);
-        else hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, false>), dim3(nb), dim3(TileGeom<false>::threads), 0, stream_, a);
+        if (small) hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, true>), dim3(nb), dim3(TileGeom<T, true>::threads), 0, stream_, a);
+        else hipLaunchKernelGGL((k_smooth_tile<T, C, P, A, false>), dim3(nb), dim3(TileGeom<T, false>::threads), 0, stream_, a);
     }
 
     template <typename T, bool C>
     void run_down(bool small, unsigned nb, const DownTileArgs<T>& a)
     {
         if (rec_) { emit((uint16_t)(kKindDown + ((tbit<T>() << 1) | (C ? 1 : 0))), nb, a); return; }
-        if (small) hipLaunchKernelGGL((k_down_tile<T, C, true>), dim3(nb), dim3(TileGeom<true>::threads), 0, stream_, a);
-        else hipLaunchKernelGGL((k_down_tile<T, C, false>), dim3(nb), dim3(TileGeom<false>::threads), 0, stream_, a);
+        if (small) hipLaunchKernelGGL((k_down_tile<T, C, true>), dim3(nb), dim3(TileGeom<T, true>::threads), 0, stream_, a);
+        else hipLaunchKernelGGL((k_down_tile<T, C, false>), dim3(nb), dim3(TileGeom<T, false>::threads), 0, stream_, a);
     }
 
     template <typename T, bool C>
@@ -3115,8 +3124,8 @@ private:
             const int k = std::min(count, kMaxFuse);
             const int ostep = kTileX - 2 * k;
             const int64_t ntc = (L.n[1] + ostep - 1) / ostep;
-            const bool small = small_tiles(((L.n[0] + TileGeom<false>::rows - 1) / TileGeom<false>::rows) * ntc);
-            const int rows = small ? TileGeom<true>::rows : TileGeom<false>::rows;
+            const bool small = small_tiles<T>(((L.n[0] + TileGeom<T, false>::rows - 1) / TileGeom<T, false>::rows) * ntc);
+            const int rows = small ? TileGeom<T, true>::rows : TileGeom<T, false>::rows;
             const unsigned nb = (unsigned)(((L.n[0] + rows - 1) / rows) * ntc);
             double* a = (k == count) ? acc : nullptr;
             const SmoothTileArgs<T> ta{L, table<T>(l, true), ncls, x, b, buf, two3, k, C, tr, half, xc, a};
@@ -3140,14 +3149,21 @@ private:
         return accd;
     }
 
-    // Tiles of 256 threads and 8 rows where the large ones (1024 threads, 32
-    // rows) would cover the level with fewer than 128 blocks, half the compute
-    // units: V(2,1) cycles of 128^2 FP64 take 16 % less time with them (13.6
-    // against 16.0 ms per 20 steps of the Langmuir run), 641 x 385 17 % less,
-    // 1024^2 0.5-2 % more.  Recorded solves share their launches with other
-    // solvers, whose blocks fill the chip: always the large ones (12 instances
-    // of 64^2..256^2: 27.3 against 28.2 ms).
-    bool small_tiles(int64_t large_blocks) const { return !rec_ && large_blocks < 128; }
+    // Tiles of 256 threads and 8 rows where the large ones would cover the
+    // level with fewer blocks than this.  FP32: 128 blocks of 1024 threads,
+    // half the compute units (1024^2 with small tiles 0.5-2 % slower).  FP64:
+    // 512 blocks of 512 threads, two a compute unit: the small tiles' launches
+    // take 10.4 and 12.1 us on 513^2 nodes (297 large blocks: 11.2 and 12.4),
+    // 17.3 and 25.7 on 1025^2 (1105 large blocks: 15.6 and 23.0).  V(2,1)
+    // cycles of 128^2 FP64 take 16 % less time with them (13.6 against 16.0 ms
+    // per 20 steps of the Langmuir run).  Recorded solves share their launches
+    // with other solvers, whose blocks fill the chip: always the large ones
+    // (12 instances of 64^2..256^2: 27.3 against 28.2 ms).
+    template <typename T>
+    bool small_tiles(int64_t large_blocks) const
+    {
+        return !rec_ && large_blocks < (sizeof(T) == 8 ? 512 : 128);
+    }
 
     // How the transfers between levels l and l + 1 step along the two axes,
     // 10 st[0] + st[1] with 2 for a halved axis and 1 for one kept as it is,
@@ -3352,8 +3368,8 @@ private:
                     if (steps) {
                         const int st[2] = {steps / 10, steps % 10};
                         const int64_t ntc = (C.n[1] + down_cols(h, st[1]) - 1) / down_cols(h, st[1]);
-                        const bool small = small_tiles(((C.n[0] + TileGeom<false>::crows - 1) / TileGeom<false>::crows) * ntc);
-                        const int rows = small ? TileGeom<true>::crows : TileGeom<false>::crows;
+                        const bool small = small_tiles<T>(((C.n[0] + TileGeom<T, false>::crows - 1) / TileGeom<T, false>::crows) * ntc);
+                        const int rows = small ? TileGeom<T, true>::crows : TileGeom<T, false>::crows;
                         const DownTileArgs<T> da{ra, table<T>(l, true), ts[l], two3, h, {st[0], st[1]}};
                         const unsigned nb = (unsigned)(((C.n[0] + rows - 1) / rows) * ntc);
                         if (host_[l].compact) run_down<T, true>(small, nb, da);
@@ -3743,7 +3759,7 @@ void mg_batch_launch(const MgBatchPlan& plan, hipStream_t st)
         const uint16_t k = g.kind;
         if (k < kKindDown) {
 #define SMT(T, C, P, A)                                                                                                   \
-    hipLaunchKernelGGL((k_smooth_tile_many<T, C, P, A>), grid, dim3(TileGeom<false>::threads), 0, st,                     \
+    hipLaunchKernelGGL((k_smooth_tile_many<T, C, P, A>), grid, dim3(TileGeom<T, false>::threads), 0, st,                     \
                        static_cast<const SmoothTileArgs<T>*>(a), f, g.n)
             switch (k - kKindSmooth) {
             case 0: SMT(float, false, false, false); break;
@@ -3763,7 +3779,7 @@ void mg_batch_launch(const MgBatchPlan& plan, hipStream_t st)
 #undef SMT
         } else if (k < kKindRR) {
 #define DWN(T, C)                                                                                                         \
-    hipLaunchKernelGGL((k_down_tile_many<T, C>), grid, dim3(TileGeom<false>::threads), 0, st,                             \
+    hipLaunchKernelGGL((k_down_tile_many<T, C>), grid, dim3(TileGeom<T, false>::threads), 0, st,                             \
                        static_cast<const DownTileArgs<T>*>(a), f, g.n)
             switch (k - kKindDown) {
             case 0: DWN(float, false); break;

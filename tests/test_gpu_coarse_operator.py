@@ -182,6 +182,8 @@ def test_switching_to_fixed_cycles_builds_nothing():
 @pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
 @pytest.mark.parametrize("kind,nodes,depth", [
     ("walls", (1100, 300), 6),       # large tiles (210 blocks) with remainders on both axes
+    ("walls", (823, 760), 6),        # large FP64 tiles (52 x 13 of 16 rows) with remainders on both axes
+    ("periodic", (720, 704), 6),     # and across the seam
     ("walls", (301, 1153), 6),       # odd counts
     ("periodic", (512, 464), 5),     # large tiles across the seam
     ("walls", (199, 62), 3),         # small tiles, even last axis
