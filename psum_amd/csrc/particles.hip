@@ -1241,6 +1241,12 @@ constexpr int kDomTile = 17408;            // nodes, 136 KB
 constexpr int kDomMax = 64;                // domains: each reads every particle
 constexpr int kDomAhead = 4;               // chunks in flight
 constexpr int64_t kDomMinParticles = (int64_t)1 << 19;   // below, the atomics take less than ~100 us
+// 2D: up to 51 domains have five blocks each, beyond it four.  2^19 FP32
+// particles on 50 domains take 99 us (103 with the atomics), on 52 109 us
+// (102), on 62 114 us (104); 2^20 on 52 182 us (188), 4M 616 us (707).  In 3D
+// (twice the atomics) 48 domains take half the time of the atomics.
+constexpr int kDomFew2D = 51;
+constexpr int64_t kDomManyParticles = (int64_t)1 << 20;
 
 struct Domains {
     uint32_t cells, count, up, splits;     // cells a domain, domains, nodes above, blocks per domain
@@ -1403,6 +1409,7 @@ static Domains plan_domains(const psum_grid* g, int64_t n)
     if (room < kDomTile / 4) return dm;
     const int64_t count = (nn + room - 1) / room;
     if (count > kDomMax) return dm;
+    if (g->dim == 2 && count > kDomFew2D && n < kDomManyParticles) return dm;
     dm.count = (uint32_t)count;
     dm.cells = (uint32_t)((nn + count - 1) / count);
     dm.up = (uint32_t)up;

@@ -55,6 +55,25 @@ def test_domains_equal_direct_adds(nodes, periodic, dx, dtype, n, ordered):
             assert torch.equal(torch.nan_to_num(s, nan=-1.0), torch.nan_to_num(t, nan=-1.0))
 
 
+@pytest.mark.parametrize("nodes,n,domains", [((1024, 800), N0, True), ((1024, 830), N0, False),
+                                             ((1024, 830), 2 * N0 - 1, False), ((1024, 830), 2 * N0, True),
+                                             ((80, 80, 80), N0, True)])
+def test_many_domains_need_many_particles(nodes, n, domains):
+    """In 2D more than 51 domains cost more than the atomics below 2^20
+    particles: both sides of the line, the same sums"""
+    from psum_amd import _lib
+    from psum_amd import engine as E
+    g = E.periodic_grid(list(nodes))
+    assert (_lib.lib().psum_hip_gather_push_workspace(C.byref(g), n) > 0) == domains
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    pos = [torch.rand(n, generator=gen, device="cuda") * m * 0.999999 for m in nodes]
+    vel = [torch.zeros(n, device="cuda") for _ in nodes]
+    ref, _ = E.deposit(g, pos, -0.7, scale=2.0 ** 40)
+    acc, _ = E.gather_push(g, pos, vel, torch.zeros(E.num_nodes(g), device="cuda"), -1.0, 0.0, 1.0, w_dep=-0.7,
+                           scale=2.0 ** 40)
+    assert torch.equal(acc, ref)
+
+
 def test_domain_sums_that_wrap_are_counted():
     """one cell takes 2^19 terms of 2^49..2^50: every node's sum leaves the
     int64 range in an LDS tile, and the counter says so"""
