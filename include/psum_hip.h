@@ -70,7 +70,8 @@ const char* psum_hip_last_error(void);
 psum_status psum_hip_bin(const psum_grid* g, int dtype, void* const* pos, int64_t n,
                          uint32_t* keys, void* stream);
 
-/* Bytes of device workspace psum_hip_sort needs for n keys. */
+/* Bytes of device workspace psum_hip_sort needs for n keys (at 4-byte
+ * alignment, as the arrays). */
 size_t psum_hip_sort_workspace(int64_t n);
 
 /* Stable LSD radix sort of keys in [0, nkeys) plus PSUM_KEY_INVALID (last).

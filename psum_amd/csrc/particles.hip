@@ -1702,7 +1702,8 @@ size_t psum_hip_sort_workspace(int64_t n)
 {
     if (n <= 0) return 256;
     const int64_t nh = (n + kSortSmallTile - 1) / kSortSmallTile << kSortMaxBits;
-    return 2 * align256((size_t)n * 4) + align256((size_t)nh * 4) + scan_workspace(nh);
+    // (8: the pairs start on 8 bytes wherever the workspace starts)
+    return 8 + 2 * align256((size_t)n * 4) + align256((size_t)nh * 4) + scan_workspace(nh);
 }
 
 psum_status psum_hip_sort(const uint32_t* keys, int64_t n, uint32_t nkeys, uint32_t* keys_out,
@@ -1716,7 +1717,7 @@ psum_status psum_hip_sort(const uint32_t* keys, int64_t n, uint32_t nkeys, uint3
     hipStream_t st = S(stream);
     const int W = sort_waves(n);
     const int nb = (int)((n + (int64_t)W * kSortWaveTile - 1) / ((int64_t)W * kSortWaveTile));
-    char* w = static_cast<char*>(work);
+    char* w = reinterpret_cast<char*>(((uintptr_t)work + 7) & ~(uintptr_t)7);
     uint32_t* pairs = reinterpret_cast<uint32_t*>(w);     // n (key, index) pairs
     w += 2 * align256((size_t)n * 4);
     uint32_t* gh = reinterpret_cast<uint32_t*>(w);

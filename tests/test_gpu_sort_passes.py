@@ -26,6 +26,24 @@ def test_every_pass_count_is_a_stable_sort(nkeys, n):
     assert np.array_equal(sk.cpu().numpy().view(np.uint32), keys[want])
 
 
+@pytest.mark.parametrize("n", [3, 5000, 70_001])
+@pytest.mark.parametrize("nkeys", [1000, 1 << 17, 1 << 20])
+def test_workspace_and_arrays_at_4_byte_alignment(n, nkeys):
+    from psum_amd import _lib
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, nkeys, n, dtype=np.uint32)
+    want = np.argsort(keys, kind="stable")
+    lib = _lib.lib()
+    wb = lib.psum_hip_sort_workspace(n)
+    a = [torch.zeros(n + 1, dtype=torch.int32, device="cuda") for _ in range(3)]
+    a[0][1:] = torch.from_numpy(keys.view(np.int32))
+    work = torch.empty(wb + 4, dtype=torch.uint8, device="cuda")
+    k, out, perm, w = (t.data_ptr() + 4 for t in a + [work])
+    _lib.check(lib.psum_hip_sort(k, n, nkeys, out, perm, w, wb, torch.cuda.current_stream().cuda_stream), "sort")
+    assert np.array_equal(a[2][1:].cpu().numpy().view(np.uint32), want.astype(np.uint32))
+    assert np.array_equal(a[1][1:].cpu().numpy().view(np.uint32), keys[want])
+
+
 def _state(st, n):
     from psum_amd import _lib
     pos, vel, m = (C.c_void_p * 3)(), (C.c_void_p * 3)(), C.c_int64(0)
