@@ -75,7 +75,8 @@ psum_status psum_hip_bin(const psum_grid* g, int dtype, void* const* pos, int64_
 size_t psum_hip_sort_workspace(int64_t n);
 
 /* Stable LSD radix sort of keys in [0, nkeys) plus PSUM_KEY_INVALID (last).
- * perm[r] = index of the r-th particle; keys_out = sorted keys.
+ * perm[r] = index of the r-th particle; keys_out = sorted keys (keys_out may
+ * be keys: the sort is then in place).
  * No reference counterpart; defines the sort order the engine uses. */
 psum_status psum_hip_sort(const uint32_t* keys, int64_t n, uint32_t nkeys, uint32_t* keys_out,
                           uint32_t* perm, void* work, size_t work_bytes, void* stream);

@@ -1722,7 +1722,10 @@ psum_status psum_hip_sort(const uint32_t* keys, int64_t n, uint32_t nkeys, uint3
     w += 2 * align256((size_t)n * 4);
     uint32_t* gh = reinterpret_cast<uint32_t*>(w);
     const int bits = 32 - __builtin_clz(nkeys);           // INVALID maps to nkeys
-    const int passes = (bits + kSortMaxBits - 1) / kSortMaxBits;
+    int passes = (bits + kSortMaxBits - 1) / kSortMaxBits;
+    // an odd count's first pass writes keys_out while it reads keys: in place
+    // (which two and four passes of 8 bits allowed) it takes one pass more
+    if (keys_out == keys && passes % 2 != 0) ++passes;
     const int width = (bits + passes - 1) / passes;
     w += align256(((size_t)nb << width) * 4);
     void* scan_work = w;

@@ -44,6 +44,24 @@ def test_workspace_and_arrays_at_4_byte_alignment(n, nkeys):
     assert np.array_equal(a[1][1:].cpu().numpy().view(np.uint32), keys[want])
 
 
+# 1, 1, 2, 3 and 4 digits of up to 10 bits
+@pytest.mark.parametrize("nkeys", [5, 1000, 60_000, 1 << 25, 0xFFFFFFFE])
+@pytest.mark.parametrize("n", [4097, 500_001])
+def test_sort_in_place(nkeys, n):
+    from psum_amd import _lib
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, nkeys, n, dtype=np.uint32)
+    want = np.argsort(keys, kind="stable")
+    lib = _lib.lib()
+    wb = lib.psum_hip_sort_workspace(n)
+    k = torch.from_numpy(keys.view(np.int32)).cuda()
+    perm, work = torch.empty_like(k), torch.empty(wb, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.psum_hip_sort(k.data_ptr(), n, nkeys, k.data_ptr(), perm.data_ptr(), work.data_ptr(), wb,
+                                 torch.cuda.current_stream().cuda_stream), "sort")
+    assert np.array_equal(perm.cpu().numpy().view(np.uint32), want.astype(np.uint32))
+    assert np.array_equal(k.cpu().numpy().view(np.uint32), keys[want])
+
+
 def _state(st, n):
     from psum_amd import _lib
     pos, vel, m = (C.c_void_p * 3)(), (C.c_void_p * 3)(), C.c_int64(0)
