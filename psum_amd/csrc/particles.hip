@@ -2083,8 +2083,13 @@ psum_status psum_hip_field_energy(const psum_grid* g, const double* phi, double 
     PSUM_HIP_TRY(hipGetLastError());
     double vol = 1.0;
     for (int d = 0; d < g->dim; ++d) vol *= g->delta[d];
-    if (eps == 0.0) vol = 0.0;   // (0 * sum: the reduction's f of 0 means no scaling)
-    return reduce4(part, nb, out, part + nb * 4, st, eps == 0.0 ? 1.0 : 0.5 * eps, vol);
+    double f = 0.5 * eps;        // (0 for the smallest eps too)
+    if (f == 0.0) {
+        // 0 * sum: the reduction's f of 0 means no scaling
+        f = 1.0;
+        vol = 0.0;
+    }
+    return reduce4(part, nb, out, part + nb * 4, st, f, vol);
 }
 
 psum_status psum_hip_f64_to_f32(const double* in, float* out, int64_t n, void* stream)

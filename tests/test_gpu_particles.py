@@ -274,3 +274,14 @@ def test_field_energy():
         ref = O.field_energy(og, phi, 0.7)
         got = float(_host(E.field_energy(eg, _dev(phi), 0.7)))
         assert abs(got - ref) <= 1e-12 * abs(ref), name
+
+
+@pytest.mark.parametrize("eps", [0.0, -0.0, 5e-324])
+def test_field_energy_of_no_permittivity(eps):
+    """0.5 * eps is 0 for the smallest eps too: the energy is 0, not the
+    unscaled sum"""
+    E = _E()
+    rng = np.random.default_rng(3)
+    for name, eg, og in _grids():
+        phi = rng.standard_normal(O.num_nodes(og))
+        assert float(_host(E.field_energy(eg, _dev(phi), eps))) == 0.0, name
