@@ -3650,8 +3650,10 @@ private:
 
     void read_norms(double* rr, double* bb)
     {
-        // a short wait watches the box; a longer one, and one for norms that
-        // a failed launch never stored, synchronises
+        // a short wait watches the box, giving way to the host's other
+        // threads between looks (steppers on more threads than cores); a
+        // longer one, and one for norms that a failed launch never stored,
+        // synchronises
         const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(2000);
         while (__atomic_load_n(&norms_->seq, __ATOMIC_ACQUIRE) < norm_seq_) {
             if (std::chrono::steady_clock::now() > until) {
@@ -3659,6 +3661,7 @@ private:
                 norm_seq_ = __atomic_load_n(&norms_->seq, __ATOMIC_ACQUIRE);
                 break;
             }
+            std::this_thread::yield();
         }
         *rr = norms_->rr;
         *bb = norms_->bb;
