@@ -122,9 +122,8 @@ def test_merged_levels_lose_no_precision_in_the_mixed_solver(n):
 
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
 def test_switching_to_fixed_cycles_keeps_the_solution(dtype):
-    """A fixed cycle count takes a smaller limit (the operator is built
-    again): the step's potential stays that of the tolerance-controlled
-    solve."""
+    """A fixed cycle count takes a smaller limit (a matrix of its own): the
+    step's potential stays that of the tolerance-controlled solve."""
     from psum_amd import engine as E
     from psum_amd.workloads import langmuir_2d
     wl = langmuir_2d(n=128, ppc=4, seed=3, dtype=np.float64 if dtype == "f64" else np.float32)

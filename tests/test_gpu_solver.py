@@ -268,63 +268,70 @@ def test_fused_2d_kernels_are_bit_identical(backend, case, prepost, stop):
     assert np.array_equal(np.float64(out[0][1][1]), np.float64(out[1][1][1]), equal_nan=True)
 
 
-@pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
-@pytest.mark.parametrize("case", ["periodic256_d6", "periodic128_d4", "walls_129x97_d5"])
-@pytest.mark.parametrize("prepost", [(3, 3), (2, 1), (0, 2)])
-def test_vcycle_tail_is_bit_identical(backend, case, prepost):
-    """The one-workgroup tail (levels from the first that fits in LDS down to
-    the coarsest, in one launch) performs the per-level kernels' operations
-    in the same order: equal bits with the tail switched off."""
+def _against_oracle(backend, problem, dims, depth, pre, post):
+    """Three cycles are the oracle's (FP64 sums in another order; mixed: FP32
+    V-cycles, each rounded apart, inside FP64 refinement), and the
+    tolerance-controlled solve ends at the oracle's solution."""
     E = _E()
-    if case.startswith("periodic"):
-        n = int(case[8:case.index("_")])
-        og, nn, r, c, v, b = _periodic_problem(n, seed=5)
-        I, J = n, n
-    else:
-        I, J = 129, 97
-        og, nn, r, c, v, b = _wall_problem_2d(I, J, seed=6)
-    depth = int(case[case.rindex("d") + 1:])
-    pre, post = prepost
-    out = []
-    for tail in (0, 1):
+    nn, r, c, v, b = problem
+    sizes = " ".join(f"{k} {m}" for k, m in zip("IJK", dims))
+    mg = O.MG(nn, r, c, v, *dims, depth=depth, pre=pre, post=post)
+    mixed = backend == "hip_multigrid32f_gpu"
+
+    def solve(opt):
         s = E.SolverBackend(backend)
-        s.set_options(f"I {I} J {J} depth {depth} pre_relax {pre} post_relax {post} "
-                      f"max_cycles 30 tol 1e-9 tail {tail}")
+        s.set_options(f"{sizes} depth {depth} pre_relax {pre} post_relax {post} {opt}")
         s.set_matrix(nn, nn, r, c, v)
         x = torch.zeros(nn, dtype=torch.float64, device="cuda")
         s.solve(_dev(b), x)
-        s.solve(_dev(b * 1.01), x)
-        out.append((x.cpu().numpy(), s.stats()))
-    assert np.array_equal(out[0][0], out[1][0])
-    assert out[0][1][0] == out[1][1][0]
+        return x.cpu().numpy(), s.stats()
+    x, _ = solve("max_cycles 3 correction_interval 1")
+    ref = mg.solve_mixed(b, np.zeros(nn), 3, 1) if mixed else mg.vcycles(b, np.zeros(nn), 3)
+    assert np.max(np.abs(x - ref)) <= (1e-5 if mixed else 1e-11) * np.max(np.abs(ref))
+    x, (cycles, rel) = solve("max_cycles 60 tol 1e-10")
+    assert rel <= 1e-10 and cycles < 60
+    ref = mg.vcycles(b, np.zeros(nn), cycles + 2)
+    assert np.max(np.abs(x - ref)) <= 1e-8 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
+@pytest.mark.parametrize("case", ["periodic256_d6", "periodic128_d4", "walls_129x97_d5"])
+@pytest.mark.parametrize("prepost", [(3, 3), (2, 1), (0, 2)])
+def test_dense_coarse_end_matches_the_oracle(backend, case, prepost):
+    """The levels from 32^2 and 33 x 25 nodes down in one dense product (three
+    or four levels merged)."""
+    if case.startswith("periodic"):
+        n = int(case[8:case.index("_")])
+        problem, dims = _periodic_problem(n, seed=5)[1:], (n, n)
+    else:
+        dims = (129, 97)
+        problem = _wall_problem_2d(*dims, seed=6)[1:]
+    _against_oracle(backend, problem, dims, int(case[case.rindex("d") + 1:]), *prepost)
 
 
 @pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
 @pytest.mark.parametrize("case", [(33, 4), (37, 4), (65, 5), (17, 3)])
 @pytest.mark.parametrize("prepost", [(3, 3), (2, 1), (0, 2)])
-def test_vcycle_tail_3d_is_bit_identical(backend, case, prepost):
-    """3D walls: the one-workgroup tail ("tail 1") runs levels of at most 9^3 nodes down
-    to a coarsest level of at most 5^3 (33^3 depth 4 and 65^3 depth 5: 9, 5;
-    37^3 depth 4: 10^3 is too large, so no tail) with the 27-point rows, 3D
-    restriction, dense solve and prolongation of the per-level kernels:
-    equal bits and cycle counts with the tail switched off."""
-    E = _E()
+def test_dense_coarse_end_3d_matches_the_oracle(backend, case, prepost):
+    """3D walls, merged from 17^3 (33^3, 65^3 nodes), 10^3 (37^3, whose 19^3 is
+    too large) and 9^3 nodes (17^3) down."""
     n, depth = case
-    og, nn, r, c, v, b, fixed = _wall_problem_3d(n, seed=11)
-    pre, post = prepost
+    _against_oracle(backend, _wall_problem_3d(n, seed=11)[1:6], (n, n, n), depth, *prepost)
+
+
+def test_tail_option_is_accepted():
+    """the option of an earlier coarse end: no effect, no error"""
+    E = _E()
+    og, nn, r, c, v, b = _wall_problem_2d(33, 29, seed=6)
     out = []
-    for tail in (0, 1):
-        s = E.SolverBackend(backend)
-        s.set_options(f"I {n} J {n} K {n} depth {depth} pre_relax {pre} post_relax {post} "
-                      f"max_cycles 30 tol 1e-9 tail {tail}")
+    for tail in ("", "tail 0", "tail 1"):
+        s = E.SolverBackend("hip_multigrid_gpu")
+        s.set_options(f"I 33 J 29 depth 3 max_cycles 2 {tail}")
         s.set_matrix(nn, nn, r, c, v)
         x = torch.zeros(nn, dtype=torch.float64, device="cuda")
         s.solve(_dev(b), x)
-        s.solve(_dev(b * 1.01), x)
-        out.append((x.cpu().numpy(), s.stats()))
-    assert np.array_equal(out[0][0], out[1][0])
-    assert out[0][1][0] == out[1][1][0]
-    assert np.array_equal(np.float64(out[0][1][1]), np.float64(out[1][1][1]), equal_nan=True)
+        out.append(x.cpu().numpy())
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
 
 
 @pytest.mark.parametrize("backend", ["hip_multigrid_gpu", "hip_multigrid32f_gpu"])
