@@ -77,7 +77,7 @@ __device__ __forceinline__ double wave_max_d(double v)
 // kAdjPPT consecutive particles per thread of k_adj_push and the nodes of its
 // deposit tile.  A block of 1024 particles in lattice or sorted order covers
 // at most ~64 cells of a row at 16 per cell, plus the drift since the order
-// was made; 4096 nodes (32 KB, 5 blocks per CU) also hold a block that
+// was made; 4096 nodes (32 KB, 4 blocks per CU) also hold a block that
 // straddles the end of a 256-node row.
 constexpr int kAdjPPT = 4;
 constexpr int kAdjTile = 4096;

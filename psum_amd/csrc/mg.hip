@@ -14,7 +14,8 @@
 //              sycl_multigrid32f_gpu.cpp:23-266 (FP32 V-cycles inside an FP64
 //              residual refinement loop; here the coarse solve stays FP64)
 //
-// MI355X form: the matrices never exist on the device.  Every level is a
+// MI355X form: the levels' matrices never exist on the device (only the
+// coarse end, as the dense matrix of its V-cycle).  Every level is a
 // structured node grid (n0 x n1 [x n2], last dimension fastest) whose rows
 // are 3^D-point stencils; rows with identical coefficients share a class,
 // so a level is a uint16 class id per node plus a small coefficient table.
@@ -3467,15 +3468,15 @@ private:
     // V-cycles (FP64) or refinement iterations (mixed: FP32 V-cycle, x += e,
     // next residual), replayed from captured hipGraphs when the solver runs on
     // its own stream.  Graphs are keyed on (b, x) (the caller's b: the checks
-    // read it) and what they hold; a few
-    // are kept so that callers alternating between solves on different
-    // buffers (a forward and an adjoint solve) do not re-capture each time.
+    // read it) and what they hold; a few are kept so that a stepper
+    // alternating between solves on different buffers (a forward and an
+    // adjoint solve) does not re-capture each time.
     //
     // Between two graph launches the GPU idles for 8 us (nodes of one graph
     // follow each other without a gap), as long as one and a half launches of
     // a small level: the cycles before the first check run in graphs of 8, 4,
-    // 2 and 1, and the checked cycle's graph holds its residual, norms and
-    // their copy.  Langmuir 128^2 FP64, 16 cycles a step: 610 -> 581 us a step.  The
+    // 2 and 1, and the checked cycle's graph holds its residual and norms.
+    // Langmuir 128^2 FP64, 16 cycles a step: 610 -> 581 us a step.  The
     // longer graphs are captured from the second solve on a pair (b, x) on: a
     // caller with new buffers each time replays one-cycle graphs.
     struct Captured {
