@@ -341,7 +341,7 @@ def test_chunked_3d_kernels_are_bit_identical(backend, n, prepost):
     """On 7-point 3D levels of 2^16 nodes or more the sweeps, residuals and
     the mixed solver's outer residual run four nodes per thread (interior
     nodes of the dominant class) plus a per-node pass over the listed rest,
-    and prolongation to 3D levels of 2^15 nodes or more runs over planes; the
+    and prolongation to 3D levels with planes of 64 nodes or more over planes; the
     mixed solver takes its first level-0 sweep from the outer residual.  The
     terms and their order are the separate kernels', so the bits equal those
     with "line 0".
